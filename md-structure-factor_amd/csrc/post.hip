@@ -215,6 +215,97 @@ __global__ void k_rz_average(const double* __restrict__ kp, int nx, int ny, int 
   }
 }
 
+// The same average for cells whose z axis is orthogonal to x and y (binv couples
+// neither: the reference driver's cells).  A sample's (u, v) then depends on
+// (r, theta) alone and w on z alone, so the trilinear sum splits into
+//   A[p] = sum_k sum_{a, b} wx_a wy_b S[i_k + a][j_k + b][p]   (every z plane p)
+//   oa[iz] = ((1 - tz) A[k] + tz A[k + 1]) / nth               (k: the cell of z)
+// with the angle, its two cells and its four weights evaluated once per (r, k)
+// instead of once per (r, z, k), and four gathers instead of eight.  One block
+// per r bin, longest rings first: the block stages kRzChunk samples' columns and
+// weights in LDS, each wave takes 64 z planes of every kRzLanes-th sample, and
+// the waves' partial sums are added in a fixed order.  Gather-bound: a wave's
+// load spans 64 z planes of the 4-channel grid, 2 KB for 512 used bytes.  The
+// plots of a 256^3 run (grids, this average, Ewald sections) take 1,185 us with
+// it against 4,481 us with k_rz_average, those of a 104 x 90 x 80 run in a 120
+// degree cell 531 against 1,455 us.
+constexpr int kRzThreads = 1024;
+constexpr int kRzChunk = 1024;          // samples staged per round
+constexpr int kRzPlanes = 256;          // z planes per round
+constexpr int kRzLanes = kRzThreads / kRzPlanes;
+constexpr int kRzMaxPlanes = 1024;      // plane sums kept in LDS (8 KB, 52 KB in all)
+
+__global__ __launch_bounds__(kRzThreads) void k_rz_average_sep(
+    const double* __restrict__ kp, int nx, int ny, int nz, const double* __restrict__ rarr,
+    const int* __restrict__ nth, int nr, const double* __restrict__ zar, int nzb, Mat3 b,
+    double* __restrict__ oa) {
+#pragma clang fp contract(off)
+  extern __shared__ __align__(16) unsigned char rz_lds[];
+  double* A = reinterpret_cast<double*>(rz_lds);              // nz plane sums
+  __shared__ double red[kRzLanes][kRzPlanes];
+  __shared__ int col[kRzChunk];                               // i * ny + j
+  __shared__ double wt[kRzChunk][4];                          // weights of (0,0) (0,1) (1,0) (1,1)
+  __shared__ int off_grid;
+  const int tid = threadIdx.x;
+  const int ir = nr - 1 - (int)blockIdx.x;
+  const double r = rarr[ir];
+  const int nt = nth[ir];
+  const double step = (2.0 * 3.141592653589793) / (double)nt;
+  const long long sx = (long long)ny * nz * 4, sy = (long long)nz * 4;
+  if (tid == 0) off_grid = 0;
+  for (int p = tid; p < nz; p += kRzThreads) A[p] = 0.0;
+  const int pl = tid % kRzPlanes, lane = tid / kRzPlanes;
+  for (int k0 = 0; k0 < nt; k0 += kRzChunk) {
+    __syncthreads();
+    const int kn = min(kRzChunk, nt - k0);
+    if (tid < kn) {
+      const double t = (double)(k0 + tid) * step;
+      const double x = r * cos(t), y = r * sin(t);
+      const double u = x * b.m[0] + y * b.m[3], v = x * b.m[1] + y * b.m[4];
+      bool oob = false;
+      const int i = find_cell(kp + 0, sx, nx, u, &oob);
+      const int j = find_cell(kp + 1, sy, ny, v, &oob);
+      const double tx = (u - kp[i * sx]) / (kp[(i + 1) * sx] - kp[i * sx]);
+      const double ty = (v - kp[1 + j * sy]) / (kp[1 + (j + 1) * sy] - kp[1 + j * sy]);
+      if (oob) off_grid = 1;
+      col[tid] = i * ny + j;
+      wt[tid][0] = (1.0 - tx) * (1.0 - ty);
+      wt[tid][1] = (1.0 - tx) * ty;
+      wt[tid][2] = tx * (1.0 - ty);
+      wt[tid][3] = tx * ty;
+    }
+    __syncthreads();
+    for (int p0 = 0; p0 < nz; p0 += kRzPlanes) {
+      const int p = min(p0 + pl, nz - 1);
+      double s = 0.0;
+#pragma unroll 4
+      for (int k = lane; k < kn; k += kRzLanes) {
+        const double* c = kp + (size_t)col[k] * (size_t)sy + 4 * (size_t)p + 3;
+        s = s + (wt[k][0] * c[0] + wt[k][1] * c[sy]) + (wt[k][2] * c[sx] + wt[k][3] * c[sx + sy]);
+      }
+      red[lane][pl] = s;
+      __syncthreads();
+      if (tid < kRzPlanes && p0 + tid < nz) {
+        double v = red[0][tid];
+#pragma unroll
+        for (int l = 1; l < kRzLanes; ++l) v = v + red[l][tid];
+        A[p0 + tid] = A[p0 + tid] + v;
+      }
+      __syncthreads();
+    }
+  }
+  __syncthreads();
+  const bool off = off_grid != 0;   // a sample off the grid: NaN over the ring
+  for (int iz = tid; iz < nzb; iz += kRzThreads) {
+    const double w = zar[iz] * b.m[8];
+    bool oob = off;
+    const int k = find_cell(kp + 2, 4, nz, w, &oob);
+    const double tz = (w - kp[2 + 4 * (size_t)k]) / (kp[2 + 4 * (size_t)(k + 1)] - kp[2 + 4 * (size_t)k]);
+    oa[(long long)ir * nzb + iz] =
+        oob ? nan("") : (A[k] * (1.0 - tz) + A[k + 1] * tz) / (double)nt;
+  }
+}
+
 // Interpolant at arbitrary points (n, 3): the RegularGridInterpolator calls
 // on plain grids (plot2d.py:588, 800-840).
 __global__ void k_interp_points(const double* __restrict__ kp, int nx, int ny, int nz,
@@ -334,8 +425,16 @@ hipError_t launch_rz_average(const double* kp, int nx, int ny, int nz, const dou
                              const double binv[9], double* oa, hipStream_t s) {
   Mat3 b;
   for (int k = 0; k < 9; ++k) b.m[k] = binv[k];
-  hipLaunchKernelGGL(k_rz_average, dim3(grid_for((long long)nr * nzb)), dim3(256), 0, s, kp, nx, ny,
-                     nz, rarr, nth, nr, zar, nzb, b, oa);
+  // z orthogonal to x and y: the separable form (its plane sums fit LDS for
+  // every grid the library plans)
+  const bool sep = b.m[2] == 0.0 && b.m[5] == 0.0 && b.m[6] == 0.0 && b.m[7] == 0.0;
+  if (sep && nz <= kRzMaxPlanes && (long long)nx * ny < (1LL << 31))
+    hipLaunchKernelGGL(k_rz_average_sep, dim3((unsigned)nr), dim3(kRzThreads),
+                       (size_t)nz * sizeof(double), s, kp, nx, ny, nz, rarr, nth, nr, zar, nzb, b,
+                       oa);
+  else
+    hipLaunchKernelGGL(k_rz_average, dim3(grid_for((long long)nr * nzb)), dim3(256), 0, s, kp, nx,
+                       ny, nz, rarr, nth, nr, zar, nzb, b, oa);
   return hipGetLastError();
 }
 

@@ -1,0 +1,75 @@
+"""The separable form of the cylindrical average (z axis orthogonal to x and y) at the edges of
+its rounds -- z planes, staged samples, z bins off the grid's own -- against the mean of the
+pointwise interpolant over the same samples (plot2d.py:605-627)."""
+import math
+
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+# a mean of up to 1,500 positive samples, each a sum of 8 products: either order of the additions
+# is within (1500 + 16) eps of the exact value, the two within twice that
+RTOL = 2 * 1516 * 2.0 ** -53
+
+
+def _average(kp, rarr, nth, zar, binv):
+    from mdsf import _lib
+    lib = _lib.load()
+    nx, ny, nz = kp.shape[:3]
+    r, z = (torch.tensor(v, dtype=torch.float64, device="cuda") for v in (rarr, zar))
+    n = torch.tensor(nth, dtype=torch.int32, device="cuda")
+    oa = torch.empty(len(rarr), len(zar), dtype=torch.float64, device="cuda")
+    p = _lib.c_void_p
+    b = np.ascontiguousarray(binv)
+    _lib.check(lib.mdsf_rz_average(p(kp.data_ptr()), nx, ny, nz, p(r.data_ptr()), p(n.data_ptr()),
+                                   len(rarr), p(z.data_ptr()), len(zar),
+                                   b.ctypes.data_as(_lib.ctypes.POINTER(_lib.c_double)),
+                                   p(oa.data_ptr()), p(torch.cuda.current_stream().cuda_stream)))
+    return oa
+
+
+@pytest.mark.parametrize("n,nzb,nth", [
+    ((6, 5, 2), 3, [1, 2, 3]),
+    ((9, 12, 255), 255, [1, 5, 64]),
+    ((8, 7, 256), 300, [3, 1023, 1024]),
+    ((7, 9, 257), 64, [1025, 4, 1500]),
+    ((5, 6, 1024), 17, [7, 1, 2]),
+    ((5, 6, 1025), 17, [7, 1, 2]),      # past the plane sums in LDS: the general form
+])
+@pytest.mark.parametrize("theta", [90, 120])
+def test_rz_average_matches_pointwise_mean(gpu, n, nzb, nth, theta):
+    from mdsf import engine
+    g = torch.Generator().manual_seed(sum(n))
+    ax = [torch.linspace(-1.0 - 0.1 * d, 1.3 + 0.2 * d, m, dtype=torch.float64)
+          for d, m in enumerate(n)]
+    kp = torch.stack(torch.meshgrid(*ax, indexing="ij")
+                     + (torch.rand(n, dtype=torch.float64, generator=g) + 0.25,), -1).cuda()
+    t = math.radians(theta)
+    binv = np.array([[1.0, 0, 0], [math.cos(t) if theta != 90 else 0.0, math.sin(t), 0], [0, 0, 1]])
+    rarr = [0.0, 0.6, 0.8][:len(nth)]
+    # one z past the grid: a NaN column
+    zar = np.concatenate([np.linspace(float(ax[2][0]), float(ax[2][-1]), nzb - 1),
+                          [float(ax[2][-1]) + 0.1]])
+    got = _average(kp, rarr, nth, zar, binv)
+    b = torch.from_numpy(binv).cuda()
+    for i, (r, m) in enumerate(zip(rarr, nth)):
+        th = torch.arange(m, dtype=torch.float64, device="cuda") * (2 * math.pi / m)
+        p = torch.empty(m, nzb, 3, dtype=torch.float64, device="cuda")
+        p[..., 0], p[..., 1] = (r * th.cos())[:, None], (r * th.sin())[:, None]
+        p[..., 2] = torch.from_numpy(zar).cuda()
+        want = engine.interp_points(kp, (p.reshape(-1, 3) @ b).reshape(m, nzb, 3)).mean(0)
+        assert bool(torch.isnan(got[i, -1])) and bool(torch.isnan(want[-1]))
+        # the sample points of the two forms agree to a few ulp, their values to the local slope
+        torch.testing.assert_close(got[i, :-1], want[:-1], rtol=RTOL, atol=200 * 2.0 ** -53)
+
+
+def test_rz_average_ring_off_the_grid_is_nan(gpu):
+    ax = [torch.linspace(-1, 1, m, dtype=torch.float64) for m in (5, 6, 7)]
+    kp = torch.stack(torch.meshgrid(*ax, indexing="ij") + (torch.ones(5, 6, 7, dtype=torch.float64),),
+                     -1).cuda()
+    got = _average(kp, [0.5, 1.2], [8, 8], [-0.5, 0.0, 0.5], np.eye(3))
+    torch.testing.assert_close(got[0], torch.ones(3, dtype=torch.float64, device="cuda"), rtol=1e-14,
+                               atol=0)
+    assert bool(torch.isnan(got[1]).all())
