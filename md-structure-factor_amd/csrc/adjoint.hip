@@ -18,6 +18,7 @@
 // values are broadcast with readlane.  Items write 3 FP64 partial sums; a
 // second kernel adds each atom's partials in a fixed order (deterministic).
 #include "clip.h"
+#include "halfgrid.h"
 #include "mdsf_internal.h"
 #include "spill.h"
 #include "tiles.h"
@@ -345,19 +346,15 @@ __global__ void k_fill_zero(double* __restrict__ p, long long n) {
 
 // w_main[kz][y][x] = 2 g[x, y, kz] (kz < m), w_nyq[x][y] = 2 g[x, y, m]: the
 // layouts the FFT keeps its spectrum and S(q) in
-__global__ void k_adjoint_weights(const double* __restrict__ g, double* __restrict__ wmain,
-                                  double* __restrict__ wnyq, int nx, int ny, int m) {
-  const long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x;
-  const long long nxy = (long long)nx * ny;
-  if (i >= nxy * (m + 1)) return;
-  const long long xy = i / (m + 1);
-  const int kz = (int)(i - xy * (m + 1));
-  if (kz < m) {
-    const long long x = xy / ny, y = xy - x * ny;
-    wmain[((long long)kz * ny + y) * nx + x] = 2.0 * g[i];
-  } else {
-    wnyq[xy] = 2.0 * g[i];
-  }
+__global__ __launch_bounds__(kHalfThreads) void k_adjoint_weights(const double* __restrict__ g,
+                                                                  double* __restrict__ wmain,
+                                                                  double* __restrict__ wnyq, int nx,
+                                                                  int ny, int m) {
+  rows_to_half<double>(
+      nx, ny, m,
+      [&](int x, int y, int kz) { return 2.0 * g[((long long)x * ny + y) * (m + 1) + kz]; },
+      [&](int kz, int y, int x, double v) { wmain[((long long)kz * ny + y) * nx + x] = v; },
+      [&](int x, int y, double v) { wnyq[(long long)x * ny + y] = v; });
 }
 
 }  // namespace
@@ -371,9 +368,9 @@ hipError_t launch_fill_zero(double* p, long long n, hipStream_t s) {
 hipError_t launch_adjoint_weights(Plan& p, const double* dsf, hipStream_t s) {
   const long long nxy = (long long)p.sys.n[0] * p.sys.n[1];
   const int m = p.sys.n[2] / 2;
-  const long long n = nxy * (m + 1);
-  hipLaunchKernelGGL(k_adjoint_weights, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, dsf,
-                     p.adj_w, p.adj_w + nxy * m, p.sys.n[0], p.sys.n[1], m);
+  hipLaunchKernelGGL(k_adjoint_weights, dim3(half_tiles(p.sys.n[0], p.sys.n[1], m)),
+                     dim3(kHalfThreads), 0, s, dsf, p.adj_w, p.adj_w + nxy * m, p.sys.n[0],
+                     p.sys.n[1], m);
   return hipGetLastError();
 }
 

@@ -36,6 +36,7 @@
 
 #include <hip/hip_ext.h>
 
+#include "halfgrid.h"
 #include "mdsf_internal.h"
 
 namespace mdsf {
@@ -1509,23 +1510,17 @@ hipError_t inverse_impl(Plan& p, const double* w_main, const double* w_nyq, void
 
 // stored spectrum (rho[kz][ky][kx] complex, nyq[x][y] FP64) -> complex128 (Nx, Ny, Nz/2+1)
 template <typename R>
-__global__ void k_spec_read(const typename V2<R>::T* __restrict__ main,
-                            const double2* __restrict__ nyq, double2* __restrict__ out, int nx,
-                            int ny, int m) {
-  const long long h = m + 1;
-  const long long total = (long long)nx * ny * h;
-  for (long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x; i < total;
-       i += (long long)gridDim.x * blockDim.x) {
-    const long long row = i / h;
-    const int kz = (int)(i - row * h);
-    const int y = (int)(row % ny), x = (int)(row / ny);
-    if (kz < m) {
-      const auto v = main[((long long)kz * ny + y) * nx + x];
-      out[i] = make_double2((double)v.x, (double)v.y);
-    } else {
-      out[i] = nyq[row];
-    }
-  }
+__global__ __launch_bounds__(kHalfThreads) void k_spec_read(
+    const typename V2<R>::T* __restrict__ main, const double2* __restrict__ nyq,
+    double2* __restrict__ out, int nx, int ny, int m) {
+  half_to_rows<double2>(
+      nx, ny, m,
+      [&](int kz, int y, int x) {
+        const auto v = main[((long long)kz * ny + y) * nx + x];
+        return make_double2((double)v.x, (double)v.y);
+      },
+      [&](int x, int y) { return nyq[(long long)x * ny + y]; },
+      [&](int x, int y, int kz, double2 v) { out[((long long)x * ny + y) * (m + 1) + kz] = v; });
 }
 
 }  // namespace
@@ -1711,16 +1706,12 @@ hipError_t fft_pass(Plan& p, int pass, const void* density, hipStream_t s) {
 
 hipError_t fft_spectrum_read(Plan& p, double* out, hipStream_t s) {
   const int nx = p.sys.n[0], ny = p.sys.n[1], m = p.sys.n[2] / 2;
-  long long total = (long long)nx * ny * (m + 1);
-  long long blocks = (total + 255) / 256;
-  if (blocks > 65536) blocks = 65536;
+  const dim3 grid(half_tiles(nx, ny, m)), block(kHalfThreads);
   if (p.fft64)
-    hipLaunchKernelGGL(k_spec_read<double>, dim3((unsigned)blocks), dim3(256), 0, s,
-                       cx<double>(p.rho), static_cast<const double2*>(p.spec_nyq),
+    hipLaunchKernelGGL(k_spec_read<double>, grid, block, 0, s, cx<double>(p.rho), static_cast<const double2*>(p.spec_nyq),
                        reinterpret_cast<double2*>(out), nx, ny, m);
   else
-    hipLaunchKernelGGL(k_spec_read<float>, dim3((unsigned)blocks), dim3(256), 0, s,
-                       cx<float>(p.rho), static_cast<const double2*>(p.spec_nyq),
+    hipLaunchKernelGGL(k_spec_read<float>, grid, block, 0, s, cx<float>(p.rho), static_cast<const double2*>(p.spec_nyq),
                        reinterpret_cast<double2*>(out), nx, ny, m);
   return hipGetLastError();
 }

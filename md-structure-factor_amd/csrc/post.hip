@@ -6,6 +6,7 @@
 //   fold of a padded grid (remap_grid[_tcl])   dens.py:65-108
 #include <cmath>
 
+#include "halfgrid.h"
 #include "mdsf_internal.h"
 
 namespace mdsf {
@@ -14,17 +15,14 @@ namespace {
 
 // sf (Nx, Ny, Nz/2+1) from the accumulators sf_main[kz][ky][kx] (kz < Nz/2)
 // and sf_nyq[kx][ky]
-__global__ void k_sf_read(const double* __restrict__ sfm, const double* __restrict__ sfn,
-                          double* __restrict__ out, int nx, int ny, int m) {
-  const long long h = m + 1;
-  const long long total = (long long)nx * ny * h;
-  for (long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x; i < total;
-       i += (long long)gridDim.x * blockDim.x) {
-    const long long row = i / h;
-    const int kz = (int)(i - row * h);
-    const long long x = row / ny, y = row - x * ny;
-    out[i] = kz < m ? sfm[((long long)kz * ny + y) * nx + x] : sfn[row];
-  }
+__global__ __launch_bounds__(kHalfThreads) void k_sf_read(const double* __restrict__ sfm,
+                                                          const double* __restrict__ sfn,
+                                                          double* __restrict__ out, int nx, int ny,
+                                                          int m) {
+  half_to_rows<double>(
+      nx, ny, m, [&](int kz, int y, int x) { return sfm[((long long)kz * ny + y) * nx + x]; },
+      [&](int x, int y) { return sfn[(long long)x * ny + y]; },
+      [&](int x, int y, int kz, double v) { out[((long long)x * ny + y) * (m + 1) + kz] = v; });
 }
 
 __device__ __forceinline__ int pm(int a, int n) {
@@ -398,8 +396,8 @@ hipError_t launch_fold_padded(const double* d0, const int n[3], const int nb[3],
 
 hipError_t launch_sf_read(const Plan& p, double* sf, hipStream_t s) {
   const int nx = p.sys.n[0], ny = p.sys.n[1], m = p.sys.n[2] / 2;
-  hipLaunchKernelGGL(k_sf_read, dim3(grid_for((long long)nx * ny * (m + 1))), dim3(256), 0, s,
-                     p.sf_main, p.sf_nyq, sf, nx, ny, m);
+  hipLaunchKernelGGL(k_sf_read, dim3(half_tiles(nx, ny, m)), dim3(kHalfThreads), 0, s, p.sf_main,
+                     p.sf_nyq, sf, nx, ny, m);
   return hipGetLastError();
 }
 
