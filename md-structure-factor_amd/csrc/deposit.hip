@@ -1372,43 +1372,57 @@ __global__ __launch_bounds__(kThreads) void k_tile_count(SysDev sys, const TypeD
   if (tid == 0) heads[tl.idx] = make_int4(0, 0, 0, nc);
 }
 
-// Region starts: exclusive scan of the region sizes in tile order (one
-// block, 4 tiles per thread and round).
+// Region starts: exclusive scan of the region sizes in tile order, 4 tiles per
+// thread and kTileScanTiles per block; a block adds up the sizes before its own
+// tiles itself.  One block running in rounds is a serial chain of load latencies:
+// 446 us for the 32,768 tiles of a 512^3 grid beside the other prepare branches
+// (6 us for 4,096, where this is one block too).  Sums per chunk of tiles kept
+// with atomics by k_tile_count, so that k_tile_lists could place its region
+// without a scan, cost the 256^3 frame loop 10%.
 constexpr int kTileScanThreads = 1024;
+constexpr int kTileScanTiles = 4 * kTileScanThreads;
 __global__ __launch_bounds__(kTileScanThreads) void k_tile_scan(int4* __restrict__ heads,
                                                                 int ntiles) {
   __shared__ int wsum[kTileScanThreads / 64];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  int carry = 0;
-  for (int r0 = 0; r0 < ntiles; r0 += 4 * kTileScanThreads) {
-    const int i0 = r0 + 4 * tid;
-    int v[4];
+  // sum over the block of one int per thread, in every thread
+  auto block_sum = [&](int x) {
 #pragma unroll
-    for (int k = 0; k < 4; ++k) v[k] = i0 + k < ntiles ? heads[i0 + k].w : 0;
-    const int sum = v[0] + v[1] + v[2] + v[3];
-    int x = sum;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-      const int y = __shfl_up(x, o, 64);
-      if (lane >= o) x += y;
-    }
-    if (lane == 63) wsum[wave] = x;
+    for (int o = 32; o > 0; o >>= 1) x += __shfl_xor(x, o, 64);
+    if (lane == 0) wsum[wave] = x;
     __syncthreads();
-    int off = 0, tot = 0;
+    int tot = 0;
 #pragma unroll
-    for (int w = 0; w < kTileScanThreads / 64; ++w) {
-      const int s = wsum[w];
-      off += w < wave ? s : 0;
-      tot += s;
-    }
-    int run = carry + off + x - sum;
+    for (int w = 0; w < kTileScanThreads / 64; ++w) tot += wsum[w];
+    __syncthreads();
+    return tot;
+  };
+  const int r0 = (int)blockIdx.x * kTileScanTiles;
+  int before = 0;
+#pragma unroll 8
+  for (int i = tid; i < r0; i += kTileScanThreads) before += heads[i].w;
+  const int carry = r0 > 0 ? block_sum(before) : 0;   // uniform branch
+  const int i0 = r0 + 4 * tid;
+  int v[4];
 #pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      if (i0 + k < ntiles) heads[i0 + k].x = run;
-      run += v[k];
-    }
-    carry += tot;
-    __syncthreads();  // wsum is rewritten by the next round
+  for (int k = 0; k < 4; ++k) v[k] = i0 + k < ntiles ? heads[i0 + k].w : 0;
+  const int sum = v[0] + v[1] + v[2] + v[3];
+  int x = sum;
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const int y = __shfl_up(x, o, 64);
+    if (lane >= o) x += y;
+  }
+  if (lane == 63) wsum[wave] = x;
+  __syncthreads();
+  int off = 0;
+#pragma unroll
+  for (int w = 0; w < kTileScanThreads / 64; ++w) off += w < wave ? wsum[w] : 0;
+  int run = carry + off + x - sum;
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    if (i0 + k < ntiles) heads[i0 + k].x = run;
+    run += v[k];
   }
 }
 
@@ -2406,7 +2420,8 @@ hipError_t launch_tile_regions(Plan& p, hipStream_t s) {
   else
     hipLaunchKernelGGL(k_tile_count<kMaxTypes>, grid, block, 0, s, sys, p.types, p.bucket_count,
                        p.tl_head);
-  hipLaunchKernelGGL(k_tile_scan, dim3(1), dim3(kTileScanThreads), 0, s, p.tl_head, (int)ntiles);
+  hipLaunchKernelGGL(k_tile_scan, dim3((unsigned)((ntiles + kTileScanTiles - 1) / kTileScanTiles)),
+                     dim3(kTileScanThreads), 0, s, p.tl_head, (int)ntiles);
   return hipGetLastError();
 }
 
