@@ -69,6 +69,12 @@ __global__ __launch_bounds__(kAdjThreads) void k_deposit_adjoint(
     const double* __restrict__ s_r, const int* __restrict__ nvalid, const R* __restrict__ grho,
     double* __restrict__ part, long long nitems) {
   const int lane = threadIdx.x & 63;
+  const int fr = blockIdx.y;   // frame of the group
+  s_ir += fr * sys.f_atoms();
+  s_r += 3 * fr * sys.f_atoms();
+  nvalid += fr * sys.f_buckets();
+  grho += fr * sys.f_points;
+  part += 3 * fr * sys.f_adji;
   // XCD-aware order: workgroups go round-robin over the 8 XCDs, so block b
   // takes the b/8-th group of XCD (b mod 8)'s contiguous share of the items.
   // Items follow the atoms' (type, home bucket) order, so each XCD's L2 sees
@@ -190,6 +196,15 @@ __global__ void k_adjoint_reduce(SysDev sys, const TypeDev* __restrict__ td,
                                  const double* __restrict__ scale3, const double* __restrict__ s_r,
                                  const R* __restrict__ grho, double* __restrict__ grad) {
   const int s = blockIdx.x * blockDim.x + threadIdx.x;
+  const int fr = blockIdx.y;   // frame of the group
+  s_ir += fr * sys.f_atoms();
+  s_idx += fr * sys.f_atoms();
+  s_r += 3 * fr * sys.f_atoms();
+  nvalid += fr * sys.f_buckets();
+  part += 3 * fr * sys.f_adji;
+  grho += fr * sys.f_points;
+  grad += 3 * fr * sys.f_atoms();
+  if (scale3) scale3 += 3 * fr;
   if (s >= *nvalid) return;
   const int4 q = s_ir[s];
   const int t = q.w & 0xffff;
@@ -236,6 +251,15 @@ __global__ void k_adjoint_tile_reduce(SysDev sys, const TypeDev* __restrict__ td
                                       const float* __restrict__ grho, double* __restrict__ grad) {
   const long long g = blockIdx.x * (long long)blockDim.x + threadIdx.x;
   const int s = (int)(g / kRedLanes), li = (int)(g % kRedLanes);
+  const int fr = blockIdx.y;   // frame of the group
+  s_ir += fr * sys.f_atoms();
+  s_idx += fr * sys.f_atoms();
+  s_r += 3 * fr * sys.f_atoms();
+  nvalid += fr * sys.f_buckets();
+  tpart += 3 * fr * sys.f_adjt;
+  grho += fr * sys.f_points;
+  grad += 3 * fr * sys.f_atoms();
+  if (scale3) scale3 += 3 * fr;
   // every lane of a 16-lane group takes the same branch, so the shuffles
   // below run with the whole group
   bool act = s < *nvalid;
@@ -379,20 +403,20 @@ hipError_t launch_deposit_adjoint(Plan& p, const void* grho, const double* scale
   const int n = p.sys.natoms;
   if (n == 0) return hipSuccess;
   hipError_t e = hipSuccess;
-  if (!grad_zeroed && (e = launch_fill_zero(grad, 3LL * n, s)) != hipSuccess) return e;
+  if (!grad_zeroed && (e = launch_fill_zero(grad, 3LL * n * p.nfr, s)) != hipSuccess) return e;
   const int* nvalid = p.bucket_off + p.sys.nbuckets;
   if (p.adj_tslots > 0 && p.adj_tpart && p.dslices) {
     // FP32 orthogonal cells: MFMA transpose of the tiled deposition
     if (!derivs_ready && (e = launch_slice_derivs(p, s)) != hipSuccess) return e;
     if ((e = launch_adjoint_tiles(p, static_cast<const float*>(grho), s)) != hipSuccess) return e;
     hipLaunchKernelGGL(k_adjoint_tile_reduce,
-                       dim3((unsigned)(((long long)n * kRedLanes + 255) / 256)), dim3(256), 0, s,
+                       dim3((unsigned)(((long long)n * kRedLanes + 255) / 256), p.nfr), dim3(256), 0, s,
                        p.sys, p.types, p.s_ir, p.s_idx, nvalid, p.adj_tpart, scale3, p.s_r,
                        static_cast<const float*>(grho), grad);
     return hipGetLastError();
   }
   if (p.adj_items > 0) {
-    const dim3 grid((unsigned)((p.adj_items + 3) / 4)), block(kAdjThreads);
+    const dim3 grid((unsigned)((p.adj_items + 3) / 4), p.nfr), block(kAdjThreads);
     if (p.fft64) {
       if (p.sys.mode == MODE_XY)
         hipLaunchKernelGGL((k_deposit_adjoint<MODE_XY, double>), grid, block, 0, s, p.sys,
@@ -416,11 +440,11 @@ hipError_t launch_deposit_adjoint(Plan& p, const void* grho, const double* scale
     if (e != hipSuccess) return e;
   }
   if (p.fft64)
-    hipLaunchKernelGGL(k_adjoint_reduce<double>, dim3((n + 255) / 256), dim3(256), 0, s, p.sys,
+    hipLaunchKernelGGL(k_adjoint_reduce<double>, dim3((n + 255) / 256, p.nfr), dim3(256), 0, s, p.sys,
                        p.types, p.s_ir, p.s_idx, nvalid, p.adj_part, scale3, p.s_r,
                        static_cast<const double*>(grho), grad);
   else
-    hipLaunchKernelGGL(k_adjoint_reduce<float>, dim3((n + 255) / 256), dim3(256), 0, s, p.sys,
+    hipLaunchKernelGGL(k_adjoint_reduce<float>, dim3((n + 255) / 256, p.nfr), dim3(256), 0, s, p.sys,
                        p.types, p.s_ir, p.s_idx, nvalid, p.adj_part, scale3, p.s_r,
                        static_cast<const float*>(grho), grad);
   return hipGetLastError();

@@ -72,7 +72,10 @@ hipError_t enqueue_system(Batch& b, int i, hipStream_t s) {
   if (e == hipSuccess) e = launch_fill_zero(p.sf_nyq, nxy, s);
   const size_t esz = f.dtype == MDSF_F32 ? 4 : 8;
   const size_t fstride = (size_t)p.sys.natoms * 3 * esz;
-  for (int64_t t = 0; t < f.nframes && e == hipSuccess; ++t) {
+  const int64_t ngroups = (f.nframes + p.group - 1) / p.group;
+  int64_t t = 0;
+  for (int64_t k = 0; k < ngroups && e == hipSuccess; ++k) {
+    p.nfr = (int)((f.nframes - t) / (ngroups - k));   // groups of nearly equal size
     void* c = const_cast<char*>(static_cast<const char*>(f.coords)) + (size_t)t * fstride;
     e = launch_prep(p, c, f.dtype, f.arith, f.types, f.scale + 3 * t, f.box, f.wrap_lo, f.wrap_hi,
                     nullptr, nullptr, s, false, /*write_back=*/false);
@@ -80,7 +83,9 @@ hipError_t enqueue_system(Batch& b, int i, hipStream_t s) {
     if (e == hipSuccess) e = launch_deposit(p, p.rho, s);
     if (e == hipSuccess) e = launch_parked(p, p.rho, s);
     if (e == hipSuccess) e = fft_forward(p, p.rho, true, s);
+    t += p.nfr;
   }
+  p.nfr = 1;
   return e;
 }
 

@@ -41,6 +41,39 @@ hipError_t dalloc(T** p, size_t count) {
   return hipMalloc(reinterpret_cast<void**>(p), count * sizeof(T));
 }
 
+// A plan's buffers, cut from one device allocation: a hipMalloc and a hipMemset
+// each for some 80 buffers were most of a small plan's set-up.  Buffers that start
+// at zero come first, so that one fill clears them.
+struct Arena {
+  struct Item {
+    void** p;
+    size_t bytes;
+    bool zero;
+  };
+  std::vector<Item> items;
+  template <typename T>
+  void add(T** p, size_t count, bool zero = false) {
+    *p = nullptr;
+    items.push_back({reinterpret_cast<void**>(p), std::max(count, (size_t)1) * sizeof(T), zero});
+  }
+  hipError_t take(void** base) {
+    size_t off = 0, cleared = 0;
+    std::vector<size_t> at(items.size());
+    for (const bool zero : {true, false}) {
+      for (size_t i = 0; i < items.size(); ++i) {
+        if (items[i].zero != zero) continue;
+        at[i] = off;
+        off = (off + items[i].bytes + 511) & ~(size_t)511;
+      }
+      if (zero) cleared = off;
+    }
+    hipError_t e = hipMalloc(base, std::max(off, (size_t)1));
+    if (e != hipSuccess) return e;
+    for (size_t i = 0; i < items.size(); ++i) *items[i].p = static_cast<char*>(*base) + at[i];
+    return cleared ? hipMemset(*base, 0, cleared) : hipSuccess;
+  }
+};
+
 // The frame pipeline's three streams (deposition, FFT, and the tile-list
 // branch of the prepare stage), one set per device shared by every plan and
 // kept until the process ends.  HIP gives a process few hardware queues
@@ -84,46 +117,41 @@ void free_plan(Plan* p) {
     for (hipEvent_t e : {p->ev_prep[b], p->ev_dep[b], p->ev_fft[b]})
       if (e) (void)hipEventDestroy(e);
   for (hipEvent_t e : p->tev) (void)hipEventDestroy(e);
-  for (FrameState& f : p->slot) {
-    void* fs[] = {f.ir4,   f.key,   f.rpos, f.bucket_count, f.bucket_off, f.bucket_cur,
-                  f.bucket_aux, f.s_tmp, f.s_idx, f.s_ir, f.s_r, f.tables, f.slices,
-                  f.dslices, f.bslices, f.corners, f.spill, f.spill_flag, f.tl_pool,
-                  f.tl_head};
-    for (void* q : fs)
-      if (q) (void)hipFree(q);
-  }
-  for (int b = 0; b < kSlots; ++b)
-    for (void* q : {p->rho_buf[b], p->nyq_buf[b], p->spec_buf[b], p->res_buf[b]})
-      if (q) (void)hipFree(q);
-  void* ptrs[] = {p->types,     p->err,       p->sf_main,
-                  p->sf_nyq,    p->ax_x.tw,   p->ax_y.tw,    p->ax_zc.tw,   p->ax_x.tw64,
-                  p->ax_y.tw64, p->ax_zc.tw64, p->tw_r2c,    p->tw_r2c64,   p->adj_part,
-                  p->adj_w,     p->adj_tpart};
-  for (void* q : ptrs)
+  for (FrameState& f : p->slot)
+    if (f.dslices) (void)hipFree(f.dslices);
+  for (void* q : {static_cast<void*>(p->adj_part), static_cast<void*>(p->adj_w),
+                  static_cast<void*>(p->adj_tpart), p->arena})
     if (q) (void)hipFree(q);
   delete p;
 }
 
-int make_axis(FftAxis& ax, int n, hipStream_t s) {
+int make_axis(FftAxis& ax, int n, Arena& arena) {
   ax.n = n;
   if (!fft_factor(n, ax.radix, &ax.nstages))
     return fail(MDSF_ERR_UNSUPPORTED, "FFT length " + std::to_string(n) + " needs too many stages");
-  MDSF_HIP(dalloc(&ax.tw, (size_t)n));
-  MDSF_HIP(dalloc(&ax.tw64, (size_t)n));
-  MDSF_HIP(fft_make_twiddles(ax.tw, ax.tw64, n, s));
+  arena.add(&ax.tw, (size_t)n);
+  arena.add(&ax.tw64, (size_t)n);
   return MDSF_OK;
 }
+
+// Sets the frames the plan's launches cover, and one again when it goes.
+struct FrameGroup {
+  Plan& p;
+  explicit FrameGroup(Plan& plan) : p(plan) {}
+  ~FrameGroup() { p.nfr = 1; }
+};
 
 int ensure_adjoint(Plan& p) {
   const size_t nxy = (size_t)p.sys.n[0] * p.sys.n[1];
   const size_t m = (size_t)p.sys.n[2] / 2;
-  if (!p.adj_part) MDSF_HIP(dalloc(&p.adj_part, 3 * (size_t)std::max(p.adj_items, 1LL)));
+  const size_t g = (size_t)p.group;
+  if (!p.adj_part) MDSF_HIP(dalloc(&p.adj_part, 3 * g * (size_t)std::max(p.adj_items, 1LL)));
   if (!p.adj_w) MDSF_HIP(dalloc(&p.adj_w, nxy * (m + 1)));
   if (p.adj_tslots > 0 && !p.adj_tpart) {
     // tiled adjoint: slice derivatives per frame slot and the result slots
     for (FrameState& f : p.slot)
-      if (!f.dslices) MDSF_HIP(dalloc(&f.dslices, (size_t)p.slice_floats));
-    MDSF_HIP(dalloc(&p.adj_tpart, 3 * (size_t)p.adj_tslots));
+      if (!f.dslices) MDSF_HIP(dalloc(&f.dslices, g * (size_t)p.slice_floats));
+    MDSF_HIP(dalloc(&p.adj_tpart, 3 * g * (size_t)p.adj_tslots));
     p.use_slot(p.cur_slot);
   }
   return MDSF_OK;
@@ -353,7 +381,32 @@ int mdsf_plan_create(const mdsf_grid_desc* desc, mdsf_plan** out) {
   }
   (void)hipGetDevice(&p->device);
 
-  const size_t nat = (size_t)desc->natoms;
+  // frames per group (kGroupTiles), within the state budget
+  s.f_slices = p->slice_floats;
+  s.f_bslices = p->bslice_floats;
+  s.f_tables = p->fft64 ? table_floats : 0;
+  const bool staged = p->spill_tiles > 0 && p->spill_tiles <= kMaxSpillBufTiles;
+  s.f_spill = staged ? p->spill_tiles * kTile * kTile * kTile : 0;
+  s.f_points = (long long)desc->n[0] * desc->n[1] * desc->n[2];
+  s.f_adjt = p->adj_tslots;
+  s.f_adji = p->adj_items;
+  s.f_pool = (int)p->tl_cap;
+  s.f_aux = s.nbuckets / 1024 + 2;
+  s.f_tiles = s.ntiles[0] * s.ntiles[1] * s.ntiles[2];
+  {
+    const size_t rs = p->fft64 ? 8 : 4;
+    const size_t bytes = (size_t)desc->natoms * 112 + (size_t)s.nbuckets * 12 +
+                         (size_t)p->slice_floats * 4 + (size_t)p->bslice_floats * 4 +
+                         (size_t)s.f_tables * 8 + (size_t)s.f_spill * rs + (size_t)p->tl_cap * 8 +
+                         (size_t)s.f_points * rs + fft_spec_bytes(s.n, p->fft64) +
+                         fft_res_bytes(s.n, p->fft64) + (size_t)desc->n[0] * desc->n[1] * 16;
+    const long long fit = (long long)(kGroupBytes / (kSlots * bytes));
+    const long long want = (kGroupTiles + s.f_tiles - 1) / s.f_tiles;
+    p->group = (int)std::max(1LL, std::min({want, fit, (long long)kMaxGroup}));
+  }
+  const size_t grp = (size_t)p->group;
+
+  const size_t nat = grp * (size_t)desc->natoms;
   const size_t nx = desc->n[0], ny = desc->n[1], nz = desc->n[2];
   const size_t m = nz / 2;
   hipError_t e = hipSuccess;
@@ -366,86 +419,66 @@ int mdsf_plan_create(const mdsf_grid_desc* desc, mdsf_plan** out) {
       return rc;                        \
     }                                   \
   } while (0)
-  TRY(dalloc(&p->types, (size_t)kMaxTypes));
-  TRY(hipMemcpy(p->types, p->types_host, sizeof(TypeDev) * kMaxTypes, hipMemcpyHostToDevice));
+  Arena arena;
+  arena.add(&p->types, (size_t)kMaxTypes);
   for (FrameState& f : p->slot) {
-    TRY(dalloc(&f.ir4, nat));
-    TRY(dalloc(&f.key, nat));
-    TRY(dalloc(&f.rpos, 3 * nat));
-    TRY(dalloc(&f.bucket_count, (size_t)s.nbuckets + 1));
-    TRY(dalloc(&f.bucket_off, (size_t)s.nbuckets + 1));
-    TRY(dalloc(&f.bucket_cur, (size_t)s.nbuckets + 1));
-    TRY(dalloc(&f.bucket_aux, (size_t)s.nbuckets / 1024 + 2));
-    TRY(hipMemset(f.bucket_count, 0, sizeof(int) * ((size_t)s.nbuckets + 1)));
-    TRY(hipMemset(f.bucket_off, 0, sizeof(int) * ((size_t)s.nbuckets + 1)));
-    TRY(dalloc(&f.s_idx, nat));
-    TRY(dalloc(&f.s_tmp, nat));
-    TRY(dalloc(&f.s_ir, nat));
-    TRY(dalloc(&f.s_r, 3 * nat));
-    if (p->fft64) {
-      double* tb = nullptr;
-      TRY(dalloc(&tb, (size_t)table_floats));
-      f.tables = tb;
-    } else {
-      float* tb = nullptr;  // unused: the FP32 path stages tile slices instead
-      TRY(dalloc(&tb, (size_t)1));
-      f.tables = tb;
-    }
-    TRY(dalloc(&f.slices, (size_t)p->slice_floats));
-    if (p->bslice_floats > 0) TRY(dalloc(&f.bslices, (size_t)p->bslice_floats));
-    TRY(dalloc(&f.corners, (size_t)2 + 2 * kCornerCap));
-    TRY(hipMemset(f.corners, 0, sizeof(int) * ((size_t)2 + 2 * kCornerCap)));
-    if (p->spill_tiles > 0 && p->spill_tiles <= kMaxSpillBufTiles) {
-      unsigned char* sb = nullptr;
-      TRY(dalloc(&sb, (size_t)p->spill_tiles * kTile * kTile * kTile * (p->fft64 ? 8 : 4)));
-      f.spill = sb;
-      TRY(dalloc(&f.spill_flag, (size_t)p->spill_tiles));
+    arena.add(&f.ir4, nat);
+    arena.add(&f.key, nat);
+    arena.add(&f.rpos, 3 * nat);
+    const size_t nbk = grp * ((size_t)s.nbuckets + 1);
+    arena.add(&f.bucket_count, nbk, true);
+    arena.add(&f.bucket_off, nbk, true);
+    arena.add(&f.bucket_cur, nbk);
+    arena.add(&f.bucket_aux, grp * (size_t)s.f_aux);
+    arena.add(&f.s_idx, nat);
+    arena.add(&f.s_tmp, nat);
+    arena.add(&f.s_ir, nat);
+    arena.add(&f.s_r, 3 * nat);
+    // (the FP32 path stages tile slices instead of tables)
+    arena.add(reinterpret_cast<double**>(&f.tables), p->fft64 ? grp * (size_t)table_floats : 1);
+    arena.add(&f.slices, grp * (size_t)p->slice_floats);
+    if (p->bslice_floats > 0) arena.add(&f.bslices, grp * (size_t)p->bslice_floats);
+    arena.add(&f.corners, grp * kCornerInts, true);
+    if (staged) {
+      arena.add(reinterpret_cast<unsigned char**>(&f.spill),
+                grp * (size_t)s.f_spill * (p->fft64 ? 8 : 4));
       // no tile is read before a frame's binning flags it (a frame without atoms
       // never runs the binning)
-      TRY(hipMemset(f.spill_flag, 0, sizeof(int) * (size_t)p->spill_tiles));
+      arena.add(&f.spill_flag, grp * (size_t)p->spill_tiles, true);
     }
     if (p->tl_cap > 0) {
-      TRY(dalloc(&f.tl_pool, (size_t)p->tl_cap));
-      TRY(dalloc(&f.tl_head, (size_t)s.ntiles[0] * s.ntiles[1] * s.ntiles[2]));
+      arena.add(&f.tl_pool, grp * (size_t)p->tl_cap);
+      arena.add(&f.tl_head, grp * (size_t)s.f_tiles);
     }
   }
-  TRY(dalloc(&p->err, (size_t)1));
-  TRY(hipMemset(p->err, 0, sizeof(int)));
+  arena.add(&p->err, (size_t)1, true);
   for (int b = 0; b < kSlots; ++b) {
-    unsigned char* rho = nullptr;
-    unsigned char* spec = nullptr;
-    double2* nyq = nullptr;
-    TRY(dalloc(&rho, nx * ny * nz * (p->fft64 ? 8 : 4)));
-    TRY(dalloc(&spec, fft_spec_bytes(s.n, p->fft64)));
-    TRY(dalloc(&nyq, nx * ny));
-    p->rho_buf[b] = rho;
-    p->spec_buf[b] = spec;
-    p->nyq_buf[b] = nyq;
-    if (fft_res_bytes(s.n, p->fft64) > 0) {
-      unsigned char* res = nullptr;
-      TRY(dalloc(&res, fft_res_bytes(s.n, p->fft64)));
-      p->res_buf[b] = res;
-    }
+    arena.add(reinterpret_cast<unsigned char**>(&p->rho_buf[b]),
+              grp * nx * ny * nz * (p->fft64 ? 8 : 4));
+    arena.add(reinterpret_cast<unsigned char**>(&p->spec_buf[b]), grp * fft_spec_bytes(s.n, p->fft64));
+    arena.add(reinterpret_cast<double2**>(&p->nyq_buf[b]), grp * nx * ny);
+    if (fft_res_bytes(s.n, p->fft64) > 0)
+      arena.add(reinterpret_cast<unsigned char**>(&p->res_buf[b]),
+                grp * fft_res_bytes(s.n, p->fft64));
   }
-  p->use_slot(0);
-  TRY(dalloc(&p->sf_main, nx * ny * m));
-  TRY(dalloc(&p->sf_nyq, nx * ny));
-  TRY(hipMemset(p->sf_main, 0, sizeof(double) * nx * ny * m));
-  TRY(hipMemset(p->sf_nyq, 0, sizeof(double) * nx * ny));
-#undef TRY
+  arena.add(&p->sf_main, nx * ny * m, true);
+  arena.add(&p->sf_nyq, nx * ny, true);
   int rc;
-  if ((rc = make_axis(p->ax_x, desc->n[0], nullptr)) != MDSF_OK ||
-      (rc = make_axis(p->ax_y, desc->n[1], nullptr)) != MDSF_OK ||
-      (rc = make_axis(p->ax_zc, desc->n[2] / 2, nullptr)) != MDSF_OK) {
+  if ((rc = make_axis(p->ax_x, desc->n[0], arena)) != MDSF_OK ||
+      (rc = make_axis(p->ax_y, desc->n[1], arena)) != MDSF_OK ||
+      (rc = make_axis(p->ax_zc, desc->n[2] / 2, arena)) != MDSF_OK) {
     free_plan(p);
     return rc;
   }
-  if ((e = dalloc(&p->tw_r2c, nz)) != hipSuccess || (e = dalloc(&p->tw_r2c64, nz)) != hipSuccess ||
-      (e = fft_make_twiddles(p->tw_r2c, p->tw_r2c64, (int)nz, nullptr)) != hipSuccess) {
-    rc = hip_fail(e, "r2c twiddles");
-    free_plan(p);
-    return rc;
-  }
+  arena.add(&p->tw_r2c, nz);
+  arena.add(&p->tw_r2c64, nz);
+  TRY(arena.take(&p->arena));
+  TRY(hipMemcpy(p->types, p->types_host, sizeof(TypeDev) * kMaxTypes, hipMemcpyHostToDevice));
+  for (FftAxis* ax : {&p->ax_x, &p->ax_y, &p->ax_zc})
+    TRY(fft_make_twiddles(ax->tw, ax->tw64, ax->n, nullptr));
+  TRY(fft_make_twiddles(p->tw_r2c, p->tw_r2c64, (int)nz, nullptr));
+  p->use_slot(0);
+#undef TRY
   if ((e = hipDeviceSynchronize()) != hipSuccess) {
     rc = hip_fail(e, "plan set-up");
     free_plan(p);
@@ -526,38 +559,44 @@ int mdsf_accumulate_frames(mdsf_plan* plan, void* d_coords, int dtype, int64_t n
   const size_t esz = dtype == MDSF_F32 ? 4 : 8;
   const size_t fstride = (size_t)p->sys.natoms * 3 * esz;
   // Three-stage pipeline over the kSlots frame slots (atom state + density
-  // buffer): frame t is prepared on `s` (its tile lists on aux_stream, its
-  // corner list and spill staging on dep_stream ahead of its deposition),
-  // deposited on dep_stream and transformed on fft_stream, so that while
-  // frame t is deposited frame t + 1 is prepared and earlier frames
-  // transformed.  A slot is reused kSlots frames later: preparing frame t
-  // waits until frame t - kSlots's deposition (tiled and parked passes) has
-  // read its atom state, depositing it until frame t - kSlots's FFT has
+  // buffer of a group of frames): group k is prepared on `s` (its tile lists on
+  // aux_stream, its corner list and spill staging on dep_stream ahead of its
+  // deposition), deposited on dep_stream and transformed on fft_stream, so that
+  // while group k is deposited group k + 1 is prepared and earlier groups
+  // transformed.  A slot is reused kSlots groups later: preparing group k
+  // waits until group k - kSlots's deposition (tiled and parked passes) has
+  // read its atom state, depositing it until group k - kSlots's FFT has
   // released its density buffer.  With three slots the deposition does not
-  // wait for the FFT of the frame just before the previous one (the FFT
+  // wait for the FFT of the group just before the previous one (the FFT
   // shares the GPU with the deposition and finishes later than it).  The
   // S(q) sum stays in frame order on one stream.
   hipStream_t d = p->dep_stream, f = p->fft_stream;
+  FrameGroup group(*p);
+  const int64_t ngroups = (nframes + p->group - 1) / p->group;
+  // groups of nearly equal size
+  auto first_of = [&](int64_t k) { return k * (nframes / ngroups) + std::min(k, nframes % ngroups); };
   // the prepare stage's branches go on their own streams on large grids; on
   // small ones the cross-stream waits cost more than the branches overlap
   const long long ntiles = (long long)p->sys.ntiles[0] * p->sys.ntiles[1] * p->sys.ntiles[2];
   const bool split = ntiles >= kSplitPrepTiles;
-  const bool pair = nframes >= 2 && fft_x_pairs(*p);
-  // timed frames accumulate over calls until mdsf_stage_times reads them
-  // (frame t of this call is timed frame tb + t), so that one-frame calls
+  const bool pair = nframes >= 2 && fft_x_pairs(*p);   // plans with one frame per group
+  // timed groups accumulate over calls until mdsf_stage_times reads them
+  // (group k of this call is timed group tb + k), so that one-frame calls
   // can be queued back to back
   int64_t tb = 0;
   if (p->timing) {
-    tb = p->timed_frames < kMaxTimedFrames ? p->timed_frames : 0;
-    while ((int64_t)p->tev.size() < kTimedEvents * (tb + nframes)) {
+    if (p->timed_groups >= kMaxTimedFrames) p->timed_groups = p->timed_frames = 0;
+    tb = p->timed_groups;
+    while ((int64_t)p->tev.size() < kTimedEvents * (tb + ngroups)) {
       hipEvent_t e;
       MDSF_HIP(hipEventCreate(&e));
       p->tev.push_back(e);
     }
-    p->timed_frames = tb + nframes;
+    p->timed_groups = tb + ngroups;
+    p->timed_frames += nframes;
   }
   // timing mode 1: every stage; mode 2: only the deposition (two events per
-  // frame on its stream, the least perturbation of the overlapped loop)
+  // group on its stream, the least perturbation of the overlapped loop)
   auto mark = [&](int64_t t, int k, hipStream_t st) -> hipError_t {
     if (!p->timing || (p->timing == 2 && k != 2 && k != 3)) return hipSuccess;
     return hipEventRecord(p->tev[kTimedEvents * (tb + t) + k], st);
@@ -569,15 +608,17 @@ int mdsf_accumulate_frames(mdsf_plan* plan, void* d_coords, int dtype, int64_t n
     MDSF_HIP(hipEventRecord(p->ev_dep[b], d));
     MDSF_HIP(hipEventRecord(p->ev_fft[b], f));
   }
-  for (int64_t t = 0; t < nframes; ++t) {
+  for (int64_t t = 0; t < ngroups; ++t) {
     const int b = (int)(t % kSlots);
-    char* c = static_cast<char*>(d_coords) + (size_t)t * fstride;
-    int32_t* home = (t == nframes - 1) ? d_home_cells : nullptr;
+    const int64_t t0 = first_of(t);
+    p->nfr = (int)(first_of(t + 1) - t0);
+    char* c = static_cast<char*>(d_coords) + (size_t)t0 * fstride;
+    int32_t* home = (t == ngroups - 1) ? d_home_cells : nullptr;   // the last frame's
     p->use_slot(b);
     MDSF_HIP(hipStreamWaitEvent(s, p->ev_dep[b], 0));
     MDSF_HIP(mark(t, 0, s));
-    MDSF_HIP(launch_prep(*p, c, dtype, arith, d_types, d_scale + 3 * t, box, wrap_lo, wrap_hi,
-                         d_occupancy, home, s));
+    MDSF_HIP(launch_prep(*p, c, dtype, arith, d_types, d_scale + 3 * t0, box, wrap_lo, wrap_hi,
+                         d_occupancy, home, s, false, true, p->nfr - 1));
     // the deposition waits for the tile-list branch itself (one cross-stream
     // wait instead of two in a row through `s`, so the binning does not join
     // the branch back into `s`); under stage timing the branch records its
@@ -604,16 +645,16 @@ int mdsf_accumulate_frames(mdsf_plan* plan, void* d_coords, int dtype, int64_t n
     MDSF_HIP(de);
     // parked atoms' clipped windows: on the deposition's stream, before
     // ev_dep[b], because they read the slot's atom state, which preparing
-    // frame t + kSlots overwrites as soon as ev_dep[b] has passed
+    // group t + kSlots overwrites as soon as ev_dep[b] has passed
     MDSF_HIP(launch_parked(*p, p->rho, d));
     MDSF_HIP(hipEventRecord(p->ev_dep[b], d));
     MDSF_HIP(hipStreamWaitEvent(f, p->ev_dep[b], 0));
-    // x passes in pairs: frame t (even) waits for frame t + 1, and one launch
-    // adds both frames' |F|^2, reading and writing the FP64 sums once; frame
-    // t's slot is released with frame t + 1's (preparing and depositing frame
-    // t + kSlots wait for it).  The last two frames of a longer call are not
-    // paired: both x passes would wait for the last y pass and lengthen the
-    // call's tail by about one x pass.
+    // x passes in pairs (one frame per group): frame t (even) waits for frame
+    // t + 1, and one launch adds both frames' |F|^2, reading and writing the
+    // FP64 sums once; frame t's slot is released with frame t + 1's (preparing
+    // and depositing frame t + kSlots wait for it).  The last two frames of a
+    // longer call are not paired: both x passes would wait for the last y pass
+    // and lengthen the call's tail by about one x pass.
     auto defers = [&](int64_t u) {
       return pair && (u % 2) == 0 && (u + 2 < nframes || nframes == 2);
     };
@@ -644,7 +685,7 @@ int mdsf_accumulate_frames(mdsf_plan* plan, void* d_coords, int dtype, int64_t n
       MDSF_HIP(hipEventRecord(p->ev_fft[b], f));
     }
   }
-  MDSF_HIP(hipStreamWaitEvent(s, p->ev_fft[(nframes - 1) % kSlots], 0));
+  MDSF_HIP(hipStreamWaitEvent(s, p->ev_fft[(ngroups - 1) % kSlots], 0));
   return MDSF_OK;
 }
 
@@ -661,8 +702,11 @@ int mdsf_rescale_wrap(mdsf_plan* plan, void* d_coords, int dtype, int64_t nframe
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   const size_t esz = dtype == MDSF_F32 ? 4 : 8;
   const size_t fstride = (size_t)p->sys.natoms * 3 * esz;
-  for (int64_t t = 0; t < nframes; ++t) {
+  constexpr int64_t kMaxY = 32768;   // frames per launch (grid y; no per-frame state is used)
+  FrameGroup group(*p);
+  for (int64_t t = 0; t < nframes; t += kMaxY) {
     char* c = static_cast<char*>(d_coords) + (size_t)t * fstride;
+    p->nfr = (int)std::min(kMaxY, nframes - t);
     MDSF_HIP(launch_prep(*p, c, dtype, arith, nullptr, d_scale + 3 * t, box, wrap_lo, wrap_hi,
                          nullptr, nullptr, s, true));
   }
@@ -705,14 +749,14 @@ int mdsf_set_stage_timing(mdsf_plan* plan, int32_t enable) {
   if (!p) return fail(MDSF_ERR_ARG, "null plan");
   if (enable < 0 || enable > 2) return fail(MDSF_ERR_ARG, "stage timing mode must be 0, 1 or 2");
   p->timing = enable;
-  p->timed_frames = 0;
+  p->timed_groups = p->timed_frames = 0;
   return MDSF_OK;
 }
 
 int mdsf_stage_times(mdsf_plan* plan, double* avg_ms) {
   Plan* p = reinterpret_cast<Plan*>(plan);
   if (!p || !avg_ms) return fail(MDSF_ERR_ARG, "null argument");
-  const int64_t n = p->timed_frames;
+  const int64_t n = p->timed_groups;
   for (int k = 0; k < 5; ++k) avg_ms[k] = 0.0;
   if (n == 0) return fail(MDSF_ERR_ARG, "no timed mdsf_accumulate_frames call");
   const bool all = p->timing != 2;
@@ -735,8 +779,8 @@ int mdsf_stage_times(mdsf_plan* plan, double* avg_ms) {
       avg_ms[k] += ms;
     }
   }
-  for (int k = 0; k < 5; ++k) avg_ms[k] /= (double)n;
-  p->timed_frames = 0;
+  for (int k = 0; k < 5; ++k) avg_ms[k] /= (double)p->timed_frames;
+  p->timed_groups = p->timed_frames = 0;
   return MDSF_OK;
 }
 
@@ -828,24 +872,30 @@ int mdsf_adjoint_frames(mdsf_plan* plan, void* d_coords, int dtype, int64_t nfra
   if (nframes == 0) return MDSF_OK;
   const size_t esz = dtype == MDSF_F32 ? 4 : 8;
   const size_t fstride = (size_t)p->sys.natoms * 3 * esz;
-  // Same slot pipeline as the forward frame loop: frame t is prepared on
+  // Same slot pipeline as the forward frame loop: group t is prepared on
   // `s`, deposited on dep_stream, and transformed forward, transformed back
-  // with the weights and gathered on fft_stream.  Slot b is reused by frame
-  // t + kSlots only after frame t's gather (the last reader of its atom state
+  // with the weights and gathered on fft_stream.  Slot b is reused by group
+  // t + kSlots only after group t's gather (the last reader of its atom state
   // and density buffer) has finished.
   hipStream_t d = p->dep_stream, f = p->fft_stream;
+  FrameGroup group(*p);
+  const int64_t ngroups = (nframes + p->group - 1) / p->group;
+  auto first_of = [&](int64_t k) { return k * (nframes / ngroups) + std::min(k, nframes % ngroups); };
   MDSF_HIP(hipEventRecord(p->ev_fork, s));
   MDSF_HIP(hipStreamWaitEvent(d, p->ev_fork, 0));
   MDSF_HIP(hipStreamWaitEvent(f, p->ev_fork, 0));
   for (int b = 0; b < kSlots; ++b) MDSF_HIP(hipEventRecord(p->ev_fft[b], f));
-  for (int64_t t = 0; t < nframes; ++t) {
+  for (int64_t t = 0; t < ngroups; ++t) {
     const int b = (int)(t % kSlots);
-    char* c = static_cast<char*>(d_coords) + (size_t)t * fstride;
-    double* grad_t = d_grad + (size_t)t * p->sys.natoms * 3;
+    const int64_t t0 = first_of(t);
+    p->nfr = (int)(first_of(t + 1) - t0);
+    char* c = static_cast<char*>(d_coords) + (size_t)t0 * fstride;
+    double* grad_t = d_grad + (size_t)t0 * p->sys.natoms * 3;
     p->use_slot(b);
     MDSF_HIP(hipStreamWaitEvent(s, p->ev_fft[b], 0));
-    MDSF_HIP(launch_fill_zero(grad_t, 3LL * p->sys.natoms, s));  // off the gather's stream
-    MDSF_HIP(launch_prep(*p, c, dtype, arith, d_types, d_scale + 3 * t, box, wrap_lo, wrap_hi,
+    // off the gather's stream
+    MDSF_HIP(launch_fill_zero(grad_t, 3LL * p->sys.natoms * p->nfr, s));
+    MDSF_HIP(launch_prep(*p, c, dtype, arith, d_types, d_scale + 3 * t0, box, wrap_lo, wrap_hi,
                          nullptr, nullptr, s));
     MDSF_HIP(launch_binning(*p, s, /*derivs=*/true));
     MDSF_HIP(hipEventRecord(p->ev_prep[b], s));
@@ -856,11 +906,11 @@ int mdsf_adjoint_frames(mdsf_plan* plan, void* d_coords, int dtype, int64_t nfra
     MDSF_HIP(launch_parked(*p, p->rho, f));
     MDSF_HIP(fft_forward(*p, p->rho, false, f));
     MDSF_HIP(fft_inverse(*p, p->adj_w, w_nyq, p->rho, f));
-    MDSF_HIP(launch_deposit_adjoint(*p, p->rho, d_scale + 3 * t, grad_t, f,
+    MDSF_HIP(launch_deposit_adjoint(*p, p->rho, d_scale + 3 * t0, grad_t, f,
                                     /*derivs_ready=*/true, /*grad_zeroed=*/true));
     MDSF_HIP(hipEventRecord(p->ev_fft[b], f));
   }
-  MDSF_HIP(hipStreamWaitEvent(s, p->ev_fft[(nframes - 1) % kSlots], 0));
+  MDSF_HIP(hipStreamWaitEvent(s, p->ev_fft[(ngroups - 1) % kSlots], 0));
   return MDSF_OK;
 }
 

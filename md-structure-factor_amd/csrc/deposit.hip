@@ -636,6 +636,8 @@ template <typename ACC>
 __device__ __forceinline__ const ACC* spill_stage_tile(const SysDev& sys, const ACC* stage,
                                                        const int* flag, const Tile& tl) {
   if (!stage) return nullptr;
+  stage += blockIdx.y * sys.f_spill;
+  flag += blockIdx.y * (sys.f_spill / (T * T * T));
   const int jx = spill_index(sys, 0, tl.t0[0] / T), jy = spill_index(sys, 1, tl.t0[1] / T),
             jz = spill_index(sys, 2, tl.t0[2] / T);
   if (jx < 0 || jy < 0 || jz < 0) return nullptr;
@@ -659,6 +661,12 @@ __global__ __launch_bounds__(kThreads) void k_deposit(SysDev sys, const TypeDev*
   __shared__ EnumShared<kMaxTypes> sh;
   const int tid = threadIdx.x;
   const int wave = tid >> 6, lane = tid & 63;
+  const int fr = blockIdx.y;   // frame of the group
+  boff += fr * sys.f_buckets();
+  s_ir += fr * sys.f_atoms();
+  s_r += 3 * fr * sys.f_atoms();
+  tables = static_cast<const ACC*>(tables) + fr * sys.f_tables;
+  rho += fr * sys.f_points;
   Tile tl;
   tile_coords(sys, tl);
   const int ci = (wave & 1) * 8 + (lane & 7);
@@ -725,6 +733,11 @@ __global__ __launch_bounds__(kThreads) void k_deposit_gen(SysDev sys,
   __shared__ EnumShared<kMaxTypes> sh;
   const int tid = threadIdx.x;
   const int wave = tid >> 6, lane = tid & 63;
+  const int fr = blockIdx.y;   // frame of the group
+  boff += fr * sys.f_buckets();
+  s_ir += fr * sys.f_atoms();
+  s_r += 3 * fr * sys.f_atoms();
+  rho += fr * sys.f_points;
   Tile tl;
   tile_coords(sys, tl);
   const int ci = (wave & 1) * 8 + (lane & 7);
@@ -922,6 +935,12 @@ void k_deposit_mfma(SysDev sys, const TypeDev* __restrict__ td,
   }
   const int tid = threadIdx.x;
   const int wave = tid >> 6, lane = tid & 63;
+  const int fr = blockIdx.y;   // frame of the group
+  boff += fr * sys.f_buckets();
+  s_ir += fr * sys.f_atoms();
+  s_r += 3 * fr * sys.f_atoms();
+  slices += fr * sys.f_slices;
+  rho += fr * sys.f_points;
   Tile tl;
   tile_coords(sys, tl);
   if (tid == 0) {
@@ -1360,6 +1379,8 @@ __global__ __launch_bounds__(kThreads) void k_tile_count(SysDev sys, const TypeD
                                                          int4* __restrict__ heads) {
   __shared__ EnumShared<MT> sh;
   const int tid = threadIdx.x;
+  bcount += blockIdx.y * sys.f_buckets();
+  heads += blockIdx.y * (long long)sys.f_tiles;
   Tile tl;
   tile_coords(sys, tl);
   const int total_cols = enum_setup(sys, td, tl, sh);
@@ -1385,6 +1406,7 @@ __global__ __launch_bounds__(kTileScanThreads) void k_tile_scan(int4* __restrict
                                                                 int ntiles) {
   __shared__ int wsum[kTileScanThreads / 64];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  heads += blockIdx.y * (long long)ntiles;   // frame of the group
   // sum over the block of one int per thread, in every thread
   auto block_sum = [&](int x) {
 #pragma unroll
@@ -1441,6 +1463,12 @@ __global__ __launch_bounds__(kThreads) void k_tile_lists(SysDev sys, const TypeD
                                                          int* __restrict__ err,
                                                          int* __restrict__ bcount, int nbk) {
   __shared__ EnumShared<MT> sh;
+  const int fr = blockIdx.y;   // frame of the group
+  boff += fr * sys.f_buckets();
+  s_ir += fr * sys.f_atoms();
+  pool += fr * (long long)cap;
+  heads += fr * (long long)sys.f_tiles;
+  bcount += fr * sys.f_buckets();
   // the bucket counts, read by k_tile_count and the bucket scan before this
   // kernel, start the slot's next frame at zero
   for (int i = blockIdx.x * kThreads + threadIdx.x; i < nbk; i += gridDim.x * kThreads)
@@ -1597,6 +1625,12 @@ __device__ __forceinline__ void deposit_lists(SysDev sys, const TypeDev* __restr
   } ty;
   const int tid = threadIdx.x;
   const int wave = tid >> 6, lane = tid & 63;
+  const int fr = blockIdx.y;   // frame of the group
+  pool += fr * (long long)sys.f_pool;
+  heads += fr * (long long)sys.f_tiles;
+  slices += fr * sys.f_slices;
+  bslices += fr * sys.f_bslices;
+  rho += fr * sys.f_points;
   for (int i = tid; i < sys.ntypes; i += kThreads) {
     const TypeDev& d = td[i];
     ty.pre[i][0] = 0;
@@ -1898,6 +1932,13 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4, 8))
   const int tid = threadIdx.x;
   const int wave = tid >> 6, lane = tid & 63;
   const int n16 = lane & 15, q4l = lane >> 4;
+  const int fr = blockIdx.y;   // frame of the group
+  boff += fr * sys.f_buckets();
+  s_ir += fr * sys.f_atoms();
+  slices += fr * sys.f_slices;
+  dslices += fr * sys.f_slices;
+  grho += fr * sys.f_points;
+  tpart += 3 * fr * sys.f_adjt;
   Tile tl;
   tile_coords(sys, tl);
   // this wave's share of the tile, zero outside the grid
@@ -2120,6 +2161,17 @@ __global__ __launch_bounds__(kThreads) void k_deposit_spill(SysDev sys,
   __shared__ ACC sez[kSpillChunk][T];
   const int tid = threadIdx.x;
   const int b = blockIdx.x;
+  const int fr = blockIdx.y;   // frame of the group
+  boff += fr * sys.f_buckets();
+  s_ir += fr * sys.f_atoms();
+  s_r += 3 * fr * sys.f_atoms();
+  corners += fr * kCornerInts;
+  if (stage) {
+    flag += fr * (sys.f_spill / (T * T * T));
+    stage += fr * sys.f_spill;
+  } else {
+    rho += fr * sys.f_points;
+  }
   const int ncorner = corners[0], nspill = corners[1 + 2 * kCornerCap];
   const bool listed = ncorner <= kCornerCap;
   // uniform over the block; a staged tile nothing spills into is not read
@@ -2281,6 +2333,11 @@ __global__ __launch_bounds__(kThreads) void k_parked(SysDev sys, const TypeDev* 
                                                      const double* __restrict__ s_r,
                                                      ACC* __restrict__ rho) {
   const TypeDev& ty = td[blockIdx.y];
+  const int fr = blockIdx.z;   // frame of the group
+  boff += fr * sys.f_buckets();
+  s_ir += fr * sys.f_atoms();
+  s_r += 3 * fr * sys.f_atoms();
+  rho += fr * sys.f_points;
   const int first = boff[ty.park], last = boff[ty.park + 1];
   for (int s = first + (int)blockIdx.x; s < last; s += (int)gridDim.x) {
     const ClipWin w = clip_window(sys, ty, s_ir[s]);
@@ -2305,11 +2362,11 @@ hipError_t launch_spill(Plan& p, ACC* out, ACC* stage, hipStream_t s) {
   const SysDev& sys = p.sys;
   if (p.spill_tiles == 0 || sys.natoms == 0) return hipSuccess;
   if (sys.mode == MODE_GEN)
-    hipLaunchKernelGGL((k_deposit_spill<ACC, true>), dim3((unsigned)p.spill_tiles), dim3(kThreads),
-                       0, s, sys, p.types, p.bucket_off, p.s_ir, p.s_r, p.corners, p.spill_flag,
+    hipLaunchKernelGGL((k_deposit_spill<ACC, true>), dim3((unsigned)p.spill_tiles, p.nfr),
+                       dim3(kThreads), 0, s, sys, p.types, p.bucket_off, p.s_ir, p.s_r, p.corners, p.spill_flag,
                        out, stage);
   else
-    hipLaunchKernelGGL((k_deposit_spill<ACC, false>), dim3((unsigned)p.spill_tiles),
+    hipLaunchKernelGGL((k_deposit_spill<ACC, false>), dim3((unsigned)p.spill_tiles, p.nfr),
                        dim3(kThreads), 0, s, sys, p.types, p.bucket_off, p.s_ir, p.s_r, p.corners,
                        p.spill_flag, out, stage);
   return hipGetLastError();
@@ -2320,7 +2377,7 @@ hipError_t launch_impl(Plan& p, ACC* out, const ACC* stage, hipStream_t s) {
   const SysDev& sys = p.sys;
   const long long ntiles = (long long)sys.ntiles[0] * sys.ntiles[1] * sys.ntiles[2];
   if (ntiles == 0) return hipSuccess;
-  const dim3 grid((unsigned)ntiles), block(kThreads);
+  const dim3 grid((unsigned)ntiles, p.nfr), block(kThreads);
   // with the plan's deposition events set (stage timing), the events are
   // recorded with the kernel's own dispatch (the kernel's begin and end)
 #define DEP_LAUNCH(K, ...)                                                              \
@@ -2393,7 +2450,7 @@ hipError_t launch_deposit(Plan& p, void* out, hipStream_t s) {
 hipError_t launch_parked(Plan& p, void* out, hipStream_t s) {
   const SysDev& sys = p.sys;
   if (sys.natoms == 0 || sys.ntypes == 0) return hipSuccess;
-  const dim3 grid(8, (unsigned)sys.ntypes), block(kThreads);
+  const dim3 grid(8, (unsigned)sys.ntypes, p.nfr), block(kThreads);
   if (p.fft64)
     hipLaunchKernelGGL(k_parked<double>, grid, block, 0, s, sys, p.types, p.bucket_off, p.s_ir,
                        p.s_r, static_cast<double*>(out));
@@ -2413,14 +2470,14 @@ hipError_t launch_tile_regions(Plan& p, hipStream_t s) {
   const SysDev& sys = p.sys;
   const long long ntiles = (long long)sys.ntiles[0] * sys.ntiles[1] * sys.ntiles[2];
   if (p.tl_cap == 0 || ntiles == 0 || sys.natoms == 0) return hipSuccess;
-  const dim3 grid((unsigned)ntiles), block(kThreads);
+  const dim3 grid((unsigned)ntiles, p.nfr), block(kThreads);
   if (sys.ntypes <= 16)
     hipLaunchKernelGGL(k_tile_count<16>, grid, block, 0, s, sys, p.types, p.bucket_count,
                        p.tl_head);
   else
     hipLaunchKernelGGL(k_tile_count<kMaxTypes>, grid, block, 0, s, sys, p.types, p.bucket_count,
                        p.tl_head);
-  hipLaunchKernelGGL(k_tile_scan, dim3((unsigned)((ntiles + kTileScanTiles - 1) / kTileScanTiles)),
+  hipLaunchKernelGGL(k_tile_scan, dim3((unsigned)((ntiles + kTileScanTiles - 1) / kTileScanTiles), p.nfr),
                      dim3(kTileScanThreads), 0, s, p.tl_head, (int)ntiles);
   return hipGetLastError();
 }
@@ -2429,7 +2486,7 @@ hipError_t launch_tile_lists(Plan& p, hipStream_t s) {
   const SysDev& sys = p.sys;
   const long long ntiles = (long long)sys.ntiles[0] * sys.ntiles[1] * sys.ntiles[2];
   if (p.tl_cap == 0 || ntiles == 0 || sys.natoms == 0) return hipSuccess;
-  const dim3 grid((unsigned)ntiles), block(kThreads);
+  const dim3 grid((unsigned)ntiles, p.nfr), block(kThreads);
   if (sys.ntypes <= 16)
     hipLaunchKernelGGL(k_tile_lists<16>, grid, block, 0, s, sys, p.types, p.bucket_off, p.s_ir,
                        p.tl_pool, (int)p.tl_cap, p.tl_head, p.err, p.bucket_count,
@@ -2445,7 +2502,7 @@ hipError_t launch_adjoint_tiles(Plan& p, const float* grho, hipStream_t s) {
   const SysDev& sys = p.sys;
   const long long ntiles = (long long)sys.ntiles[0] * sys.ntiles[1] * sys.ntiles[2];
   if (ntiles == 0) return hipSuccess;
-  const dim3 grid((unsigned)ntiles), block(kThreads);
+  const dim3 grid((unsigned)ntiles, p.nfr), block(kThreads);
   if (sys.ntypes <= 16)
     hipLaunchKernelGGL(k_adjoint_mfma<16>, grid, block, 0, s, sys, p.types, p.bucket_off, p.s_ir,
                        p.slices, p.dslices, grho, p.adj_tpart);

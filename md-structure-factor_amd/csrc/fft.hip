@@ -336,12 +336,17 @@ __global__ void k_twiddles(float2* __restrict__ tw, double2* __restrict__ tw64, 
 // --- pencil passes -----------------------------------------------------------------
 // Pencil p of a block at slow index s and first fast index f0 reads its element
 // e at in + s*in_s + (f0+p)*in_f + e*in_e and writes its element k to
-// out + s*out_s + (f0+p)*out_f + k*out_e.  Blocks run over (s, f-tile).
+// out + s*out_s + (f0+p)*out_f + k*out_e.  Blocks run over (s, f-tile), and over
+// the frames of the group as blockIdx.y, except in accumulating passes (which
+// have one slow index), whose blocks take the frames in turn.  in_F, out_F:
+// elements from one frame to the next.
 struct Geom {
-  long long in_s, in_f, in_e, out_s, out_f, out_e;
+  int in_s, in_f, in_e, out_s, out_f, out_e;   // at most a plane of 4096^2
+  long long in_F, out_F;
   int nf;            // fast indices per slow index
+  int ns;            // slow indices
   int tiles_f;       // ceil(nf / P)
-  long long blocks;  // slow count * tiles_f
+  long long blocks;  // ns * tiles_f
 };
 
 enum Epilogue { EPI_STORE = 0, EPI_ACC = 1 };
@@ -360,56 +365,63 @@ struct PassArgs {
   int P;
   int n;
   FftAxis ax;
-  // Nyquist plane (FP64, in place): blocks [g.blocks, g.blocks + nq_pencils)
-  // take one pencil each: element e at nyq + pencil*nq_p + e*nq_e
+  // Nyquist plane (FP64, in place): blocks from g.blocks on take one pencil
+  // each: element e of frame h's pencil at nyq + h*nq_F + pencil*nq_p + e*nq_e
   double2* nyq;
   double* nyq_acc;
   const double* nyq_w;
-  long long nq_p, nq_e;
-  int nq_pencils;
+  int nq_p, nq_e;
+  long long nq_F;
+  int nq_pencils;               // per frame
   int tpb;                      // tiles per block of the register-staged pass
-  // EPI_ACC, register-staged pass: a second spectrum (the next frame's, with
-  // its residuals and Nyquist plane) transformed by the same blocks, its
-  // |X|^2 added after the first one's, so that the FP64 sums are read and
-  // written once for two frames (null: one spectrum)
-  const typename V2<R>::T* in2;
-  const unsigned char* res_in2;
-  double2* nyq2;
+  // frames of the launch.  EPI_ACC: the same blocks transform every frame's
+  // spectrum (and residuals, Nyquist plane) in turn and add its |X|^2, so that
+  // the FP64 sums are read and written once for all of them; res_F: residual
+  // bytes from one frame to the next
+  int nfr;
+  long long res_F;
 };
 
-// One Nyquist-plane pencil per block, every stage in LDS (FP64).
+// One Nyquist-plane pencil per block, every stage in LDS (FP64): of the block's
+// frame, or (accumulating passes) of every frame in turn.
 template <bool INV, int EPI, typename A>
 __device__ void nyq_pencil(const A& a, int pencil, double* lds) {
   const int n = a.n, pitch = lds_pitch(n);
-  double* re = lds;
-  double* im = lds + pitch;
+  const int h0 = EPI == EPI_ACC ? 0 : blockIdx.y, h1 = EPI == EPI_ACC ? a.nfr : h0 + 1;
   const long long base = (long long)pencil * a.nq_p;
-  __syncthreads();  // the LDS may still be read for the previous pencil or tile
-  for (int e = threadIdx.x; e < n; e += kFftThreads) {
-    const long long g = base + e * a.nq_e;
-    const double2 v = a.nyq[g];
-    const double sc = a.nyq_w ? a.nyq_w[g] : 1.0;
-    re[e] = v.x * sc;
-    im[e] = v.y * sc;
-  }
-  __syncthreads();
-  const int cur = run_stages<INV>(lds, n, 1, pitch, a.ax);
-  re = lds + 2 * cur * pitch;
-  im = re + pitch;
-  for (int e = threadIdx.x; e < n; e += kFftThreads) {
-    const long long g = base + e * a.nq_e;
-    if (EPI == EPI_STORE) a.nyq[g] = make_double2(re[e], im[e]);
-    else a.nyq_acc[g] += re[e] * re[e] + im[e] * im[e];
+  for (int h = h0; h < h1; ++h) {
+    double2* nyq = a.nyq + h * a.nq_F;
+    double* re = lds;
+    double* im = lds + pitch;
+    __syncthreads();  // the LDS may still be read for the previous pencil or tile
+    for (int e = threadIdx.x; e < n; e += kFftThreads) {
+      const long long g = base + (long long)e * a.nq_e;
+      const double2 v = nyq[g];
+      const double sc = a.nyq_w ? a.nyq_w[g] : 1.0;
+      re[e] = v.x * sc;
+      im[e] = v.y * sc;
+    }
+    __syncthreads();
+    const int cur = run_stages<INV>(lds, n, 1, pitch, a.ax);
+    re = lds + 2 * cur * pitch;
+    im = re + pitch;
+    for (int e = threadIdx.x; e < n; e += kFftThreads) {
+      const long long g = base + (long long)e * a.nq_e;
+      if (EPI == EPI_STORE) nyq[g] = make_double2(re[e], im[e]);
+      else a.nyq_acc[g] += re[e] * re[e] + im[e] * im[e];
+    }
   }
 }
 
 // Global element access of a pass: load with the optional weight and
-// residual, store / accumulate with the optional residual.
+// residual, store / accumulate with the optional residual.  in, res_in, out and
+// res_out are the frame's (the weights are every frame's).
 template <typename R, int RES>
-__device__ __forceinline__ Cx pass_load(const PassArgs<R>& a, long long gi) {
-  Cx x = load_cx<R>(a.in, gi);
+__device__ __forceinline__ Cx pass_load(const PassArgs<R>& a, const typename V2<R>::T* in,
+                                        const unsigned char* res_in, long long gi) {
+  Cx x = load_cx<R>(in, gi);
   if constexpr ((RES & RES_IN) != 0) {
-    const unsigned b = a.res_in[gi];
+    const unsigned b = res_in[gi];
     x.x += res_value(b & 15u, (float)x.x);
     x.y += res_value(b >> 4, (float)x.y);
   }
@@ -417,13 +429,14 @@ __device__ __forceinline__ Cx pass_load(const PassArgs<R>& a, long long gi) {
   return x;
 }
 template <typename R, int EPI, int RES>
-__device__ __forceinline__ void pass_store(const PassArgs<R>& a, long long go, Cx v) {
+__device__ __forceinline__ void pass_store(const PassArgs<R>& a, typename V2<R>::T* out,
+                                           unsigned char* res_out, long long go, Cx v) {
   if constexpr (EPI == EPI_ACC) {
     a.acc[go] += v.x * v.x + v.y * v.y;
   } else {
-    store_cx<R>(a.out, go, v);
+    store_cx<R>(out, go, v);
     if constexpr ((RES & RES_OUT) != 0)
-      a.res_out[go] = (unsigned char)(res_nibble(v.x, (float)v.x) | (res_nibble(v.y, (float)v.y) << 4));
+      res_out[go] = (unsigned char)(res_nibble(v.x, (float)v.x) | (res_nibble(v.y, (float)v.y) << 4));
   }
 }
 
@@ -573,18 +586,24 @@ __global__ __launch_bounds__(kFftThreads) void k_pass_stream(PassArgs<R> a) {
   };
   T2 raw[16];
   uint4 rq;  // RES_IN: bytes 16 tid .. 16 tid + 15 of the tile's residuals (P whole rows)
-  // EPI_ACC with a second spectrum: each tile is transformed twice (sub-tile
-  // h = 0: a.in, h = 1: a.in2), into the same accumulator values
-  const int nsub = (EPI == EPI_ACC && a.in2) ? 2 : 1;
-  // sub-tile vt = nsub tile + h
-  auto load = [&](long long vt) __attribute__((always_inline)) {
-    const long long tile = nsub == 2 ? vt >> 1 : vt;
-    const bool second = nsub == 2 && (vt & 1);
+  // EPI_ACC: each tile is transformed once per frame (sub), into the same
+  // accumulator values; else the block's frame
+  const int nsub = EPI == EPI_ACC ? a.nfr : 1;
+  const T2* in = a.in;
+  T2* out = a.out;
+  unsigned char* res_out = a.res_out;
+  if constexpr (EPI != EPI_ACC) {
+    in += blockIdx.y * g.in_F;
+    out += blockIdx.y * g.out_F;
+    if constexpr ((RES & RES_OUT) != 0) res_out += blockIdx.y * a.res_F;
+  }
+  auto load = [&](long long tile, int sub) __attribute__((always_inline)) {
     const unsigned s = (unsigned)(tile / tiles_f);
     const int f0 = (int)((unsigned)tile - s * tiles_f) * P;
     const int pc = min(P, g.nf - f0);
     const long long ib = (long long)s * g.in_s + (long long)f0 * g.in_f;
-    const T2* src = (second ? a.in2 : a.in) + ib;
+    const T2* src = in + ib;
+    if constexpr (EPI == EPI_ACC) src += sub * g.in_F;
 #pragma unroll
     for (int t = 0; t < 16 / R1; ++t) {
       unsigned o;
@@ -595,148 +614,151 @@ __global__ __launch_bounds__(kFftThreads) void k_pass_stream(PassArgs<R> a) {
     if constexpr ((RES & RES_IN) != 0) {
       // past a partial tile's rows: the tile's first bytes (never used)
       const unsigned q = 16u * (unsigned)tid < (unsigned)(pc * n) ? (unsigned)tid : 0u;
-      rq = at(reinterpret_cast<const uint4*>((second ? a.res_in2 : a.res_in) + ib), q);
+      const int hr = EPI == EPI_ACC ? sub : (int)blockIdx.y;
+      rq = at(reinterpret_cast<const uint4*>(a.res_in + hr * a.res_F + ib), q);
     }
   };
   const long long nblk = (ntiles + a.tpb - 1) / a.tpb;
   if ((long long)blockIdx.x >= nblk) {
-    // the Nyquist-plane pencils: one per block after the tile blocks (the
-    // second spectrum's after the first's, into the same sums)
+    // the Nyquist-plane pencils: one per block after the tile blocks
     if (a.nyq) nyq_pencil<INV, EPI>(a, (int)((long long)blockIdx.x - nblk), plane);
-    if constexpr (EPI == EPI_ACC) {
-      if (a.nyq2) {
-        PassArgs<R> b = a;
-        b.nyq = a.nyq2;
-        nyq_pencil<INV, EPI>(b, (int)((long long)blockIdx.x - nblk), plane);
-      }
-    }
     return;
   }
-  const long long vend = min(ntiles, (long long)(blockIdx.x + 1) * a.tpb) * nsub;
-  long long vt = (long long)blockIdx.x * a.tpb * nsub;
-  if (PF) load(vt);
+  const long long tend = min(ntiles, (long long)(blockIdx.x + 1) * a.tpb);
+  long long tile = (long long)blockIdx.x * a.tpb;
+  if (PF) load(tile, 0);
   for (int i = threadIdx.x; i < n; i += kFftThreads) twl[i] = a.ax.tw64[i];
   double accv[EPI == EPI_ACC ? 16 : 1];  // this tile's accumulator values (EPI_ACC)
-  for (; vt < vend; ++vt) {
-    tid = opaque(tid);
-    if (!PF) load(vt);
-    const long long tile = nsub == 2 ? vt >> 1 : vt;
-    const bool first = nsub == 2 && !(vt & 1);  // a first spectrum's sub-tile (accumulator kept)
+  for (; tile < tend; ++tile) {
     const unsigned s = (unsigned)(tile / tiles_f);
     const int f0 = (int)((unsigned)tile - s * tiles_f) * P;
     const int pc = min(P, g.nf - f0);
     const long long ib = (long long)s * g.in_s + (long long)f0 * g.in_f;
     const long long ob = (long long)s * g.out_s + (long long)f0 * g.out_f;
-    Cx v[16];
-#pragma unroll
-    for (int i = 0; i < 16; ++i) v[i] = mk((double)raw[i].x, (double)raw[i].y);
-    if constexpr ((RES & RES_IN) != 0) {
-      // the previous tile's last reads of resl preceded its exchange barriers
-      reinterpret_cast<uint4*>(resl)[tid] = rq;
-      lds_barrier();
-#pragma unroll
-      for (int t = 0; t < 16 / R1; ++t) {
-        const int b = tid + t * kFftThreads;
-        const int q = (b / nq1) * n + b % nq1;  // row p, element j (in_f = n, in_e = 1)
-#pragma unroll
-        for (int r = 0; r < R1; ++r) {
-          const unsigned rb = resl[q + r * nq1];
-          const int i = t * R1 + r;
-          v[i].x += res_value(rb & 15u, raw[i].x);
-          v[i].y += res_value(rb >> 4, raw[i].y);
-        }
-      }
-    }
-    if constexpr (WGT) {
-#pragma unroll
-      for (int t = 0; t < 16 / R1; ++t) {
-        unsigned o;
-        in_pos(t, pc, &o);
-#pragma unroll
-        for (int r = 0; r < R1; ++r) v[t * R1 + r] = cscale(at(a.w + ib, o + (unsigned)(r * nq1) * in_e), v[t * R1 + r]);
-      }
-    }
-    if (PF && vt + 1 < vend) load(vt + 1);
     // the accumulator values this tile adds to, loaded now so that their
     // latency passes during the transform (pencils past a partial tile read
-    // the last one and are not stored); with two spectra, loaded with the
-    // first and kept in registers through the second
+    // the last one and are not stored), kept in registers through the frames
     if constexpr (EPI == EPI_ACC) {
-      if (!(nsub == 2 && (vt & 1))) {
 #pragma unroll
-        for (int t = 0; t < 16 / RL; ++t) {
-          const int b = tid + t * kFftThreads;
-          int p = OUT_E ? b / nsL : b % P;
-          const int k = OUT_E ? b % nsL : b / P;
-          p = p < pc ? p : pc - 1;
-          const unsigned o = (unsigned)p * out_f + (unsigned)k * out_e;
-#pragma unroll
-          for (int r = 0; r < RL; ++r) accv[t * RL + r] = at(a.acc + ob, o + (unsigned)(r * nsL) * out_e);
-        }
-      }
-    }
-    // stage 1 (span 1): DFT_R1; output position j R1 + r
-#pragma unroll
-    for (int t = 0; t < 16 / R1; ++t) dft<R1, INV>(v + t * R1);
-    auto out1 = [&](int i) __attribute__((always_inline)) {
-      const int b = tid + (i / R1) * kFftThreads, r = i % R1;
-      const int p = IN_E ? b / nq1 : b % P, j = IN_E ? b % nq1 : b / P;
-      return p * pitch + reg_pos(j * R1 + r);
-    };
-    // last stage inputs: element k + r nsL of pencil p
-    auto inL = [&](int i) __attribute__((always_inline)) {
-      const int b = tid + (i / RL) * kFftThreads, r = i % RL;
-      const int p = OUT_E ? b / nsL : b % P, k = OUT_E ? b % nsL : b / P;
-      return p * pitch + reg_pos(k + r * nsL);
-    };
-    if constexpr (R3 > 1) {
-      // middle stage (span R1, radix R2): LDS -> DFT_R2 -> LDS
-      constexpr int nq2 = n / R2, ns2 = R1;
-      auto in2 = [&](int i) __attribute__((always_inline)) {
-        const int b = tid + (i / R2) * kFftThreads, r = i % R2;
-        return (b % P) * pitch + reg_pos(b / P + r * nq2);
-      };
-      auto out2 = [&](int i) __attribute__((always_inline)) {
-        const int b = tid + (i / R2) * kFftThreads, r = i % R2;
-        const int j = b / P, k = j % ns2;
-        return (b % P) * pitch + reg_pos((j / ns2) * ns2 * R2 + k + r * ns2);
-      };
-      lds_exchange<16>(plane, v, out1, in2);
-#pragma unroll
-      for (int t = 0; t < 16 / R2; ++t) {
+      for (int t = 0; t < 16 / RL; ++t) {
         const int b = tid + t * kFftThreads;
-        twiddle_in<R2, INV>(v + t * R2, (b / P) % ns2, n / (ns2 * R2), tw);
-        dft<R2, INV>(v + t * R2);
-      }
-      lds_exchange<16>(plane, v, out2, inL);
-    } else {
-      lds_exchange<16>(plane, v, out1, inL);
-    }
-#pragma unroll
-    for (int t = 0; t < 16 / RL; ++t) {
-      const int b = tid + t * kFftThreads;
-      const int p = OUT_E ? b / nsL : b % P, k = OUT_E ? b % nsL : b / P;
-      Cx* x = v + t * RL;
-      twiddle_in<RL, INV>(x, k, 1, tw);
-      dft<RL, INV>(x);
-      if (p < pc) {
+        int p = OUT_E ? b / nsL : b % P;
+        const int k = OUT_E ? b % nsL : b / P;
+        p = p < pc ? p : pc - 1;
         const unsigned o = (unsigned)p * out_f + (unsigned)k * out_e;
 #pragma unroll
-        for (int r = 0; r < RL; ++r) {
-          const unsigned oe = o + (unsigned)(r * nsL) * out_e;
-          if constexpr (EPI == EPI_ACC) {
-            const double sum = accv[t * RL + r] + (x[r].x * x[r].x + x[r].y * x[r].y);
-            if (first) accv[t * RL + r] = sum;
-            else at(a.acc + ob, oe) = sum;
-          } else {
+        for (int r = 0; r < RL; ++r) accv[t * RL + r] = at(a.acc + ob, o + (unsigned)(r * nsL) * out_e);
+      }
+    }
+    for (int sub = 0; sub < nsub; ++sub) {
+      tid = opaque(tid);
+      if (!PF) load(tile, sub);
+      Cx v[16];
+#pragma unroll
+      for (int i = 0; i < 16; ++i) v[i] = mk((double)raw[i].x, (double)raw[i].y);
+      if constexpr ((RES & RES_IN) != 0) {
+        // the previous tile's last reads of resl preceded its exchange barriers
+        reinterpret_cast<uint4*>(resl)[tid] = rq;
+        lds_barrier();
+#pragma unroll
+        for (int t = 0; t < 16 / R1; ++t) {
+          const int b = tid + t * kFftThreads;
+          const int q = (b / nq1) * n + b % nq1;  // row p, element j (in_f = n, in_e = 1)
+#pragma unroll
+          for (int r = 0; r < R1; ++r) {
+            const unsigned rb = resl[q + r * nq1];
+            const int i = t * R1 + r;
+            v[i].x += res_value(rb & 15u, raw[i].x);
+            v[i].y += res_value(rb >> 4, raw[i].y);
+          }
+        }
+      }
+      if constexpr (WGT) {
+#pragma unroll
+        for (int t = 0; t < 16 / R1; ++t) {
+          unsigned o;
+          in_pos(t, pc, &o);
+#pragma unroll
+          for (int r = 0; r < R1; ++r) v[t * R1 + r] = cscale(at(a.w + ib, o + (unsigned)(r * nq1) * in_e), v[t * R1 + r]);
+        }
+      }
+      if (PF) {
+        if (sub + 1 < nsub) load(tile, sub + 1);
+        else if (tile + 1 < tend) load(tile + 1, 0);
+      }
+      // stage 1 (span 1): DFT_R1; output position j R1 + r
+#pragma unroll
+      for (int t = 0; t < 16 / R1; ++t) dft<R1, INV>(v + t * R1);
+      auto out1 = [&](int i) __attribute__((always_inline)) {
+        const int b = tid + (i / R1) * kFftThreads, r = i % R1;
+        const int p = IN_E ? b / nq1 : b % P, j = IN_E ? b % nq1 : b / P;
+        return p * pitch + reg_pos(j * R1 + r);
+      };
+      // last stage inputs: element k + r nsL of pencil p
+      auto inL = [&](int i) __attribute__((always_inline)) {
+        const int b = tid + (i / RL) * kFftThreads, r = i % RL;
+        const int p = OUT_E ? b / nsL : b % P, k = OUT_E ? b % nsL : b / P;
+        return p * pitch + reg_pos(k + r * nsL);
+      };
+      if constexpr (R3 > 1) {
+        // middle stage (span R1, radix R2): LDS -> DFT_R2 -> LDS
+        constexpr int nq2 = n / R2, ns2 = R1;
+        auto in2 = [&](int i) __attribute__((always_inline)) {
+          const int b = tid + (i / R2) * kFftThreads, r = i % R2;
+          return (b % P) * pitch + reg_pos(b / P + r * nq2);
+        };
+        auto out2 = [&](int i) __attribute__((always_inline)) {
+          const int b = tid + (i / R2) * kFftThreads, r = i % R2;
+          const int j = b / P, k = j % ns2;
+          return (b % P) * pitch + reg_pos((j / ns2) * ns2 * R2 + k + r * ns2);
+        };
+        lds_exchange<16>(plane, v, out1, in2);
+#pragma unroll
+        for (int t = 0; t < 16 / R2; ++t) {
+          const int b = tid + t * kFftThreads;
+          twiddle_in<R2, INV>(v + t * R2, (b / P) % ns2, n / (ns2 * R2), tw);
+          dft<R2, INV>(v + t * R2);
+        }
+        lds_exchange<16>(plane, v, out2, inL);
+      } else {
+        lds_exchange<16>(plane, v, out1, inL);
+      }
+#pragma unroll
+      for (int t = 0; t < 16 / RL; ++t) {
+        const int b = tid + t * kFftThreads;
+        const int p = OUT_E ? b / nsL : b % P, k = OUT_E ? b % nsL : b / P;
+        Cx* x = v + t * RL;
+        twiddle_in<RL, INV>(x, k, 1, tw);
+        dft<RL, INV>(x);
+        if constexpr (EPI == EPI_ACC) {
+#pragma unroll
+          for (int r = 0; r < RL; ++r)
+            accv[t * RL + r] = accv[t * RL + r] + (x[r].x * x[r].x + x[r].y * x[r].y);
+        } else if (p < pc) {
+          const unsigned o = (unsigned)p * out_f + (unsigned)k * out_e;
+#pragma unroll
+          for (int r = 0; r < RL; ++r) {
+            const unsigned oe = o + (unsigned)(r * nsL) * out_e;
             T2 st;
             st.x = (R)x[r].x;
             st.y = (R)x[r].y;
-            at(a.out + ob, oe) = st;
+            at(out + ob, oe) = st;
             if constexpr ((RES & RES_OUT) != 0)  // element k + r nsL of pencil p
               resl[(k + r * nsL) * P + p] =
                   (unsigned char)(res_nibble(x[r].x, st.x) | (res_nibble(x[r].y, st.y) << 4));
           }
+        }
+      }
+    }
+    if constexpr (EPI == EPI_ACC) {
+#pragma unroll
+      for (int t = 0; t < 16 / RL; ++t) {
+        const int b = tid + t * kFftThreads;
+        const int p = OUT_E ? b / nsL : b % P, k = OUT_E ? b % nsL : b / P;
+        if (p < pc) {
+          const unsigned o = (unsigned)p * out_f + (unsigned)k * out_e;
+#pragma unroll
+          for (int r = 0; r < RL; ++r) at(a.acc + ob, o + (unsigned)(r * nsL) * out_e) = accv[t * RL + r];
         }
       }
     }
@@ -747,7 +769,7 @@ __global__ __launch_bounds__(kFftThreads) void k_pass_stream(PassArgs<R> a) {
       lds_barrier();
       const unsigned q = 16u * (unsigned)tid;
       const int row = (int)(q / P), col = (int)(q % P);
-      unsigned char* dst = a.res_out + ob;
+      unsigned char* dst = res_out + ob;
       if (P >= 16 && (out_e & 15u) == 0 && col + 16 <= pc) {
         at(reinterpret_cast<uint4*>(dst + (size_t)row * out_e + col), 0u) =
             *reinterpret_cast<const uint4*>(resl + q);
@@ -779,23 +801,29 @@ __global__ __launch_bounds__(kFftThreads) void k_pass_lds(PassArgs<R> a) {
   const int pc = min(P, g.nf - f0);
   const long long ib = s * g.in_s + (long long)f0 * g.in_f;
   const long long ob = s * g.out_s + (long long)f0 * g.out_f;
-  double* re = lds;
-  double* im = lds + P * pitch;
   const bool in_e = g.in_e == 1, out_e = g.out_e == 1;
-  for (int idx = threadIdx.x; idx < pc * n; idx += kFftThreads) {
-    const int p = in_e ? idx / n : idx % pc, e = in_e ? idx % n : idx / pc;
-    const Cx x = pass_load<R, RES>(a, ib + (long long)p * g.in_f + (long long)e * g.in_e);
-    re[p * pitch + e] = x.x;
-    im[p * pitch + e] = x.y;
-  }
-  __syncthreads();
-  const int cur = run_stages<INV>(lds, n, P, pitch, a.ax);
-  re = lds + 2 * cur * P * pitch;
-  im = re + P * pitch;
-  for (int idx = threadIdx.x; idx < pc * n; idx += kFftThreads) {
-    const int p = out_e ? idx / n : idx % pc, k = out_e ? idx % n : idx / pc;
-    pass_store<R, EPI, RES>(a, ob + (long long)p * g.out_f + (long long)k * g.out_e,
-                            mk(re[p * pitch + k], im[p * pitch + k]));
+  const int h0 = EPI == EPI_ACC ? 0 : blockIdx.y, h1 = EPI == EPI_ACC ? a.nfr : h0 + 1;
+  for (int h = h0; h < h1; ++h) {
+    double* re = lds;
+    double* im = lds + P * pitch;
+    if (h > h0) __syncthreads();   // the previous frame's results are read
+    for (int idx = threadIdx.x; idx < pc * n; idx += kFftThreads) {
+      const int p = in_e ? idx / n : idx % pc, e = in_e ? idx % n : idx / pc;
+      const Cx x = pass_load<R, RES>(a, a.in + h * g.in_F, a.res_in + h * a.res_F,
+                                     ib + (long long)p * g.in_f + (long long)e * g.in_e);
+      re[p * pitch + e] = x.x;
+      im[p * pitch + e] = x.y;
+    }
+    __syncthreads();
+    const int cur = run_stages<INV>(lds, n, P, pitch, a.ax);
+    re = lds + 2 * cur * P * pitch;
+    im = re + P * pitch;
+    for (int idx = threadIdx.x; idx < pc * n; idx += kFftThreads) {
+      const int p = out_e ? idx / n : idx % pc, k = out_e ? idx % n : idx / pc;
+      pass_store<R, EPI, RES>(a, a.out + h * g.out_F, a.res_out + h * a.res_F,
+                              ob + (long long)p * g.out_f + (long long)k * g.out_e,
+                              mk(re[p * pitch + k], im[p * pitch + k]));
+    }
   }
 }
 
@@ -1183,11 +1211,12 @@ template <typename R, int R1, int R2, int R3, bool INV, bool IN_E, bool OUT_E, i
 void launch_stream(size_t lds, hipStream_t s, PassArgs<R> a) {
   const void* k =
       reinterpret_cast<const void*>(&k_pass_stream<R, R1, R2, R3, INV, IN_E, OUT_E, EPI, RES, WGT>);
-  a.tpb = stream_tpb(k, lds, a.g.blocks);
+  const unsigned ny = EPI == EPI_ACC ? 1 : a.nfr;   // frames as grid y
+  a.tpb = stream_tpb(k, lds, a.g.blocks * ny);
   const long long grid = (a.g.blocks + a.tpb - 1) / a.tpb + (a.nyq ? a.nq_pencils : 0);
   if (grid == 0) return;
-  pass_launch(k_pass_stream<R, R1, R2, R3, INV, IN_E, OUT_E, EPI, RES, WGT>, dim3((unsigned)grid),
-              lds, s, a);
+  pass_launch(k_pass_stream<R, R1, R2, R3, INV, IN_E, OUT_E, EPI, RES, WGT>,
+              dim3((unsigned)grid, ny), lds, s, a);
 }
 
 template <typename R, bool INV, bool IN_E, bool OUT_E, int EPI, int RES, bool WGT>
@@ -1235,10 +1264,10 @@ hipError_t run_pass(PassArgs<R> a, PassKind kind, hipStream_t s, int choice) {
   if (nyq_lds > lds) lds = nyq_lds;
   if (lds > max_lds_per_block()) return hipErrorInvalidValue;
   a.g.tiles_f = (a.g.nf + a.P - 1) / a.P;
-  a.g.blocks *= a.g.tiles_f;   // caller set the slow count
+  a.g.blocks = (long long)a.g.ns * a.g.tiles_f;
   const long long total = a.g.blocks + (a.nyq ? a.nq_pencils : 0);
   if (total == 0) return hipSuccess;
-  const dim3 g((unsigned)total);
+  const dim3 g((unsigned)total, kind == PK_X_ACC ? 1 : a.nfr);   // frames as grid y
   const bool f32 = sizeof(R) == 4;
   switch (kind) {
     case PK_Y:
@@ -1314,7 +1343,8 @@ void launch_z_stream(long long ntiles, hipStream_t s, ZArgs<R> a) {
 
 template <typename R>
 hipError_t pass_z(Plan& p, const void* density, hipStream_t s) {
-  const int nx = p.sys.n[0], ny = p.sys.n[1], m = p.sys.n[2] / 2;
+  // the group's frames lie one after the other: nx rows of planes each
+  const int nx = p.sys.n[0] * p.nfr, ny = p.sys.n[1], m = p.sys.n[2] / 2;
   ZArgs<R> a;
   a.in = static_cast<const R*>(density);
   a.out = cx<R>(p.spec);
@@ -1352,6 +1382,11 @@ PassArgs<R> base_args(Plan& p, int n, const FftAxis& ax) {
   PassArgs<R> a{};
   a.n = n;
   a.ax = ax;
+  a.nfr = p.nfr;
+  // the group's frames one after the other: half spectrum (also in the density
+  // buffer), residuals, Nyquist plane
+  a.g.in_F = a.g.out_F = a.res_F = (long long)p.sys.n[0] * p.sys.n[1] * (p.sys.n[2] / 2);
+  a.nq_F = (long long)p.sys.n[0] * p.sys.n[1];
   return a;
 }
 
@@ -1370,7 +1405,7 @@ hipError_t pass_y(Plan& p, hipStream_t s) {
   a.g.out_f = 1;
   a.g.out_e = nx;
   a.g.nf = nx;
-  a.g.blocks = m;
+  a.g.ns = m;
   a.nyq = static_cast<double2*>(p.spec_nyq);
   a.nq_p = ny;
   a.nq_e = 1;
@@ -1395,7 +1430,7 @@ PassArgs<R> x_args(Plan& p, void* rho, void* res, void* nyq) {
   a.g.out_f = nx;
   a.g.out_e = 1;
   a.g.nf = m * ny;
-  a.g.blocks = 1;
+  a.g.ns = 1;
   a.nyq = static_cast<double2*>(nyq);
   a.nyq_acc = p.sf_nyq;
   a.nq_p = 1;
@@ -1416,9 +1451,10 @@ hipError_t pass_x(Plan& p, bool accumulate, hipStream_t s) {
 template <typename R>
 hipError_t pass_x_pair(Plan& p, int sa, int sb, hipStream_t s) {
   PassArgs<R> a = x_args<R>(p, p.rho_buf[sa], p.res_buf[sa], p.nyq_buf[sa]);
-  a.in2 = cx<R>(p.rho_buf[sb]);
-  a.res_in2 = static_cast<const unsigned char*>(p.res_buf[sb]);
-  a.nyq2 = static_cast<double2*>(p.nyq_buf[sb]);
+  a.nfr = 2;   // "frames" a slot's buffers apart
+  a.g.in_F = cx<R>(p.rho_buf[sb]) - a.in;
+  a.res_F = static_cast<const unsigned char*>(p.res_buf[sb]) - a.res_in;
+  a.nq_F = static_cast<double2*>(p.nyq_buf[sb]) - a.nyq;
   return run_pass<R>(a, PK_X_ACC, s, p.tune_x);
 }
 
@@ -1451,7 +1487,7 @@ hipError_t inverse_impl(Plan& p, const double* w_main, const double* w_nyq, void
     a.g.out_f = nx;
     a.g.out_e = 1;
     a.g.nf = m * ny;
-    a.g.blocks = 1;
+    a.g.ns = 1;
     a.nyq = static_cast<double2*>(p.spec_nyq);
     a.nyq_w = w_nyq;
     a.nq_p = 1;
@@ -1471,7 +1507,7 @@ hipError_t inverse_impl(Plan& p, const double* w_main, const double* w_nyq, void
     a.g.out_f = (long long)m * ny;
     a.g.out_e = 1;
     a.g.nf = nx;
-    a.g.blocks = m;
+    a.g.ns = m;
     a.nyq = static_cast<double2*>(p.spec_nyq);
     a.nq_p = ny;
     a.nq_e = 1;
@@ -1483,7 +1519,7 @@ hipError_t inverse_impl(Plan& p, const double* w_main, const double* w_nyq, void
   c.spec = cx<R>(p.spec);
   c.nyq = static_cast<const double2*>(p.spec_nyq);
   c.out = static_cast<R*>(out);
-  c.nx = nx;
+  c.nx = nx * p.nfr;   // the group's frames one after the other
   c.ny = ny;
   c.m = m;
   c.ax = p.ax_zc;
@@ -1491,7 +1527,7 @@ hipError_t inverse_impl(Plan& p, const double* w_main, const double* w_nyq, void
   if (z_reg_rows(m) > 0) {
     c.P = z_reg_rows(m);
     c.tiles_y = (ny + c.P - 1) / c.P;
-    const dim3 g((unsigned)((long long)nx * c.tiles_y)), b(kFftThreads);
+    const dim3 g((unsigned)((long long)c.nx * c.tiles_y)), b(kFftThreads);
     switch (m) {
       case 32: hipLaunchKernelGGL((k_c2r_z_reg<R, 8, 4>), g, b, 0, s, c); break;
       case 64: hipLaunchKernelGGL((k_c2r_z_reg<R, 8, 8>), g, b, 0, s, c); break;
@@ -1503,7 +1539,7 @@ hipError_t inverse_impl(Plan& p, const double* w_main, const double* w_nyq, void
   c.P = lds_pencils(m);
   while (c.P > 1 && lds_bytes(m, c.P) > max_lds_per_block()) c.P /= 2;
   c.tiles_y = (ny + c.P - 1) / c.P;
-  hipLaunchKernelGGL((k_c2r_z<R>), dim3((unsigned)((long long)nx * c.tiles_y)), dim3(kFftThreads),
+  hipLaunchKernelGGL((k_c2r_z<R>), dim3((unsigned)((long long)c.nx * c.tiles_y)), dim3(kFftThreads),
                      lds_bytes(m, c.P), s, c);
   return hipGetLastError();
 }
@@ -1688,7 +1724,7 @@ bool fft_pass_events_used() { return t_pass_ev_used; }
 
 bool fft_x_pairs(const Plan& p) {
   int r1, r2, r3;
-  return (p.tune_x == 0 || p.tune_x == kTuneReg) && reg_split(p.sys.n[0], &r1, &r2, &r3);
+  return p.group == 1 && (p.tune_x == 0 || p.tune_x == kTuneReg) && reg_split(p.sys.n[0], &r1, &r2, &r3);
 }
 
 hipError_t fft_x_pair(Plan& p, int slot_a, int slot_b, hipStream_t s) {

@@ -18,6 +18,7 @@ constexpr int kMaxStages = 16;  // FFT stages per axis
 constexpr int kTuneReg = 100;   // FFT pencil choice: register-staged kernel
 constexpr int kMaxSpillBufTiles = 4096;  // spill tiles staged per frame slot (else added in place)
 constexpr int kCornerCap = 512;     // corner atoms listed per frame for the spill pass
+constexpr int kCornerInts = 2 + 2 * kCornerCap;  // the list's ints per frame (FrameState::corners)
 constexpr int kListNoSlice = 255;  // tile-list entry: no slice on that axis (a byte per axis)
 constexpr long long kSplitPrepTiles = 2048;  // tiles from which the frame loop splits its prepare stage
 // stage-timing events per frame: prepare start / end (caller's stream), the
@@ -105,6 +106,14 @@ struct SysDev {
   // corner-fold spill tiles per axis: [0, sp_k0) and [sp_fh, ntiles), sp_cnt
   // of them (all tiles when the two ranges meet); none when nb = 0
   int sp_k0[3], sp_fh[3], sp_cnt[3];
+  // elements from one frame of a group to the next (a slot's arrays hold its
+  // frames one after the other; the frame of a block is blockIdx.y): slices,
+  // cross rows, tables, spill tiles (all cells), grid points, tile-list
+  // entries, scan totals, adjoint result slots and work items
+  long long f_slices, f_bslices, f_tables, f_spill, f_points, f_adjt, f_adji;
+  int f_pool, f_aux, f_tiles;
+  __host__ __device__ long long f_atoms() const { return natoms; }
+  __host__ __device__ long long f_buckets() const { return nbuckets + 1; }
 };
 
 // One FFT axis: length, radix sequence and twiddles W_n^k (k < n), FP32
@@ -152,16 +161,30 @@ struct FrameState {
   int4* tl_head = nullptr;
 };
 
-// Frame slots of a plan (atom state + density / spectrum buffers): frame t
-// uses slot t mod kSlots, so that a frame can be prepared, the previous one
+// Frame slots of a plan (atom state + density / spectrum buffers): frame group
+// k uses slot k mod kSlots, so that a group can be prepared, the previous one
 // deposited and the ones before it transformed without waiting for a buffer.
 constexpr int kSlots = 3;
+
+// Frames per group.  A small grid's frame leaves most of the chip idle (64
+// tiles of a 64^3 grid for 256 CUs) and its dozen and a half launches each take
+// their few microseconds of latency, so the frame loops hand every kernel the
+// frames of a group at once, as blockIdx.y: as many as make kGroupTiles tiles,
+// at most kMaxGroup, within kGroupBytes of state for the slots together.  Grids
+// of kGroupTiles tiles and more fill the chip with one frame.  Before and after:
+// ten frames of 2,700 atoms at 64^3 1,091 -> 292 us, sixteen forward and backward
+// frames at 128^3 4,865 -> 3,242 us, eight systems of 64^3 to 192^3 in one graph
+// 11,778 -> 9,012 us; one frame per group at 256^3, 4,930 and 4,915 us.
+constexpr int kGroupTiles = 2048;
+constexpr int kMaxGroup = 16;
+constexpr size_t kGroupBytes = (size_t)2 << 30;
 
 struct Plan {
   SysDev sys{};
   TypeDev types_host[kMaxTypes]{};
   TypeDev* types = nullptr;
   int device = 0;
+  void* arena = nullptr;  // the allocation that every buffer is cut from (but the adjoint's)
   long long table_floats = 0;
   // per-atom scratch (unsorted)
   int4* ir4 = nullptr;
@@ -208,6 +231,8 @@ struct Plan {
   // Frame slot b: its atom state and density / spectrum buffer become the
   // ones the launches below use (kernel arguments are taken at launch).
   int cur_slot = 0;
+  int group = 1;                 // frames a slot holds
+  int nfr = 1;                   // frames the next launches cover (the frame loops set it)
   void use_slot(int b) {
     b %= kSlots;
     cur_slot = b;
@@ -256,12 +281,13 @@ struct Plan {
   hipEvent_t ev_lfork = nullptr, ev_lgath = nullptr, ev_ljoin = nullptr;
   // optional stage timing of mdsf_accumulate_frames: 10 timing events per
   // frame (prepare, deposit, z, y, x: start / end, each on its stream)
-  int timing = 0;  // 0 off, 1 every stage, 2 the deposition only
+  int timing = 0;  // 0 off, 1 every stage, 2 the deposition only (per group)
   // events the next tiled deposition records with its own dispatch (begin,
   // end), or null: set by the timed frame loop around launch_deposit
   hipEvent_t dep_ev[2] = {nullptr, nullptr};
   std::vector<hipEvent_t> tev;
-  int64_t timed_frames = 0;  // frames timed since the last mdsf_stage_times
+  int64_t timed_groups = 0;  // groups timed since the last mdsf_stage_times
+  int64_t timed_frames = 0;  // and their frames
   hipEvent_t ev_fork = nullptr;
   hipEvent_t ev_prep[kSlots] = {}, ev_dep[kSlots] = {}, ev_fft[kSlots] = {};
   // adjoint (allocated on first use)
@@ -287,7 +313,7 @@ int hip_fail(hipError_t e, const char* what);
 hipError_t launch_prep(Plan& p, void* coords, int dtype, int arith, const int32_t* types,
                        const double* scale3, const double box[3], int64_t wrap_lo,
                        int64_t wrap_hi, uint32_t* occ, int32_t* home, hipStream_t s,
-                       bool coords_only = false, bool write_back = true);
+                       bool coords_only = false, bool write_back = true, int home_frame = 0);
 // sorts the prepared atoms and builds their tile slices; with `derivs` (and
 // dslices allocated) also the slices' derivatives for the tiled adjoint.
 // With `aux`, the tile lists are built on that stream, in parallel with the

@@ -8,6 +8,7 @@
 //   home cell      dens.py:285     ir = int(r / dr)   (FP64 IEEE division, truncation)
 //   window         dens.py:287-297 padded indices [ir-A+Nb, ir+A+Nb)
 //   Gaussian       dens.py:299-308 (Nel/sig^3) exp(-|(r - x_v) ucell|^2 / (2 sig^2))
+#include <algorithm>
 #include <climits>
 
 #include "mdsf_internal.h"
@@ -31,9 +32,17 @@ __global__ void k_prep(T* __restrict__ coords, SysDev sys, const TypeDev* __rest
                        int4* __restrict__ ir4, int* __restrict__ key, double* __restrict__ rpos,
                        int* __restrict__ bcount, unsigned* __restrict__ occ,
                        int* __restrict__ home, int* __restrict__ err, int coords_only,
-                       int write_back) {
+                       int write_back, int home_frame) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= sys.natoms) return;
+  const int fr = blockIdx.y;
+  coords += 3 * fr * sys.f_atoms();
+  scale += 3 * fr;
+  ir4 += fr * sys.f_atoms();
+  key += fr * sys.f_atoms();
+  rpos += 3 * fr * sys.f_atoms();
+  bcount += fr * sys.f_buckets();
+  if (fr != home_frame) home = nullptr;
   T x[3];
   x[0] = coords[3 * (size_t)i + 0];
   x[1] = coords[3 * (size_t)i + 1];
@@ -139,8 +148,11 @@ __device__ __forceinline__ int block_excl_scan(int v, int* wsum, int* total) {
 __global__ __launch_bounds__(kScanThreads) void k_scan_blocks(int* __restrict__ bcount,
                                                               int* __restrict__ boff,
                                                               int* __restrict__ aux, int nbk,
-                                                              int clear) {
+                                                              int clear, int naux) {
   __shared__ int wsum[kScanThreads / 64];
+  bcount += blockIdx.y * (nbk + 1LL);
+  boff += blockIdx.y * (nbk + 1LL);
+  aux += blockIdx.y * naux;
   const int i = blockIdx.x * kScanThreads + threadIdx.x;
   const int v = i < nbk ? bcount[i] : 0;
   int total;
@@ -155,8 +167,13 @@ __global__ __launch_bounds__(kScanThreads) void k_scan_blocks(int* __restrict__ 
 __global__ __launch_bounds__(kScanThreads) void k_scan_add(int* __restrict__ boff,
                                                            int* __restrict__ bcur,
                                                            const int* __restrict__ aux, int nbk,
-                                                           int nblocks, int* __restrict__ corners) {
+                                                           int nblocks, int* __restrict__ corners,
+                                                           int naux) {
   __shared__ int base_sh;
+  boff += blockIdx.y * (nbk + 1LL);
+  bcur += blockIdx.y * (nbk + 1LL);
+  aux += blockIdx.y * naux;
+  corners += blockIdx.y * kCornerInts;
   if (blockIdx.x == 0 && threadIdx.x == 0) corners[0] = 0;  // refilled by k_rank_gather
   if (threadIdx.x < 64) {
     int s = 0;
@@ -177,9 +194,12 @@ __global__ __launch_bounds__(kScanThreads) void k_scan_add(int* __restrict__ bof
 }
 
 __global__ void k_fill(const int* __restrict__ key, int* __restrict__ bcur,
-                       int* __restrict__ s_tmp, int natoms) {
+                       int* __restrict__ s_tmp, int natoms, int nbk) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= natoms) return;
+  key += blockIdx.y * (long long)natoms;
+  s_tmp += blockIdx.y * (long long)natoms;
+  bcur += blockIdx.y * (nbk + 1LL);
   const int b = key[i];
   if (b < 0) return;
   const int pos = atomicAdd(&bcur[b], 1);
@@ -197,9 +217,19 @@ __global__ void k_rank_gather(const int* __restrict__ key, const int* __restrict
                               const int* __restrict__ s_tmp, int* __restrict__ s_idx,
                               const int4* __restrict__ ir4, const double* __restrict__ rpos,
                               int4* __restrict__ s_ir, double* __restrict__ s_r,
-                              const int* __restrict__ nvalid, int* __restrict__ corners) {
+                              int natoms, int nbk, int* __restrict__ corners) {
   const int p = blockIdx.x * blockDim.x + threadIdx.x;
-  if (p >= *nvalid) return;
+  const long long fa = blockIdx.y * (long long)natoms;
+  boff += blockIdx.y * (nbk + 1LL);
+  if (p >= boff[nbk]) return;
+  key += fa;
+  s_tmp += fa;
+  s_idx += fa;
+  ir4 += fa;
+  rpos += 3 * fa;
+  s_ir += fa;
+  s_r += 3 * fa;
+  corners += blockIdx.y * kCornerInts;
   const int i = s_tmp[p];
   const int b = key[i];
   const int lo = boff[b], hi = boff[b + 1];
@@ -232,6 +262,9 @@ __global__ __launch_bounds__(kOrderThreads) void k_corner_order(SysDev sys,
                                                                 int nflag) {
   __shared__ int lst[kCornerCap];
   __shared__ int nrel;
+  s_ir += blockIdx.y * sys.f_atoms();
+  corners += blockIdx.y * kCornerInts;
+  if (flag) flag += blockIdx.y * (long long)nflag;
   const int n = min(corners[0], kCornerCap);
   if (threadIdx.x == 0) nrel = 0;
   // spill tile flags (staged spill): cleared, then set per spilling atom below;
@@ -276,6 +309,9 @@ __global__ void k_tables(SysDev sys, const TypeDev* __restrict__ td, const int4*
 #pragma clang fp contract(off)
   const long long g = blockIdx.x * (long long)blockDim.x + threadIdx.x;
   if (g >= total) return;
+  s_ir += blockIdx.y * sys.f_atoms();
+  s_r += 3 * blockIdx.y * sys.f_atoms();
+  tables += blockIdx.y * sys.f_tables;
   int t = 0;
   while (t + 1 < sys.ntypes && td[t + 1].table_base <= g) ++t;
   const TypeDev& ty = td[t];
@@ -329,14 +365,21 @@ __global__ void k_tables(SysDev sys, const TypeDev* __restrict__ td, const int4*
 // regular x slice cells and BY = b_y at the regular y slice cells (0 outside
 // the window).
 __global__ void k_slices(SysDev sys, const TypeDev* __restrict__ td, const int4* __restrict__ s_ir,
-                         const double* __restrict__ s_r, const int* __restrict__ nvalid,
+                         const double* __restrict__ s_r, const int* __restrict__ boff,
                          float* __restrict__ slices, float* __restrict__ dslices,
                          float* __restrict__ bslices, int mode) {
 #pragma clang fp contract(off)
+  const int fr = blockIdx.y;
+  boff += fr * sys.f_buckets();
+  s_ir += fr * sys.f_atoms();
+  s_r += 3 * fr * sys.f_atoms();
+  slices += fr * sys.f_slices;
+  dslices += fr * sys.f_slices;
+  bslices += fr * sys.f_bslices;
   const long long g = blockIdx.x * (long long)blockDim.x + threadIdx.x;
   const int pair = (int)(g / kTile), i = (int)(g - (long long)pair * kTile);
   const int s = pair / 3, d = pair - 3 * (pair / 3);
-  if (s >= *nvalid) return;
+  if (s >= boff[sys.nbuckets]) return;
   const int4 q = s_ir[s];
   const int t = q.w & 0xffff;
   if (t >= sys.ntypes || (q.w & kAtomParked)) return;  // parked atoms have no slices
@@ -438,24 +481,27 @@ __global__ void k_slices(SysDev sys, const TypeDev* __restrict__ td, const int4*
 hipError_t launch_prep(Plan& p, void* coords, int dtype, int arith, const int32_t* types,
                        const double* scale3, const double box[3], int64_t wrap_lo,
                        int64_t wrap_hi, uint32_t* occ, int32_t* home, hipStream_t s,
-                       bool coords_only, bool write_back) {
+                       bool coords_only, bool write_back, int home_frame) {
   const int n = p.sys.natoms;
   const int co = coords_only ? 1 : 0;
   const int wb = write_back ? 1 : 0;
   if (n == 0) return hipSuccess;
-  const dim3 grid((n + 255) / 256), block(256);
+  const dim3 grid((n + 255) / 256, p.nfr), block(256);
   if (dtype == MDSF_F32 && arith == MDSF_F32) {
     hipLaunchKernelGGL((k_prep<float, float>), grid, block, 0, s, (float*)coords, p.sys, p.types,
                        types, scale3, box[0], box[1], box[2], (long long)wrap_lo,
-                       (long long)wrap_hi, p.ir4, p.key, p.rpos, p.bucket_count, occ, home, p.err, co, wb);
+                       (long long)wrap_hi, p.ir4, p.key, p.rpos, p.bucket_count, occ, home, p.err, co, wb,
+                       home_frame);
   } else if (dtype == MDSF_F32) {
     hipLaunchKernelGGL((k_prep<float, double>), grid, block, 0, s, (float*)coords, p.sys, p.types,
                        types, scale3, box[0], box[1], box[2], (long long)wrap_lo,
-                       (long long)wrap_hi, p.ir4, p.key, p.rpos, p.bucket_count, occ, home, p.err, co, wb);
+                       (long long)wrap_hi, p.ir4, p.key, p.rpos, p.bucket_count, occ, home, p.err, co, wb,
+                       home_frame);
   } else {
     hipLaunchKernelGGL((k_prep<double, double>), grid, block, 0, s, (double*)coords, p.sys,
                        p.types, types, scale3, box[0], box[1], box[2], (long long)wrap_lo,
-                       (long long)wrap_hi, p.ir4, p.key, p.rpos, p.bucket_count, occ, home, p.err, co, wb);
+                       (long long)wrap_hi, p.ir4, p.key, p.rpos, p.bucket_count, occ, home, p.err, co, wb,
+                       home_frame);
   }
   return hipGetLastError();
 }
@@ -465,23 +511,24 @@ hipError_t launch_rescale(void* coords, int dtype, int arith, long long nframes,
   if (natoms == 0 || nframes == 0) return hipSuccess;
   SysDev sys{};
   sys.natoms = natoms;
-  const dim3 grid((natoms + 255) / 256), block(256);
   const size_t fstride = (size_t)natoms * 3;
-  for (long long t = 0; t < nframes; ++t) {
+  constexpr long long kMaxY = 32768;   // frames per launch (grid y)
+  for (long long t = 0; t < nframes; t += kMaxY) {
+    const dim3 grid((natoms + 255) / 256, (unsigned)std::min(kMaxY, nframes - t)), block(256);
     // wrap range [0, 0): the coordinates are only rescaled (dens.py:54-58)
     if (dtype == MDSF_F32 && arith == MDSF_F32)
       hipLaunchKernelGGL((k_prep<float, float>), grid, block, 0, s, (float*)coords + t * fstride,
                          sys, nullptr, nullptr, scale + 3 * t, 0.0, 0.0, 0.0, 0LL, 0LL, nullptr,
-                         nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, 1, 1);
+                         nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, 1, 1, 0);
     else if (dtype == MDSF_F32)
       hipLaunchKernelGGL((k_prep<float, double>), grid, block, 0, s, (float*)coords + t * fstride,
                          sys, nullptr, nullptr, scale + 3 * t, 0.0, 0.0, 0.0, 0LL, 0LL, nullptr,
-                         nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, 1, 1);
+                         nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, 1, 1, 0);
     else
       hipLaunchKernelGGL((k_prep<double, double>), grid, block, 0, s,
                          (double*)coords + t * fstride, sys, nullptr, nullptr, scale + 3 * t, 0.0,
                          0.0, 0.0, 0LL, 0LL, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr,
-                         nullptr, 1, 1);
+                         nullptr, 1, 1, 0);
   }
   return hipGetLastError();
 }
@@ -489,9 +536,9 @@ hipError_t launch_rescale(void* coords, int dtype, int arith, long long nframes,
 hipError_t launch_slice_derivs(Plan& p, hipStream_t s) {
   const int n = p.sys.natoms;
   if (n == 0 || p.slice_floats == 0 || !p.dslices) return hipSuccess;
-  hipLaunchKernelGGL(k_slices, dim3((unsigned)((3LL * kTile * n + 255) / 256)), dim3(256), 0, s,
-                     p.sys, p.types, p.s_ir, p.s_r, p.bucket_off + p.sys.nbuckets, p.slices,
-                     p.dslices, p.bslices, 2);
+  hipLaunchKernelGGL(k_slices, dim3((unsigned)((3LL * kTile * n + 255) / 256), p.nfr), dim3(256), 0,
+                     s, p.sys, p.types, p.s_ir, p.s_r, p.bucket_off, p.slices, p.dslices, p.bslices,
+                     2);
   return hipGetLastError();
 }
 
@@ -515,16 +562,17 @@ hipError_t launch_binning(Plan& p, hipStream_t s, bool derivs, hipStream_t aux,
         (e = launch_tile_regions(p, aux)) != hipSuccess)
       return e;
   }
-  hipLaunchKernelGGL(k_scan_blocks, dim3(nblk), dim3(kScanThreads), 0, s, p.bucket_count,
-                     p.bucket_off, p.bucket_aux, nbk, lists ? 0 : 1);
-  hipLaunchKernelGGL(k_scan_add, dim3(nblk), dim3(kScanThreads), 0, s, p.bucket_off,
-                     p.bucket_cur, p.bucket_aux, nbk, nblk, p.corners);
+  const unsigned nf = (unsigned)p.nfr;
+  hipLaunchKernelGGL(k_scan_blocks, dim3(nblk, nf), dim3(kScanThreads), 0, s, p.bucket_count,
+                     p.bucket_off, p.bucket_aux, nbk, lists ? 0 : 1, p.sys.f_aux);
+  hipLaunchKernelGGL(k_scan_add, dim3(nblk, nf), dim3(kScanThreads), 0, s, p.bucket_off,
+                     p.bucket_cur, p.bucket_aux, nbk, nblk, p.corners, p.sys.f_aux);
   if (n == 0) return hipGetLastError();
-  hipLaunchKernelGGL(k_fill, dim3((n + 255) / 256), dim3(256), 0, s, p.key, p.bucket_cur,
-                     p.s_tmp, n);
-  hipLaunchKernelGGL(k_rank_gather, dim3((n + 255) / 256), dim3(256), 0, s, p.key,
-                     p.bucket_off, p.s_tmp, p.s_idx, p.ir4, p.rpos, p.s_ir, p.s_r,
-                     p.bucket_off + nbk, p.corners);
+  hipLaunchKernelGGL(k_fill, dim3((n + 255) / 256, nf), dim3(256), 0, s, p.key, p.bucket_cur,
+                     p.s_tmp, n, nbk);
+  hipLaunchKernelGGL(k_rank_gather, dim3((n + 255) / 256, nf), dim3(256), 0, s, p.key,
+                     p.bucket_off, p.s_tmp, p.s_idx, p.ir4, p.rpos, p.s_ir, p.s_r, n, nbk,
+                     p.corners);
   if (split || side) {
     if ((e = hipEventRecord(p.ev_lgath, s)) != hipSuccess) return e;
   }
@@ -540,19 +588,19 @@ hipError_t launch_binning(Plan& p, hipStream_t s, bool derivs, hipStream_t aux,
   }
   const hipStream_t cs = side ? side : s;
   if (side && (e = hipStreamWaitEvent(side, p.ev_lgath, 0)) != hipSuccess) return e;
-  hipLaunchKernelGGL(k_corner_order, dim3(1), dim3(kOrderThreads), 0, cs, p.sys, p.types, p.s_ir,
+  hipLaunchKernelGGL(k_corner_order, dim3(1, nf), dim3(kOrderThreads), 0, cs, p.sys, p.types, p.s_ir,
                      p.corners, p.spill ? p.spill_flag : nullptr,
                      (int)(p.spill ? p.spill_tiles : 0));
   // the corner-fold spill, staged for the deposition of this frame
   if ((e = launch_spill_stage(p, cs)) != hipSuccess) return e;
   if (p.slice_floats > 0)
-    hipLaunchKernelGGL(k_slices, dim3((unsigned)((3LL * kTile * n + 255) / 256)), dim3(256), 0, s,
-                       p.sys, p.types, p.s_ir, p.s_r, p.bucket_off + nbk, p.slices, p.dslices,
+    hipLaunchKernelGGL(k_slices, dim3((unsigned)((3LL * kTile * n + 255) / 256), nf), dim3(256), 0,
+                       s, p.sys, p.types, p.s_ir, p.s_r, p.bucket_off, p.slices, p.dslices,
                        p.bslices, (derivs && p.dslices) ? 1 : 0);
   // factor tables feed the FP64 gather
   const long long total = p.fft64 ? p.table_floats : 0;
   if (total > 0) {
-    const dim3 grid((unsigned)((total + 255) / 256)), block(256);
+    const dim3 grid((unsigned)((total + 255) / 256), nf), block(256);
     if (p.fft64)
       hipLaunchKernelGGL(k_tables<double>, grid, block, 0, s, p.sys, p.types, p.s_ir, p.s_r,
                          static_cast<double*>(p.tables), total);
