@@ -21,27 +21,27 @@ def _check(n, fp64=True):
     from mdsf import engine
     plan = engine.Plan(n, 0, [1.0] * 3, np.eye(3), [], [], [], [], fft64=fp64)
     g = torch.Generator().manual_seed(sum(n))
-    d = torch.rand(n, dtype=torch.float64, generator=g).cuda() - 0.5
+    d = torch.rand(n, dtype=torch.float64, generator=g) - 0.5
     if not fp64:
         d = d.float().double()
-    want = torch.fft.rfftn(d)
+    want = torch.fft.rfftn(d)   # on the host
     top = float(want.abs().max())
     # direct DFTs of primes up to 509 add 254 products: (n_x + n_y + n_z) eps of the largest bin
     # bounds every stage; FP32 storage adds half an ulp (2^-24) of each pass's values, spread by the
     # next pass over sqrt(n) bins
     tol = sum(n) * EPS if fp64 else 3 * 2.0 ** -24
-    got = plan.rfft3(d)
+    got = plan.rfft3(d).cpu()
     assert float((got - want).abs().max()) <= tol * top * (1 if fp64 else 4)
     s = want.abs().square()
     plan.reset()
     plan.accumulate_density(d)
     plan.accumulate_density(d)
-    assert float((plan.sf() - 2 * s).abs().max()) <= 16 * tol * float(s.max())
+    assert float((plan.sf().cpu() - 2 * s).abs().max()) <= 16 * tol * float(s.max())
     if fp64:
-        w = torch.randn(s.shape, dtype=torch.float64, generator=g).cuda()
+        w = torch.randn(s.shape, dtype=torch.float64, generator=g)
         x = d.clone().requires_grad_(True)
         (torch.fft.rfftn(x).abs().square() * w).sum().backward()
-        grad = plan.density_adjoint(d, w)
+        grad = plan.density_adjoint(d, w).cpu()
         bound = 4 * sum(n) * EPS * float((w * want).abs().square().sum().sqrt()) * 4
         assert float((grad - x.grad).abs().max()) <= bound
     plan.close()
