@@ -313,7 +313,10 @@ int mdsf_plan_create(const mdsf_grid_desc* desc, mdsf_plan** out) {
     const double c = 2.0 * std::fabs(s.g01) * 1.4426950408889634 / ty.two_sig2;
     if (c * (ty.half[0] + 1) * s.dr[0] * (ty.half[1] + 1) * s.dr[1] > 100.0) xy_lists = false;
   }
-  p->slice_floats = (!p->fft64 && (s.mode == MODE_DIAG || xy_lists)) ? slice_floats : 0;
+  // FP64 orthogonal cells too, as long as their slices and lists fit the bounds
+  // (else, and in the other cells, the FP64 plan gathers from factor tables)
+  p->slice_floats = (s.mode == MODE_DIAG || xy_lists) ? slice_floats : 0;
+  if (p->fft64 && (s.mode != MODE_DIAG || slice_floats >= (1LL << 31))) p->slice_floats = 0;
   p->bslice_floats = xy_lists ? regular_floats : 0;
   if (p->slice_floats >= (1LL << 31)) {  // the deposition addresses slices with 32-bit offsets
     free_plan(p);
@@ -341,6 +344,7 @@ int mdsf_plan_create(const mdsf_grid_desc* desc, mdsf_plan** out) {
       cap += (long long)ty.count * per_atom;
     }
     if (ok && cap < (1LL << 31)) p->tl_cap = std::max(cap, 1LL);
+    if (p->fft64 && p->tl_cap == 0) p->slice_floats = 0;
   }
   {  // tiled adjoint result slots: per atom one per tile slice triple
     long long slots = 0;
@@ -349,7 +353,7 @@ int mdsf_plan_create(const mdsf_grid_desc* desc, mdsf_plan** out) {
       ty.adjt_base = slots;
       slots += (long long)ty.count * ty.nsl[0] * ty.nsl[1] * ty.nsl[2];
     }
-    p->adj_tslots = (p->slice_floats > 0 && s.mode == MODE_DIAG) ? slots : 0;
+    p->adj_tslots = (p->slice_floats > 0 && s.mode == MODE_DIAG && !p->fft64) ? slots : 0;
   }
   // adjoint work items (atom, x-chunk of <= 64 planes, chunk of (y, z)
   // pairs sized for ~16k window voxels), heaviest windows numbered first so
@@ -384,7 +388,8 @@ int mdsf_plan_create(const mdsf_grid_desc* desc, mdsf_plan** out) {
   // frames per group (kGroupTiles), within the state budget
   s.f_slices = p->slice_floats;
   s.f_bslices = p->bslice_floats;
-  s.f_tables = p->fft64 ? table_floats : 0;
+  const bool tables = p->fft64 && s.mode != MODE_GEN && p->slice_floats == 0;
+  s.f_tables = tables ? table_floats : 0;
   const bool staged = p->spill_tiles > 0 && p->spill_tiles <= kMaxSpillBufTiles;
   s.f_spill = staged ? p->spill_tiles * kTile * kTile * kTile : 0;
   s.f_points = (long long)desc->n[0] * desc->n[1] * desc->n[2];
@@ -396,7 +401,7 @@ int mdsf_plan_create(const mdsf_grid_desc* desc, mdsf_plan** out) {
   {
     const size_t rs = p->fft64 ? 8 : 4;
     const size_t bytes = (size_t)desc->natoms * 112 + (size_t)s.nbuckets * 12 +
-                         (size_t)p->slice_floats * 4 + (size_t)p->bslice_floats * 4 +
+                         (size_t)p->slice_floats * rs + (size_t)p->bslice_floats * 4 +
                          (size_t)s.f_tables * 8 + (size_t)s.f_spill * rs + (size_t)p->tl_cap * 8 +
                          (size_t)s.f_points * rs + fft_spec_bytes(s.n, p->fft64) +
                          fft_res_bytes(s.n, p->fft64) + (size_t)desc->n[0] * desc->n[1] * 16;
@@ -434,9 +439,8 @@ int mdsf_plan_create(const mdsf_grid_desc* desc, mdsf_plan** out) {
     arena.add(&f.s_tmp, nat);
     arena.add(&f.s_ir, nat);
     arena.add(&f.s_r, 3 * nat);
-    // (the FP32 path stages tile slices instead of tables)
-    arena.add(reinterpret_cast<double**>(&f.tables), p->fft64 ? grp * (size_t)table_floats : 1);
-    arena.add(&f.slices, grp * (size_t)p->slice_floats);
+    arena.add(reinterpret_cast<double**>(&f.tables), grp * (size_t)s.f_tables);
+    arena.add(&f.slices, grp * (size_t)p->slice_floats * (p->fft64 ? 2 : 1));   // plan precision
     if (p->bslice_floats > 0) arena.add(&f.bslices, grp * (size_t)p->bslice_floats);
     arena.add(&f.corners, grp * kCornerInts, true);
     if (staged) {

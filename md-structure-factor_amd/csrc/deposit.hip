@@ -1357,7 +1357,8 @@ void k_deposit_mfma(SysDev sys, const TypeDev* __restrict__ td,
 }
 
 // ---------------------------------------------------------------------------
-// Tile lists (FP32 orthogonal cells).  The candidate enumeration of the tiled
+// Tile lists (FP32 orthogonal and xy-coupled cells, FP64 orthogonal cells).  The
+// candidate enumeration of the tiled
 // deposition runs in the prepare stage as kernels of its own.  Each tile
 // gets a region of the slot's pool with one entry per candidate (the atoms of
 // the bucket columns that can reach it): k_tile_count counts them,
@@ -1591,30 +1592,58 @@ __global__ __launch_bounds__(kThreads) void k_tile_lists(SysDev sys, const TypeD
 // waves per SIMD ran 13% faster (126 -> 109 us at 256^3, 50 k atoms)
 constexpr int kXYStageBuffers = 1;
 
-template <bool XY>
+template <bool XY, typename F>
 struct StageRows {
-  __align__(16) float vx[NV + 1][T];  // row NV stays zero: the lists' padding row
-  __align__(16) float vy[NV + 1][T];
-  __align__(16) float vz[NV + 1][T];
+  __align__(16) F vx[NV + 1][T];  // row NV stays zero: the lists' padding row
+  __align__(16) F vy[NV + 1][T];
+  __align__(16) F vz[NV + 1][T];
   __align__(16) float cx[XY ? NV + 1 : 1][T];
   __align__(16) float by[XY ? NV + 1 : 1][T];
   // per row and wave w: nonzero X on x rows 4w..4w+3
   __align__(4) unsigned char vq[NV][4];
 };
 
-template <int MT, bool XY>
+// FP64 plans (F = double): the same with v_mfma_f64_16x16x4f64 (lane l holds rows
+// l / 16 + 4 r of column l % 16), one staging buffer (26 KB) and one running sum
+// (it rounds to nearest).
+template <typename F>
+struct Mfma;
+template <>
+struct Mfma<float> {
+  typedef float V __attribute__((ext_vector_type(4)));
+  typedef float4 Q;   // a quarter row
+  static __device__ __forceinline__ V mul(float a, float b, V c) {
+    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+  }
+  static __device__ __forceinline__ int row(int lane, int r) { return 4 * (lane >> 4) + r; }
+};
+template <>
+struct Mfma<double> {
+  typedef double V __attribute__((ext_vector_type(4)));
+  typedef double Q __attribute__((ext_vector_type(4), aligned(16)));
+  static __device__ __forceinline__ V mul(double a, double b, V c) {
+    return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
+  }
+  static __device__ __forceinline__ int row(int lane, int r) { return (lane >> 4) + 4 * r; }
+};
+
+template <int MT, bool XY, typename F>
 __device__ __forceinline__ void deposit_lists(SysDev sys, const TypeDev* __restrict__ td,
                                               const int2* __restrict__ pool,
                                               const int4* __restrict__ heads,
-                                              const float* __restrict__ slices,
+                                              const F* __restrict__ slices,
                                               const float* __restrict__ bslices,
-                                              const float* __restrict__ spill,
+                                              const F* __restrict__ spill,
                                               const int* __restrict__ spill_flag,
-                                              float* __restrict__ rho) {
+                                              F* __restrict__ rho) {
+  using M = Mfma<F>;
+  using Q = typename M::Q;
+  using V = typename M::V;
+  constexpr bool F32 = sizeof(F) == 4;
   // staging buffers: two (the next batch is staged while this one's MFMAs
-  // run) or, for xy-coupled cells, kXYStageBuffers
-  constexpr int NB = XY ? kXYStageBuffers : 2;
-  __shared__ StageRows<XY> st[NB];
+  // run) or, for xy-coupled cells and in FP64, kXYStageBuffers
+  constexpr int NB = XY || !F32 ? kXYStageBuffers : 2;
+  __shared__ StageRows<XY, F> st[NB];
   // per wave: the rows it accumulates, padded to a multiple of 4 with NV
   __shared__ unsigned char wl[kThreads / 64][NV + 4];
   // per type: slice axis offsets (in slices) of the regular and the corner
@@ -1651,7 +1680,7 @@ __device__ __forceinline__ void deposit_lists(SysDev sys, const TypeDev* __restr
   if (tid < T) {
 #pragma unroll
     for (int b = 0; b < NB; ++b) {
-      st[b].vx[NV][tid] = st[b].vy[NV][tid] = st[b].vz[NV][tid] = 0.f;
+      st[b].vx[NV][tid] = st[b].vy[NV][tid] = st[b].vz[NV][tid] = (F)0;
       if constexpr (XY) st[b].cx[NV][tid] = st[b].by[NV][tid] = 0.f;
     }
   }
@@ -1666,22 +1695,23 @@ __device__ __forceinline__ void deposit_lists(SysDev sys, const TypeDev* __restr
   // rounds its partial sums toward zero (measured: 99.5% of a dense tile's
   // voxels came out low, by 9e-7 relative after a few hundred rank-1 terms),
   // so the biased roundings act on batch-sized partial sums only.
-  v4f tot[4];
+  V tot[4];
 #pragma unroll
-  for (int b = 0; b < 4; ++b) tot[b] = v4f{0.f, 0.f, 0.f, 0.f};
+  for (int b = 0; b < 4; ++b) tot[b] = V{0, 0, 0, 0};
   const int q4 = tid & 3;
   // a virtual atom's quarter rows: X, Y (XY: LY), Z and (XY) CX, BY
   struct Rows {
-    float4 x, y, z, cx, by;
+    Q x, y, z;
+    float4 cx, by;
   };
   // quarter slices at float offsets o0..o2 (-1: none, zero; XY: a missing LY
   // is -inf) and (XY) the cross rows at ox, oy (-1: none, zero); a missing one
   // loads the buffer's first quarter slice and replaces it, so the loads go
   // out unconditionally
   auto load = [&](int o0, int o1, int o2, int ox, int oy, Rows& v) {
-    v.x = *reinterpret_cast<const float4*>(slices + max(o0, 0) + 4 * q4);
-    v.y = *reinterpret_cast<const float4*>(slices + max(o1, 0) + 4 * q4);
-    v.z = *reinterpret_cast<const float4*>(slices + max(o2, 0) + 4 * q4);
+    v.x = *reinterpret_cast<const Q*>(slices + max(o0, 0) + 4 * q4);
+    v.y = *reinterpret_cast<const Q*>(slices + max(o1, 0) + 4 * q4);
+    v.z = *reinterpret_cast<const Q*>(slices + max(o2, 0) + 4 * q4);
     const float4 z4 = make_float4(0.f, 0.f, 0.f, 0.f);
     if constexpr (XY) {
       v.cx = *reinterpret_cast<const float4*>(bslices + max(ox, 0) + 4 * q4);
@@ -1689,23 +1719,29 @@ __device__ __forceinline__ void deposit_lists(SysDev sys, const TypeDev* __restr
       if (ox < 0) v.cx = z4;
       if (oy < 0) v.by = z4;
     }
-    const float ly0 = XY ? -__builtin_inff() : 0.f;
-    if (o0 < 0) v.x = z4;
-    if (o1 < 0) v.y = make_float4(ly0, ly0, ly0, ly0);
-    if (o2 < 0) v.z = z4;
+    if constexpr (F32) {
+      const float ly0 = XY ? -__builtin_inff() : 0.f;
+      if (o0 < 0) v.x = z4;
+      if (o1 < 0) v.y = make_float4(ly0, ly0, ly0, ly0);
+      if (o2 < 0) v.z = z4;
+    } else {
+      if (o0 < 0) v.x = Q{0, 0, 0, 0};
+      if (o1 < 0) v.y = Q{0, 0, 0, 0};
+      if (o2 < 0) v.z = Q{0, 0, 0, 0};
+    }
   };
-  auto stage = [&](StageRows<XY>& sb, int row, const Rows& v) {
-    *reinterpret_cast<float4*>(&sb.vx[row][4 * q4]) = v.x;
-    *reinterpret_cast<float4*>(&sb.vy[row][4 * q4]) = v.y;
-    *reinterpret_cast<float4*>(&sb.vz[row][4 * q4]) = v.z;
+  auto stage = [&](StageRows<XY, F>& sb, int row, const Rows& v) {
+    *reinterpret_cast<Q*>(&sb.vx[row][4 * q4]) = v.x;
+    *reinterpret_cast<Q*>(&sb.vy[row][4 * q4]) = v.y;
+    *reinterpret_cast<Q*>(&sb.vz[row][4 * q4]) = v.z;
     if constexpr (XY) {
       *reinterpret_cast<float4*>(&sb.cx[row][4 * q4]) = v.cx;
       *reinterpret_cast<float4*>(&sb.by[row][4 * q4]) = v.by;
     }
-    sb.vq[row][q4] = (v.x.x != 0.f || v.x.y != 0.f || v.x.z != 0.f || v.x.w != 0.f) ? 1 : 0;
+    sb.vq[row][q4] = (v.x.x != 0 || v.x.y != 0 || v.x.z != 0 || v.x.w != 0) ? 1 : 0;
   };
   // A operand of virtual atom k at x row xr, y = jj
-  auto aop = [&](const StageRows<XY>& sb, int k, int xr, float yv, float bv) -> float {
+  auto aop = [&](const StageRows<XY, F>& sb, int k, int xr, F yv, float bv) -> F {
     if constexpr (XY)
       return sb.vx[k][xr] * __builtin_amdgcn_exp2f(fmaf(sb.cx[k][xr], bv, yv));
     else
@@ -1714,7 +1750,7 @@ __device__ __forceinline__ void deposit_lists(SysDev sys, const TypeDev* __restr
   // MFMA accumulation of staged rows [0, vtot) of sb: the wave's list holds
   // the rows with nonzero X on its 4 x rows, padded with the zero row NV;
   // the first group starts from a zero accumulator
-  auto accumulate = [&](const StageRows<XY>& sb, int vtot) {
+  auto accumulate = [&](const StageRows<XY, F>& sb, int vtot) {
     const int kk = lane >> 4, jj = lane & 15;
     const bool on = lane < vtot && sb.vq[lane][wave] != 0;
     const unsigned long long bm = __ballot(on);
@@ -1725,25 +1761,30 @@ __device__ __forceinline__ void deposit_lists(SysDev sys, const TypeDev* __restr
     if (lane >= cnt && lane < kend) wl[wave][lane] = (unsigned char)NV;
     __builtin_amdgcn_wave_barrier();
     if (kend == 0) return;
-    v4f acc[4];
-    {
+    V acc[4];
+    if constexpr (F32) {
       const int k = wl[wave][kk];
-      const float zv = sb.vz[k][jj], yv = sb.vy[k][jj], bv = XY ? sb.by[k][jj] : 0.f;
+      const F zv = sb.vz[k][jj], yv = sb.vy[k][jj];
+      const float bv = XY ? sb.by[k][jj] : 0.f;
 #pragma unroll
       for (int b = 0; b < 4; ++b)
-        acc[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(aop(sb, k, 4 * wave + b, yv, bv), zv,
-                                                      v4f{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+        acc[b] = M::mul(aop(sb, k, 4 * wave + b, yv, bv), zv, V{0, 0, 0, 0});
+    } else {
+#pragma unroll
+      for (int b = 0; b < 4; ++b) acc[b] = tot[b];
     }
-    for (int k0 = 4; k0 < kend; k0 += 4) {
+    for (int k0 = F32 ? 4 : 0; k0 < kend; k0 += 4) {
       const int k = wl[wave][k0 + kk];
-      const float zv = sb.vz[k][jj], yv = sb.vy[k][jj], bv = XY ? sb.by[k][jj] : 0.f;
+      const F zv = sb.vz[k][jj], yv = sb.vy[k][jj];
+      const float bv = XY ? sb.by[k][jj] : 0.f;
 #pragma unroll
-      for (int b = 0; b < 4; ++b)
-        acc[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(aop(sb, k, 4 * wave + b, yv, bv), zv, acc[b],
-                                                      0, 0, 0);
+      for (int b = 0; b < 4; ++b) acc[b] = M::mul(aop(sb, k, 4 * wave + b, yv, bv), zv, acc[b]);
     }
 #pragma unroll
-    for (int b = 0; b < 4; ++b) tot[b] += acc[b];
+    for (int b = 0; b < 4; ++b) {
+      if constexpr (F32) tot[b] += acc[b];
+      else tot[b] = acc[b];
+    }
   };
 
   // regular atoms: lanes 4a .. 4a + 3 take atom a of the batch
@@ -1828,17 +1869,17 @@ __device__ __forceinline__ void deposit_lists(SysDev sys, const TypeDev* __restr
     accumulate(st[0], 4 * nca);
   }
 
-  // D[y][z] of block b: lane l holds y = 4 (l / 16) + r, z = l % 16
+  // D[y][z] of block b: lane l holds y = row(l, r), z = l % 16
   const int gz = tl.t0[2] + (lane & 15);
-  const float* sp = spill_stage_tile(sys, spill, spill_flag, tl);
+  const F* sp = spill_stage_tile(sys, spill, spill_flag, tl);
 #pragma unroll
   for (int b = 0; b < 4; ++b) {
     const int gx = tl.t0[0] + 4 * wave + b;
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-      const int gy = tl.t0[1] + 4 * (lane >> 4) + r;
+      const int gy = tl.t0[1] + M::row(lane, r);
       if (gx < tl.t1[0] && gy < tl.t1[1] && gz < tl.t1[2]) {
-        float v = tot[b][r];
+        F v = tot[b][r];
         if (sp) v += sp[((gy - tl.t0[1]) * T + (gx - tl.t0[0])) * T + (gz - tl.t0[2])];
         rho[((size_t)gx * sys.n[1] + gy) * sys.n[2] + gz] = v;
       }
@@ -1853,7 +1894,7 @@ void k_deposit_lists(SysDev sys, const TypeDev* __restrict__ td, const int2* __r
                      const int4* __restrict__ heads, const float* __restrict__ slices,
                      const float* __restrict__ bslices, const float* __restrict__ spill,
                      const int* __restrict__ spill_flag, float* __restrict__ rho) {
-  deposit_lists<MT, false>(sys, td, pool, heads, slices, bslices, spill, spill_flag, rho);
+  deposit_lists<MT, false, float>(sys, td, pool, heads, slices, bslices, spill, spill_flag, rho);
 }
 
 // xy-coupled cells: five rows per virtual atom in one staging buffer, 22 KB
@@ -1864,7 +1905,20 @@ void k_deposit_lists_xy(SysDev sys, const TypeDev* __restrict__ td, const int2* 
                         const int4* __restrict__ heads, const float* __restrict__ slices,
                         const float* __restrict__ bslices, const float* __restrict__ spill,
                         const int* __restrict__ spill_flag, float* __restrict__ rho) {
-  deposit_lists<MT, true>(sys, td, pool, heads, slices, bslices, spill, spill_flag, rho);
+  deposit_lists<MT, true, float>(sys, td, pool, heads, slices, bslices, spill, spill_flag, rho);
+}
+
+// FP64 plans, orthogonal cells.  The gather they took (k_deposit: its own candidate
+// enumeration, a lane per (x, y) column and 16 FMAs per atom fed from LDS) ran a
+// frame of 20,000 atoms at 128^3 in 289 us; the loop over four of them took 1,077 us
+// and takes 431.
+template <int MT>
+__global__ __launch_bounds__(kThreads)
+void k_deposit_lists64(SysDev sys, const TypeDev* __restrict__ td, const int2* __restrict__ pool,
+                       const int4* __restrict__ heads, const double* __restrict__ slices,
+                       const double* __restrict__ spill, const int* __restrict__ spill_flag,
+                       double* __restrict__ rho) {
+  deposit_lists<MT, false, double>(sys, td, pool, heads, slices, nullptr, spill, spill_flag, rho);
 }
 
 // ---------------------------------------------------------------------------
@@ -2418,7 +2472,13 @@ hipError_t launch_impl(Plan& p, ACC* out, const ACC* stage, hipStream_t s) {
       DEP_LAUNCH((k_deposit_mfma<MODE_XY, kMaxTypes>), sys, p.types,
                          p.bucket_off, p.s_ir, p.s_r, p.slices, stage, p.spill_flag, out);
   } else {
-    if (sys.mode == MODE_DIAG)
+    if (sys.mode == MODE_DIAG && p.tl_cap > 0 && sys.ntypes <= 16)
+      DEP_LAUNCH((k_deposit_lists64<16>), sys, p.types, p.tl_pool, p.tl_head,
+                 reinterpret_cast<const double*>(p.slices), stage, p.spill_flag, out);
+    else if (sys.mode == MODE_DIAG && p.tl_cap > 0)
+      DEP_LAUNCH((k_deposit_lists64<kMaxTypes>), sys, p.types, p.tl_pool, p.tl_head,
+                 reinterpret_cast<const double*>(p.slices), stage, p.spill_flag, out);
+    else if (sys.mode == MODE_DIAG)
       DEP_LAUNCH((k_deposit<MODE_DIAG, ACC>), sys, p.types,
                          p.bucket_off, p.s_ir, p.s_r, p.tables, stage, p.spill_flag, out);
     else

@@ -301,10 +301,9 @@ __global__ __launch_bounds__(kOrderThreads) void k_corner_order(SysDev sys,
 // Per-atom 1-D factor tables, one thread per entry:
 //   x: amp * exp(-g00 bx^2 / 2s^2), y: exp(-g11 by^2 / 2s^2), z: exp(-g22 bz^2 / 2s^2)
 // with b = r - (ir - A + k) dr in FP64 exactly as buf = r - grid (dens.py:252-256,299),
-// k in [0, 2A).  Values are rounded once to the plan's precision (FP32 or FP64).
-template <typename TT>
+// k in [0, 2A).  For the FP64 plans that do not deposit from tile slices.
 __global__ void k_tables(SysDev sys, const TypeDev* __restrict__ td, const int4* __restrict__ s_ir,
-                         const double* __restrict__ s_r, TT* __restrict__ tables,
+                         const double* __restrict__ s_r, double* __restrict__ tables,
                          long long total) {
 #pragma clang fp contract(off)
   const long long g = blockIdx.x * (long long)blockDim.x + threadIdx.x;
@@ -344,16 +343,16 @@ __global__ void k_tables(SysDev sys, const TypeDev* __restrict__ td, const int4*
   const double qv = (gm * (b * b)) / ty.two_sig2;
   double v = exp(-qv);
   if (d == 0) v = ty.amp * v;
-  tables[g] = (TT)v;
+  tables[g] = v;
 }
 
-// Tile slices for the FP32 deposition.  16 lanes per (sorted atom, axis),
+// Tile slices for the deposition from tile lists.  16 lanes per (sorted atom, axis),
 // lane i owning cell i of every slice, so that each slice row is written as
 // one contiguous 64-byte segment.  Slice j holds cell c = 16 T + i of tile
 // T = (T0 + j) mod ntiles (T0 = tile of the window start lo mod N); its value
 // is the sum over the periodic images u = c + sN (s = -1, 0, 1) inside the
 // window [lo, lo + 2A) of amp^[d==0] exp(-g_dd (r - u dr)^2 / 2 s^2): the
-// exponent in FP64, exp in FP32 (dens.py:252-256, 299-308).  Cells past N
+// exponent in FP64, exp in FP32 for FP32 plans (dens.py:252-256, 299-308).  Cells past N
 // are zero.
 //
 // xy-coupled cells (FP32 plans whose windows meet each x and y tile through
@@ -364,9 +363,13 @@ __global__ void k_tables(SysDev sys, const TypeDev* __restrict__ td, const int4*
 // instead of the factor; bslices holds CX = -2 g01 log2(e) / 2 s^2 b_x at the
 // regular x slice cells and BY = b_y at the regular y slice cells (0 outside
 // the window).
+//
+// F: the plan's element type.  FP64 plans (orthogonal cells) take the exponent and
+// exp as k_tables does, without derivatives.
+template <typename F>
 __global__ void k_slices(SysDev sys, const TypeDev* __restrict__ td, const int4* __restrict__ s_ir,
                          const double* __restrict__ s_r, const int* __restrict__ boff,
-                         float* __restrict__ slices, float* __restrict__ dslices,
+                         F* __restrict__ slices, F* __restrict__ dslices,
                          float* __restrict__ bslices, int mode) {
 #pragma clang fp contract(off)
   const int fr = blockIdx.y;
@@ -394,7 +397,9 @@ __global__ void k_slices(SysDev sys, const TypeDev* __restrict__ td, const int4*
   const double dr = d == 0 ? sys.dr[0] : (d == 1 ? sys.dr[1] : sys.dr[2]);
   const double gm = d == 0 ? sys.g00 : (d == 1 ? sys.g11 : sys.g22);
   const double gk = gm / ty.two_sig2;
-  const float am = d == 0 ? ty.amp_f : 1.f;
+  constexpr bool F32 = sizeof(F) == 4;
+  const F am = d == 0 ? (F32 ? (F)ty.amp_f : (F)ty.amp) : (F)1;
+  const double ts2 = ty.two_sig2;
   const double r = s_r[3 * (size_t)s + d];
   const int lo = ir - A, hi = ir + A;
   const int off_d = d == 0 ? 0 : (d == 1 ? kTile * ty.nsl[0] : kTile * (ty.nsl[0] + ty.nsl[1]));
@@ -404,24 +409,28 @@ __global__ void k_slices(SysDev sys, const TypeDev* __restrict__ td, const int4*
                                           : 2 * kTile * ty.nsl[0] + 3 * kTile * ty.nsl[1]);
   const long long acoff = ty.corner_base + (long long)slot * ty.corner_stride + coff_d + i;
   // mode 0: slices, 1: slices and derivatives, 2: derivatives only
-  const bool wv = mode != 2, wd = mode != 0;
+  const bool wv = mode != 2, wd = F32 && mode != 0;
   // factor of the image at grid coordinate u, 0 outside the window, and its
   // derivative in r: am exp(-gk b^2) and am exp(-gk b^2) (-2 gk b), b = r - u dr
-  auto f = [&](int u, float& df) -> float {
-    df = 0.f;
-    if (u < lo || u >= hi) return 0.f;
+  auto f = [&](int u, F& df) -> F {
+    df = (F)0;
+    if (u < lo || u >= hi) return (F)0;
     const double b = r - (double)u * dr;
-    const float v = am * expf(-(float)(gk * (b * b)));
-    df = v * (float)(-2.0 * gk * b);
-    return v;
+    if constexpr (F32) {
+      const float v = am * expf(-(float)(gk * (b * b)));
+      df = v * (float)(-2.0 * gk * b);
+      return v;
+    } else {
+      return am * exp(-((gm * (b * b)) / ts2));
+    }
   };
-  auto put = [&](long long o, float v, float dv) {
+  auto put = [&](long long o, F v, F dv) {
     if (wv) slices[o] = v;
     if (wd) dslices[o] = dv;
   };
   // xy-coupled cells (the branch is uniform across the grid; within it only
   // the bslices store depends on the axis)
-  const bool xy = sys.mode == MODE_XY;
+  const bool xy = F32 && sys.mode == MODE_XY;
   const bool ylog = xy && d == 1;
   constexpr double kLog2e = 1.4426950408889634;
   const double cxy = -2.0 * sys.g01 * kLog2e / ty.two_sig2;
@@ -436,8 +445,8 @@ __global__ void k_slices(SysDev sys, const TypeDev* __restrict__ td, const int4*
   for (int j = 0; j < nsl; ++j) {
     const int c = T * kTile + i;
     const bool in = c < N;
-    float dL = 0.f, dC = 0.f, dH = 0.f;
-    float vL = in ? f(c - N, dL) : 0.f, vC = in ? f(c, dC) : 0.f, vH = in ? f(c + N, dH) : 0.f;
+    F dL = 0, dC = 0, dH = 0;
+    F vL = in ? f(c - N, dL) : (F)0, vC = in ? f(c, dC) : (F)0, vH = in ? f(c + N, dH) : (F)0;
     if (xy) {
       // at most one image in the window (the plan's condition): its b gives
       // CX (x) or BY (y); y values become log2 (then the regular value, the
@@ -452,7 +461,8 @@ __global__ void k_slices(SysDev sys, const TypeDev* __restrict__ td, const int4*
         vH = in ? lg(c + N) : -__builtin_inff();
       }
     }
-    put(aoff + j * kTile, ylog ? fmaxf(fmaxf(vL, vC), vH) : vC + vL + vH, dC + dL + dH);
+    put(aoff + j * kTile, ylog ? (F)fmaxf(fmaxf((float)vL, (float)vC), (float)vH) : vC + vL + vH,
+        dC + dL + dH);
     if (corner) {
       // the components the corner virtual atoms take (dens.py:101-107): on z
       // the slots where the reference's corner copy lands for y on L / on H
@@ -465,9 +475,9 @@ __global__ void k_slices(SysDev sys, const TypeDev* __restrict__ td, const int4*
         put(acoff + (2 * nsl + j) * kTile, vH, dH);
       } else {
         const int u1 = c + sys.nb, u2 = c - sys.nb;
-        float d1 = 0.f, d2 = 0.f;
-        const float v1 = in && u1 >= N ? f(u1, d1) : 0.f;
-        const float v2 = in && u2 < 0 ? f(u2, d2) : 0.f;
+        F d1 = 0, d2 = 0;
+        const F v1 = in && u1 >= N ? f(u1, d1) : (F)0;
+        const F v2 = in && u2 < 0 ? f(u2, d2) : (F)0;
         put(acoff + j * kTile, vC + vL + v1, dC + dL + d1);
         put(acoff + (nsl + j) * kTile, vC + vH + v2, dC + dH + d2);
       }
@@ -536,8 +546,8 @@ hipError_t launch_rescale(void* coords, int dtype, int arith, long long nframes,
 hipError_t launch_slice_derivs(Plan& p, hipStream_t s) {
   const int n = p.sys.natoms;
   if (n == 0 || p.slice_floats == 0 || !p.dslices) return hipSuccess;
-  hipLaunchKernelGGL(k_slices, dim3((unsigned)((3LL * kTile * n + 255) / 256), p.nfr), dim3(256), 0,
-                     s, p.sys, p.types, p.s_ir, p.s_r, p.bucket_off, p.slices, p.dslices, p.bslices,
+  hipLaunchKernelGGL(k_slices<float>, dim3((unsigned)((3LL * kTile * n + 255) / 256), p.nfr),
+                     dim3(256), 0, s, p.sys, p.types, p.s_ir, p.s_r, p.bucket_off, p.slices, p.dslices, p.bslices,
                      2);
   return hipGetLastError();
 }
@@ -593,21 +603,20 @@ hipError_t launch_binning(Plan& p, hipStream_t s, bool derivs, hipStream_t aux,
                      (int)(p.spill ? p.spill_tiles : 0));
   // the corner-fold spill, staged for the deposition of this frame
   if ((e = launch_spill_stage(p, cs)) != hipSuccess) return e;
-  if (p.slice_floats > 0)
-    hipLaunchKernelGGL(k_slices, dim3((unsigned)((3LL * kTile * n + 255) / 256), nf), dim3(256), 0,
-                       s, p.sys, p.types, p.s_ir, p.s_r, p.bucket_off, p.slices, p.dslices,
-                       p.bslices, (derivs && p.dslices) ? 1 : 0);
+  const dim3 sgrid((unsigned)((3LL * kTile * n + 255) / 256), nf);
+  if (p.slice_floats > 0 && p.fft64)
+    hipLaunchKernelGGL(k_slices<double>, sgrid, dim3(256), 0, s, p.sys, p.types, p.s_ir, p.s_r,
+                       p.bucket_off, reinterpret_cast<double*>(p.slices),
+                       static_cast<double*>(nullptr), p.bslices, 0);
+  else if (p.slice_floats > 0)
+    hipLaunchKernelGGL(k_slices<float>, sgrid, dim3(256), 0, s, p.sys, p.types, p.s_ir, p.s_r,
+                       p.bucket_off, p.slices, p.dslices, p.bslices,
+                       (derivs && p.dslices) ? 1 : 0);
   // factor tables feed the FP64 gather
-  const long long total = p.fft64 ? p.table_floats : 0;
-  if (total > 0) {
-    const dim3 grid((unsigned)((total + 255) / 256), nf), block(256);
-    if (p.fft64)
-      hipLaunchKernelGGL(k_tables<double>, grid, block, 0, s, p.sys, p.types, p.s_ir, p.s_r,
-                         static_cast<double*>(p.tables), total);
-    else
-      hipLaunchKernelGGL(k_tables<float>, grid, block, 0, s, p.sys, p.types, p.s_ir, p.s_r,
-                         static_cast<float*>(p.tables), total);
-  }
+  const long long total = p.sys.f_tables;
+  if (total > 0)
+    hipLaunchKernelGGL(k_tables, dim3((unsigned)((total + 255) / 256), nf), dim3(256), 0, s, p.sys,
+                       p.types, p.s_ir, p.s_r, static_cast<double*>(p.tables), total);
   if (split && join && (e = hipStreamWaitEvent(s, p.ev_ljoin, 0)) != hipSuccess) return e;
   return hipGetLastError();
 }
