@@ -707,21 +707,59 @@ __global__ __launch_bounds__(kThreads) void k_deposit(SysDev sys, const TypeDev*
 
 // ---------------------------------------------------------------------------
 // General cell (the metric G = U U^T couples z with x or y, dens.py:301 with
-// any ucell): nothing separates, so every image is evaluated per voxel in
-// FP64, amp exp(-(b^T G b) / 2 s^2), b = r - u dr, and rounded once to the
-// plan precision.  Lane = one (x, y) column with 16 z accumulators; the
-// enumeration and visit order are the other kernels'.  Per (x, y) image pair
-// the z sources of tile cell c are u = c - N, c, c + N, except where the
-// corner slot applies (x and y off the core): for y on L the H source is
-// u = c + Nb (u >= N), for y on H the L source is u = c - Nb (u < 0).
+// any ucell): nothing separates, so every image is evaluated in FP64,
+// amp exp(-(b^T G b) / 2 s^2), b = r - u dr, and rounded once to the plan
+// precision.  Lane = one (x, y) column with 16 z accumulators; the
+// enumeration and visit order are the other kernels'.
+//
+// Column atoms: an atom off the corner regions that meets each axis of the tile
+// through one image has b_z evenly spaced along a column, so that
+//   exp(-(b^T G b) k2) = Z(z) E rho^(z - h),   k2 = 1 / 2 s^2,
+//   Z = exp(-k2 g22 b_z^2) (staged, 0 outside the window), c = 2 (g02 b_x + g12 b_y),
+//   E = exp(-k2 (g00 b_x^2 + 2 g01 b_x b_y + g11 b_y^2 + c b_z(h))), rho = exp(k2 c dr_z):
+// with the anchors h = 4 and 12, four exponentials per column instead of sixteen;
+// the powers are products outward from the anchors (at most 4 roundings; S(q) of FP64
+// plans stays as near to 64 bits as with an exponential per voxel, 4e-16).  The
+// kernel is bound by its FP64 instructions: four frames of 8,000 atoms in a
+// dodecahedral cell on a grid of 100^3 took 2,317 us in all with an exponential
+// per voxel and image and take 912 (866 with one exponential per column and the
+// cross factors of each pair of axes staged per atom, which rounds more often).
+// Types whose factors could leave FP64's range (a cell matrix far from unit edges)
+// and the atoms left over take the full evaluation per voxel and image.
+//
+// Of those, per (x, y) image pair the z sources of tile cell c are u = c - N, c,
+// c + N, except where the corner slot applies (x and y off the core): for y on L
+// the H source is u = c + Nb (u >= N), for y on H the L source is u = c - Nb (u < 0).
 struct StageGen {
   double r[NB][3];
   double amp[NB], k2[NB];  // Nel / sigma^3, 1 / (2 sigma^2)
   int lo[NB][3], len[NB][3];
+  // column atoms: the cells met along x and y, b at the cells, Z, and b_z at the
+  // tile's cells 4 and 12
+  int col[NB], xm[NB], ym[NB];
+  double bx[NB][T], by[NB][T], z[NB][T], bz[NB][2];
 };
 
+// The one image (side) through which the window [lo, lo + len) meets the tile's
+// cells [t0, t0 + tn) of an axis of N cells: its shift u - c, or kNoImage when more
+// than one does.
+constexpr int kNoImage = 1 << 30;
+__device__ __forceinline__ int one_image(int lo, int len, int t0, int tn, int N) {
+  int shift = 0, met = 0;
+#pragma unroll
+  for (int sd = -1; sd <= 1; ++sd) {
+    const int a = t0 + sd * N;
+    if (a < lo + len && lo < a + tn) {
+      ++met;
+      shift = sd * N;
+    }
+  }
+  return met <= 1 ? shift : kNoImage;
+}
+
 template <typename ACC>
-__global__ __launch_bounds__(kThreads) void k_deposit_gen(SysDev sys,
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4)))
+void k_deposit_gen(SysDev sys,
                                                           const TypeDev* __restrict__ td,
                                                           const int* __restrict__ boff,
                                                           const int4* __restrict__ s_ir,
@@ -768,11 +806,71 @@ __global__ __launch_bounds__(kThreads) void k_deposit_gen(SysDev sys,
         st.len[tid][d] = ok ? 2 * ty.half[d] : 0;
       }
       st.amp[tid] = ty.amp;
-      st.k2[tid] = 1.0 / ty.two_sig2;
+      const double k2 = 1.0 / ty.two_sig2;
+      st.k2[tid] = k2;
+      // column atom?  Its columns lie within (A + 1) dr along x and y, the tile's
+      // cells within (A + 17) dr along z
+      const double Bx = (ty.half[0] + 1) * sys.dr[0], By = (ty.half[1] + 1) * sys.dr[1],
+                   Bz = (ty.half[2] + 17) * sys.dr[2];
+      const double big = k2 * (g00 * Bx * Bx + g11 * By * By + fabs(g01x2) * Bx * By +
+                               (fabs(g02x2) * Bx + fabs(g12x2) * By) * Bz);
+      bool col = ok && !(q.w & kAtomCorner) && big < 600.0;
+#pragma unroll
+      for (int d = 0; d < 3; ++d)
+        col = col && one_image(ir[d] - ty.half[d], 2 * ty.half[d], tl.t0[d], tl.t1[d] - tl.t0[d],
+                               sys.n[d]) != kNoImage;
+      st.col[tid] = col;
+      st.xm[tid] = st.ym[tid] = 0;
+    }
+    __syncthreads();
+    // rows of the column atoms: 16 lanes per (atom, axis)
+    for (int it = tid; it < nbatch * 3 * T; it += kThreads) {
+      const int i = it % T, ad = it / T, a = ad / 3, d = ad - 3 * a;
+      if (!st.col[a]) continue;
+      const int t0 = pick3(tl.t0, d), tn = pick3(tl.t1, d) - t0, N = pick3(sys.n, d);
+      const int lo = st.lo[a][d], len = st.len[a][d];
+      const int u = t0 + i + one_image(lo, len, t0, tn, N);
+      const bool in = i < tn && u >= lo && u < lo + len;
+      const double dr = d == 0 ? sys.dr[0] : (d == 1 ? sys.dr[1] : sys.dr[2]);
+      const double bv = st.r[a][d] - (double)u * dr;
+      if (d < 2) {
+        (d == 0 ? st.bx : st.by)[a][i] = bv;
+        if (in) atomicOr(d == 0 ? &st.xm[a] : &st.ym[a], 1 << i);
+      } else {
+        st.z[a][i] = in ? exp(-(g22 * bv * bv) * st.k2[a]) : 0.0;
+        if (i == 4 || i == 12) st.bz[a][i / 8] = bv;
+      }
     }
     __syncthreads();
     if (gx < N0 && gy < N1) {
       for (int a = 0; a < nbatch; ++a) {
+        if (st.col[a]) {
+          const int xm = __builtin_amdgcn_readfirstlane(st.xm[a]);
+          const int ym = __builtin_amdgcn_readfirstlane(st.ym[a]);
+          if (((xm >> ((wave & 1) * 8)) & 0xff) == 0 || ((ym >> ((wave >> 1) * 8)) & 0xff) == 0)
+            continue;   // no column of this wave
+          if (!((xm >> ci) & 1) || !((ym >> cj) & 1)) continue;
+          const double k2 = st.k2[a], bx = st.bx[a][ci], by = st.by[a][cj];
+          const double c = g02x2 * bx + g12x2 * by;
+          const double qxy = g00 * bx * bx + g01x2 * bx * by + g11 * by * by;
+          const double lr = c * sys.dr[2] * k2;
+          const double up = exp(lr), down = exp(-lr);
+#pragma unroll
+          for (int h = 4; h < T; h += 8) {
+            const double e = st.amp[a] * exp(-(qxy + c * st.bz[a][h / 8]) * k2);
+            double gu = e, gd = e;
+            acc[h] = fma(st.z[a][h], e, acc[h]);
+#pragma unroll
+            for (int k = 1; k < 4; ++k) {
+              gu *= up;
+              gd *= down;
+              acc[h + k] = fma(st.z[a][h + k], gu, acc[h + k]);
+              acc[h - k] = fma(st.z[a][h - k], gd, acc[h - k]);
+            }
+            acc[h - 4] = fma(st.z[a][h - 4], gd * down, acc[h - 4]);
+          }
+          continue;
+        }
         const int lox = st.lo[a][0], loy = st.lo[a][1], loz = st.lo[a][2];
         const int lnx = st.len[a][0], lny = st.len[a][1], lnz = st.len[a][2];
         const double rx = st.r[a][0], ry = st.r[a][1], rz = st.r[a][2];
@@ -793,17 +891,15 @@ __global__ __launch_bounds__(kThreads) void k_deposit_gen(SysDev sys,
             // z offsets of the L and H sources (the C source is u = c)
             const int offL = (slot_rule && sy == SIDE_H) ? -nb : -N2;
             const int offH = (slot_rule && sy == SIDE_L) ? nb : N2;
+#pragma unroll 1
+            for (int j = 0; j < 3; ++j) {
+              const int off = j == 0 ? offL : (j == 1 ? 0 : offH);
 #pragma unroll
-            for (int k = 0; k < T; ++k) {
-              if (k >= nz) continue;
-              const int c = tl.t0[2] + k;
-              const int us[3] = {c + offL, c, c + offH};
-#pragma unroll
-              for (int j = 0; j < 3; ++j) {
-                const int uz = us[j];
+              for (int k = 0; k < T; ++k) {
+                const int uz = tl.t0[2] + k + off;
                 // the moved slots take only off-core sources (u < 0 / u >= N)
                 const bool side_ok = j == 1 || (j == 0 ? uz < 0 : uz >= N2);
-                if (!side_ok || uz < loz || uz >= loz + lnz) continue;
+                if (k >= nz || !side_ok || uz < loz || uz >= loz + lnz) continue;
                 const double bz = rz - (double)uz * sys.dr[2];
                 const double qv = qxy + g22 * bz * bz + cz * bz;
                 acc[k] += amp * exp(-qv * k2);
