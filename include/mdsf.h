@@ -329,6 +329,13 @@ int mdsf_rz_average(const double* d_kgridplt, int32_t nx, int32_t ny, int32_t nz
                     const double* d_zar, int32_t nzb, const double binv[9], double* d_oa,
                     mdsf_stream stream);
 
+/* What PLOT_RAD_NEW does with the averages (plot2d.py:629-637), in place on d_oa
+ * (nr, nzb): NaN bins take the smallest value, the mean divides when `normalise`,
+ * and d_final (2 nr - 1, nzb) receives the rows mirrored to negative r.  d_work:
+ * 3 nr doubles of scratch. */
+int mdsf_rz_finish(double* d_oa, int32_t nr, int32_t nzb, int32_t normalise, double* d_final,
+                   double* d_work, mdsf_stream stream);
+
 /* The same interpolant at npts points d_pts (npts, 3) -> d_out (npts), NaN
  * outside the grid (the plain-grid sections of plot2d.py:800-840). */
 int mdsf_interp_points(const double* d_kgridplt, int32_t nx, int32_t ny, int32_t nz,

@@ -990,6 +990,16 @@ int mdsf_rz_average(const double* d_kgridplt, int32_t nx, int32_t ny, int32_t nz
   return MDSF_OK;
 }
 
+int mdsf_rz_finish(double* d_oa, int32_t nr, int32_t nzb, int32_t normalise, double* d_final,
+                   double* d_work, mdsf_stream stream) {
+  if (nr < 0 || nzb < 0) return fail(MDSF_ERR_ARG, "negative bin count");
+  if ((long long)nr * nzb == 0) return MDSF_OK;
+  if (!d_oa || !d_final || !d_work) return fail(MDSF_ERR_ARG, "null array");
+  MDSF_HIP(launch_rz_finish(d_oa, nr, nzb, normalise, d_final, d_work,
+                            reinterpret_cast<hipStream_t>(stream)));
+  return MDSF_OK;
+}
+
 int mdsf_interp_points(const double* d_kgridplt, int32_t nx, int32_t ny, int32_t nz,
                        const double* d_pts, int64_t npts, double* d_out, mdsf_stream stream) {
   if (!d_kgridplt) return fail(MDSF_ERR_ARG, "null kgridplt");

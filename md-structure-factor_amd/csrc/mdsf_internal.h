@@ -395,6 +395,10 @@ hipError_t launch_ewald(const double* kp, int nx, int ny, int nz, double wl, dou
 hipError_t launch_rz_average(const double* kp, int nx, int ny, int nz, const double* rarr,
                              const int* nth, int nr, const double* zar, int nzb,
                              const double binv[9], double* oa, hipStream_t s);
+// oa (nr, nzb) finished in place, its mirrored rows in fin (2 nr - 1, nzb);
+// work: 3 nr doubles
+hipError_t launch_rz_finish(double* oa, int nr, int nzb, int normalise, double* fin, double* work,
+                            hipStream_t s);
 hipError_t launch_interp_points(const double* kp, int nx, int ny, int nz, const double* pts,
                                 long long n, double* out, hipStream_t s);
 

@@ -462,8 +462,10 @@ def rz_bins(X, Y, Z, ucell, rbins=RBINS):
     rarr = np.linspace(0.0, rmax, rbins)
     zar = np.linspace(Z[0], Z[-1], zbins)
     circ = 2. * np.pi * rarr
-    nth = np.array([max(int(THETA_BINS_PER_INV_ANG * c), MIN_THETA_BINS) for c in circ],
-                   dtype=np.int32)
+    per = THETA_BINS_PER_INV_ANG * circ
+    if per.size:
+        np.int32(int(per.max()))       # NaN and what exceeds 32 bits raise
+    nth = np.maximum(per.astype(np.int32), MIN_THETA_BINS)
     return rarr, zar, nth
 
 
@@ -500,32 +502,31 @@ def rz_average(kgridplt, ucell, format=False, rbins=RBINS):
     lib = _lib.load()
     kp = kgridplt.to(dtype=torch.float64).contiguous()
     nx, ny, nz = (int(x) for x in kp.shape[:3])
-    X = kp[:, 0, 0, 0].cpu().numpy()
-    Y = kp[0, :, 0, 1].cpu().numpy()
-    Z = kp[0, 0, :, 2].cpu().numpy()
+    axes = torch.cat([kp[:, 0, 0, 0], kp[0, :, 0, 1], kp[0, 0, :, 2]]).cpu().numpy()
+    X, Y, Z = axes[:nx], axes[nx:nx + ny], axes[nx + ny:]
     for ax in (X, Y, Z):
         if not np.all(np.diff(ax) > 0):
             raise ValueError("kgridplt axes must be strictly ascending")
     rarr, zar, nth = rz_bins(X, Y, Z, ucell, rbins)
     binv = np.ascontiguousarray(reciprocal_inverse(ucell), dtype=np.float64)
     dev = kp.device
-    d_r = torch.from_numpy(rarr).to(dev)
-    d_z = torch.from_numpy(zar).to(dev)
-    d_n = torch.from_numpy(nth).to(dev)
-    oa = torch.empty((len(rarr), len(zar)), dtype=torch.float64, device=dev)
+    nr, nzb = len(rarr), len(zar)
+    # the bins in one transfer: r, z, then the samples per r bin
+    counts = np.append(nth, np.zeros(nr % 2, dtype=np.int32)).view(np.float64)
+    bins = torch.from_numpy(np.concatenate([rarr, zar, counts])).to(dev)
+    d_r, d_z, d_n = bins.data_ptr(), bins.data_ptr() + 8 * nr, bins.data_ptr() + 8 * (nr + nzb)
+    oa = torch.empty((nr, nzb), dtype=torch.float64, device=dev)
+    final = torch.empty((max(2 * nr - 1, 0), nzb), dtype=torch.float64, device=dev)
+    work = torch.empty(3 * nr, dtype=torch.float64, device=dev)
     s = _lib.c_void_p(torch.cuda.current_stream(dev).cuda_stream)
-    _lib.check(lib.mdsf_rz_average(_lib.c_void_p(kp.data_ptr()), nx, ny, nz,
-                                   _lib.c_void_p(d_r.data_ptr()), _lib.c_void_p(d_n.data_ptr()),
-                                   len(rarr), _lib.c_void_p(d_z.data_ptr()), len(zar),
+    _lib.check(lib.mdsf_rz_average(_lib.c_void_p(kp.data_ptr()), nx, ny, nz, _lib.c_void_p(d_r),
+                                   _lib.c_void_p(d_n), nr, _lib.c_void_p(d_z), nzb,
                                    binv.ctypes.data_as(_lib.ctypes.POINTER(_lib.c_double)),
                                    _lib.c_void_p(oa.data_ptr()), s))
-    nan = torch.isnan(oa)
-    finite = oa[~nan]
-    mn = finite.min() if finite.numel() else torch.tensor(float("nan"), dtype=oa.dtype, device=dev)
-    oa = torch.where(nan, mn, oa)                                     # plot2d.py:629-630
-    if not format:
-        oa = oa / torch.mean(oa)                                      # plot2d.py:632-634
-    final = torch.cat([torch.flip(oa, [0]), oa[1:]], 0)              # plot2d.py:637
+    # NaN bins, mean, mirror: plot2d.py:629-637
+    _lib.check(lib.mdsf_rz_finish(_lib.c_void_p(oa.data_ptr()), nr, nzb, 0 if format else 1,
+                                  _lib.c_void_p(final.data_ptr()), _lib.c_void_p(work.data_ptr()),
+                                  s))
     rfin = np.append(-rarr[::-1], rarr[1:])                          # plot2d.py:638
     zfin = zar[None, :].copy()                                        # plot2d.py:639
     if format:

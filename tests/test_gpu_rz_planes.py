@@ -73,3 +73,34 @@ def test_rz_average_ring_off_the_grid_is_nan(gpu):
     torch.testing.assert_close(got[0], torch.ones(3, dtype=torch.float64, device="cuda"), rtol=1e-14,
                                atol=0)
     assert bool(torch.isnan(got[1]).all())
+
+
+@pytest.mark.parametrize("nr,nzb", [(1, 1), (1, 300), (3, 255), (257, 64), (400, 257)])
+@pytest.mark.parametrize("nans", ["none", "some", "all"])
+@pytest.mark.parametrize("normalise", [0, 1])
+def test_rz_finish(gpu, nr, nzb, nans, normalise):
+    """NaN bins, mean and mirror (plot2d.py:629-637) against torch's operations."""
+    from mdsf import _lib
+    g = torch.Generator().manual_seed(nr + nzb)
+    oa = torch.rand(nr, nzb, dtype=torch.float64, generator=g) + 0.25
+    if nans == "all":
+        oa[:] = float("nan")
+    elif nans == "some":
+        oa[torch.rand(nr, nzb, generator=g) < 0.3] = float("nan")
+    bad = torch.isnan(oa)
+    low = oa[~bad].min() if bool((~bad).any()) else torch.tensor(float("nan"), dtype=torch.float64)
+    want = torch.where(bad, low, oa)
+    if normalise:
+        want = want / want.mean()
+    d = oa.cuda()
+    fin = torch.empty(2 * nr - 1, nzb, dtype=torch.float64, device="cuda")
+    work = torch.empty(3 * nr, dtype=torch.float64, device="cuda")
+    p = _lib.c_void_p
+    _lib.check(_lib.load().mdsf_rz_finish(p(d.data_ptr()), nr, nzb, normalise, p(fin.data_ptr()),
+                                          p(work.data_ptr()),
+                                          p(torch.cuda.current_stream().cuda_stream)))
+    # the mean: sums of positive values in two orders
+    tol = 2 * (nr * nzb) ** 0.5 * 2.0 ** -53 * 8
+    torch.testing.assert_close(d.cpu(), want, rtol=tol, atol=0, equal_nan=True)
+    mirrored = torch.cat([torch.flip(d, [0]), d[1:]], 0)
+    torch.testing.assert_close(fin, mirrored, rtol=0, atol=0, equal_nan=True)
