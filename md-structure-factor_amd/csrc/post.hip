@@ -38,62 +38,69 @@ __device__ __forceinline__ double kdiv(double num, double L, int f32) {
   return num / L;
 }
 
-__global__ void k_outputs(const double* __restrict__ sf, int nx, int ny, int nz, double L0,
-                          double L1, double L2, int f32, double* __restrict__ sfplt,
-                          double* __restrict__ kgrid, double* __restrict__ kgridplt) {
+// sfplt, kgrid and kgridplt, a wave per z row.  A voxel of the 4-channel grids is two
+// lanes' 16-byte stores, so a wave stores 1 KB without gaps, and the row's two
+// coordinates are divided once per row.  Bound by the stores (927 MB at 256^3 in
+// 225 us, 4.7 TB/s with the 135 MB of reads): four 8-byte stores a thread, 32
+// bytes apart, took 286 us; these stores without the nontemporal hint, which keeps
+// them from displacing sf in the caches, 268 us (the 8-byte stores of sfplt are
+// combined in L2: with the hint 282 us).
+constexpr int kOutThreads = 256;
+typedef double out2 __attribute__((ext_vector_type(2), aligned(8)));   // caller's alignment
+
+__global__ __launch_bounds__(kOutThreads) void k_outputs(
+    const double* __restrict__ sf, int nx, int ny, int nz, double L0, double L1, double L2, int f32,
+    double* __restrict__ sfplt, double* __restrict__ kgrid, double* __restrict__ kgridplt) {
 #pragma clang fp contract(off)
-  const double twopi = 6.283185307179586;  // 2.0 * math.pi
   const double pi = 3.141592653589793;
   const int h = nz / 2 + 1;
-  const long long nkg = (long long)nx * ny * h;
   const int px = nx - 2, py = ny - 2, pz = nz - 1;
-  const long long nplt = (px > 0 && py > 0 && pz > 0) ? (long long)px * py * pz : 0;
-  const long long total = nkg > nplt ? nkg : nplt;
-  for (long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x; i < total;
-       i += (long long)gridDim.x * blockDim.x) {
-    if (kgrid && i < nkg) {
-      const int iz = (int)(i % h);
-      const int iy = (int)((i / h) % ny);
-      const int ix = (int)(i / ((long long)h * ny));
+  const long long pltrows =
+      (sfplt || kgridplt) && px > 0 && py > 0 && pz > 0 ? (long long)px * py : 0;
+  const long long rows = pltrows + (kgrid ? (long long)nx * ny : 0);
+  const int lane = threadIdx.x & 63, odd = lane & 1;
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const long long waves = (long long)gridDim.x * (kOutThreads / 64);
+  for (long long row = (long long)blockIdx.x * (kOutThreads / 64) + wave; row < rows; row += waves) {
+    if (row < pltrows) {
+      const int a = (int)(row / py), b = (int)(row - (long long)a * py);
+      const int kx = a + 1 - nx / 2, ky = b + 1 - ny / 2;
+      const double vx = kdiv(((double)a - (double)px / 2.0) * 2.0 * pi, L0, f32);
+      const double vy = kdiv(((double)b - (double)py / 2.0) * 2.0 * pi, L1, f32);
+      const double* pos = sf + ((long long)pm(kx, nx) * ny + pm(ky, ny)) * h;
+      const double* neg = sf + ((long long)pm(-kx, nx) * ny + pm(-ky, ny)) * h;
+      const long long o = row * pz;
+      for (int c = lane >> 1; c < pz; c += 32) {
+        const int kz = c + 1 - nz / 2;
+        double v = kz >= 0 ? pos[kz] : neg[-kz];
+        if (kx == 0 && ky == 0 && kz == 0) {
+          const double s100 = sf[((long long)1 * ny + 0) * h + 0];
+          const double s010 = sf[((long long)0 * ny + 1) * h + 0];
+          const double s001 = sf[((long long)0 * ny + 0) * h + 1];
+          v = 1.0 / 3.0 * (s100 + s010 + s001);
+        }
+        if (sfplt && odd) sfplt[o + c] = v;
+        if (kgridplt) {
+          const double vz = kdiv(((double)c - (double)pz / 2.0) * 2.0 * pi, L2, f32);
+          __builtin_nontemporal_store(odd ? out2{vz, v} : out2{vx, vy},
+                                      reinterpret_cast<out2*>(kgridplt) + 2 * (o + c) + odd);
+        }
+      }
+    } else {
+      const long long g = row - pltrows;
+      const int ix = (int)(g / ny), iy = (int)(g - (long long)ix * ny);
       double kx, ky;
       if (ix < nx / 2) kx = kdiv((double)ix * 2.0 * pi, L0, f32);
       else kx = kdiv(-((double)(nx - 1 - ix) + 0.5) * 2.0 * pi, L0, f32);
       if (iy < ny / 2) ky = kdiv((double)iy * 2.0 * pi, L1, f32);
       else ky = kdiv(-((double)(ny - 1 - iy) + 0.5) * 2.0 * pi, L1, f32);
-      const double kz = kdiv((double)iz * 2.0 * pi, L2, f32);
-      double* o = kgrid + 4 * i;
-      o[0] = kx;
-      o[1] = ky;
-      o[2] = kz;
-      o[3] = 0.0;
-    }
-    if (i < nplt) {
-      const int c = (int)(i % pz);
-      const int b = (int)((i / pz) % py);
-      const int a = (int)(i / ((long long)pz * py));
-      const int kx = a + 1 - nx / 2, ky = b + 1 - ny / 2, kz = c + 1 - nz / 2;
-      double v;
-      if (kx == 0 && ky == 0 && kz == 0) {
-        const double s100 = sf[((long long)1 * ny + 0) * h + 0];
-        const double s010 = sf[((long long)0 * ny + 1) * h + 0];
-        const double s001 = sf[((long long)0 * ny + 0) * h + 1];
-        v = 1.0 / 3.0 * (s100 + s010 + s001);
-      } else if (kz >= 0) {
-        v = sf[((long long)pm(kx, nx) * ny + pm(ky, ny)) * h + kz];
-      } else {
-        v = sf[((long long)pm(-kx, nx) * ny + pm(-ky, ny)) * h + (-kz)];
-      }
-      if (sfplt) sfplt[i] = v;
-      if (kgridplt) {
-        double* o = kgridplt + 4 * i;
-        o[0] = kdiv(((double)a - (double)px / 2.0) * 2.0 * pi, L0, f32);
-        o[1] = kdiv(((double)b - (double)py / 2.0) * 2.0 * pi, L1, f32);
-        o[2] = kdiv(((double)c - (double)pz / 2.0) * 2.0 * pi, L2, f32);
-        o[3] = v;
+      for (int iz = lane >> 1; iz < h; iz += 32) {
+        const double kz = kdiv((double)iz * 2.0 * pi, L2, f32);
+        __builtin_nontemporal_store(odd ? out2{kz, 0.0} : out2{kx, ky},
+                                    reinterpret_cast<out2*>(kgrid) + 2 * (g * h + iz) + odd);
       }
     }
   }
-  (void)twopi;
 }
 
 // --- Ewald sections: RegularGridInterpolator(method="linear", bounds_error=False)
@@ -220,39 +227,48 @@ __global__ void k_rz_average(const double* __restrict__ kp, int nx, int ny, int 
 //   oa[iz] = ((1 - tz) A[k] + tz A[k + 1]) / nth               (k: the cell of z)
 // with the angle, its two cells and its four weights evaluated once per (r, k)
 // instead of once per (r, z, k), and four gathers instead of eight.  One block
-// per r bin, longest rings first: the block stages kRzChunk samples' columns and
-// weights in LDS, each wave takes 64 z planes of every kRzLanes-th sample, and
-// the waves' partial sums are added in a fixed order.  Gather-bound: a wave's
-// load spans 64 z planes of the 4-channel grid, 2 KB for 512 used bytes.  The
-// plots of a 256^3 run (grids, this average, Ewald sections) took 1,185 us with
-// it against 4,481 us with k_rz_average, those of a 104 x 90 x 80 run in a 120
-// degree cell 531 against 1,455 us.
-constexpr int kRzThreads = 1024;
-constexpr int kRzChunk = 1024;          // samples staged per round
-constexpr int kRzPlanes = 256;          // z planes per round
-constexpr int kRzLanes = kRzThreads / kRzPlanes;
-constexpr int kRzMaxPlanes = 1024;      // plane sums kept in LDS (8 KB, 52 KB in all)
+// per r bin and band of z cells, longest rings first: the block stages kRzChunk
+// samples' columns and weights in LDS, its threads are (planes of the band) x
+// (lanes), a lane takes every lanes-th sample, and the lanes' partial sums are
+// added in a fixed order.
+//
+// Bound by the gathers out of L2: 8 of every 32 bytes of the 4-channel grid are
+// used.  Workgroups go round the 8 XCDs, and the band is the fastest index, so a
+// column's bytes belong to one XCD's L2, where the next rings (about three to a
+// grid cell) find them; with a block per ring over all planes each XCD fetched
+// most of the grid for itself and the longest ring set the time: 424 us at 256^3
+// with 400 rings, 282-308 us now (16 bands: 350 us, 32: 440 us, each band repeats
+// the samples' angles and cells).
+constexpr int kRzThreads = 512;
+constexpr int kRzChunk = 512;           // samples staged per round
+constexpr int kRzBands = 8;
+constexpr int kRzMaxPlanes = 1024;      // a band's planes (129 of 1024) are threads of a block
 
 __global__ __launch_bounds__(kRzThreads) void k_rz_average_sep(
     const double* __restrict__ kp, int nx, int ny, int nz, const double* __restrict__ rarr,
     const int* __restrict__ nth, int nr, const double* __restrict__ zar, int nzb, Mat3 b,
     double* __restrict__ oa) {
 #pragma clang fp contract(off)
-  extern __shared__ __align__(16) unsigned char rz_lds[];
-  double* A = reinterpret_cast<double*>(rz_lds);              // nz plane sums
-  __shared__ double red[kRzLanes][kRzPlanes];
+  __shared__ double red[kRzThreads];
   __shared__ int col[kRzChunk];                               // i * ny + j
   __shared__ double wt[kRzChunk][4];                          // weights of (0,0) (0,1) (1,0) (1,1)
   __shared__ int off_grid;
   const int tid = threadIdx.x;
-  const int ir = nr - 1 - (int)blockIdx.x;
+  const int band = (int)blockIdx.x % kRzBands;
+  const int cells = (nz - 1 + kRzBands - 1) / kRzBands;       // z cells of a band
+  const int c0 = band * cells;
+  const int np = min(cells, nz - 1 - c0) + 1;                 // planes c0 .. c0 + np - 1
+  if (np < 2 && band > 0) return;
+  const int ir = nr - 1 - (int)blockIdx.x / kRzBands;
   const double r = rarr[ir];
   const int nt = nth[ir];
   const double step = (2.0 * 3.141592653589793) / (double)nt;
   const long long sx = (long long)ny * nz * 4, sy = (long long)nz * 4;
   if (tid == 0) off_grid = 0;
-  for (int p = tid; p < nz; p += kRzThreads) A[p] = 0.0;
-  const int pl = tid % kRzPlanes, lane = tid / kRzPlanes;
+  const int lanes = kRzThreads / np;
+  const int lane = tid / np, pl = tid - lane * np;
+  const double* base = kp + 4 * (size_t)(c0 + pl) + 3;
+  double s = 0.0;
   for (int k0 = 0; k0 < nt; k0 += kRzChunk) {
     __syncthreads();
     const int kn = min(kRzChunk, nt - k0);
@@ -273,34 +289,34 @@ __global__ __launch_bounds__(kRzThreads) void k_rz_average_sep(
       wt[tid][3] = tx * ty;
     }
     __syncthreads();
-    for (int p0 = 0; p0 < nz; p0 += kRzPlanes) {
-      const int p = min(p0 + pl, nz - 1);
-      double s = 0.0;
+    if (lane < lanes) {
 #pragma unroll 4
-      for (int k = lane; k < kn; k += kRzLanes) {
-        const double* c = kp + (size_t)col[k] * (size_t)sy + 4 * (size_t)p + 3;
+      for (int k = lane; k < kn; k += lanes) {
+        const double* c = base + (size_t)col[k] * (size_t)sy;
         s = s + (wt[k][0] * c[0] + wt[k][1] * c[sy]) + (wt[k][2] * c[sx] + wt[k][3] * c[sx + sy]);
       }
-      red[lane][pl] = s;
-      __syncthreads();
-      if (tid < kRzPlanes && p0 + tid < nz) {
-        double v = red[0][tid];
-#pragma unroll
-        for (int l = 1; l < kRzLanes; ++l) v = v + red[l][tid];
-        A[p0 + tid] = A[p0 + tid] + v;
-      }
-      __syncthreads();
     }
   }
+  red[tid] = s;
+  __syncthreads();
+  if (tid < np) {
+    for (int l = 1; l < lanes; ++l) s = s + red[l * np + tid];
+  }
+  __syncthreads();
+  double* A = red;                  // the band's plane sums
+  if (tid < np) A[tid] = s;
   __syncthreads();
   const bool off = off_grid != 0;   // a sample off the grid: NaN over the ring
   for (int iz = tid; iz < nzb; iz += kRzThreads) {
     const double w = zar[iz] * b.m[8];
-    bool oob = off;
-    const int k = find_cell(kp + 2, 4, nz, w, &oob);
-    const double tz = (w - kp[2 + 4 * (size_t)k]) / (kp[2 + 4 * (size_t)(k + 1)] - kp[2 + 4 * (size_t)k]);
+    bool oob = false;
+    const int k = find_cell(kp + 2, 4, nz, w, &oob);   // 0 where w is off the grid
+    const int kb = k - c0;
+    if (kb < 0 || kb >= cells) continue;
+    const double z0 = kp[2 + 4 * (size_t)k], z1 = kp[2 + 4 * (size_t)(k + 1)];
+    const double tz = (w - z0) / (z1 - z0);
     oa[(long long)ir * nzb + iz] =
-        oob ? nan("") : (A[k] * (1.0 - tz) + A[k + 1] * tz) / (double)nt;
+        oob || off ? nan("") : (A[kb] * (1.0 - tz) + A[kb + 1] * tz) / (double)nt;
   }
 }
 
@@ -486,9 +502,11 @@ hipError_t launch_sf_read(const Plan& p, double* sf, hipStream_t s) {
 
 hipError_t launch_outputs(const int n[3], const double* sf, const double box[3], int box_f32,
                           double* sfplt, double* kgrid, double* kgridplt, hipStream_t s) {
-  const long long nkg = (long long)n[0] * n[1] * (n[2] / 2 + 1);
-  hipLaunchKernelGGL(k_outputs, dim3(grid_for(nkg)), dim3(256), 0, s, sf, n[0], n[1], n[2],
-                     box[0], box[1], box[2], box_f32, sfplt, kgrid, kgridplt);
+  const long long rows = 2LL * n[0] * n[1];
+  long long blocks = (rows + kOutThreads / 64 - 1) / (kOutThreads / 64);
+  if (blocks > 16384) blocks = 16384;
+  hipLaunchKernelGGL(k_outputs, dim3((unsigned)blocks), dim3(kOutThreads), 0, s, sf, n[0], n[1],
+                     n[2], box[0], box[1], box[2], box_f32, sfplt, kgrid, kgridplt);
   return hipGetLastError();
 }
 
@@ -509,10 +527,9 @@ hipError_t launch_rz_average(const double* kp, int nx, int ny, int nz, const dou
   // z orthogonal to x and y: the separable form (its plane sums fit LDS for
   // every grid the library plans)
   const bool sep = b.m[2] == 0.0 && b.m[5] == 0.0 && b.m[6] == 0.0 && b.m[7] == 0.0;
-  if (sep && nz <= kRzMaxPlanes && (long long)nx * ny < (1LL << 31))
-    hipLaunchKernelGGL(k_rz_average_sep, dim3((unsigned)nr), dim3(kRzThreads),
-                       (size_t)nz * sizeof(double), s, kp, nx, ny, nz, rarr, nth, nr, zar, nzb, b,
-                       oa);
+  if (sep && nz <= kRzMaxPlanes && (long long)nx * ny < (1LL << 31) && nr < (1 << 28))
+    hipLaunchKernelGGL(k_rz_average_sep, dim3((unsigned)(nr * kRzBands)), dim3(kRzThreads), 0, s,
+                       kp, nx, ny, nz, rarr, nth, nr, zar, nzb, b, oa);
   else
     hipLaunchKernelGGL(k_rz_average, dim3(grid_for((long long)nr * nzb)), dim3(256), 0, s, kp, nx,
                        ny, nz, rarr, nth, nr, zar, nzb, b, oa);

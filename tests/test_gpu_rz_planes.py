@@ -65,6 +65,12 @@ def test_rz_average_matches_pointwise_mean(gpu, n, nzb, nth, theta):
         torch.testing.assert_close(got[i, :-1], want[:-1], rtol=RTOL, atol=200 * 2.0 ** -53)
 
 
+@pytest.mark.parametrize("nz", [3, 8, 9, 10, 12, 17, 18])
+def test_rz_average_of_few_planes(gpu, nz):
+    """Bands of z cells that are empty, of one cell, or short at the end."""
+    test_rz_average_matches_pointwise_mean(gpu, (6, 7, nz), 2 * nz + 1, [1, 600, 37], 120)
+
+
 def test_rz_average_ring_off_the_grid_is_nan(gpu):
     ax = [torch.linspace(-1, 1, m, dtype=torch.float64) for m in (5, 6, 7)]
     kp = torch.stack(torch.meshgrid(*ax, indexing="ij") + (torch.ones(5, 6, 7, dtype=torch.float64),),
@@ -104,3 +110,47 @@ def test_rz_finish(gpu, nr, nzb, nans, normalise):
     torch.testing.assert_close(d.cpu(), want, rtol=tol, atol=0, equal_nan=True)
     mirrored = torch.cat([torch.flip(d, [0]), d[1:]], 0)
     torch.testing.assert_close(fin, mirrored, rtol=0, atol=0, equal_nan=True)
+
+
+@pytest.mark.parametrize("n", [(2, 4, 6), (4, 2, 6), (4, 6, 2), (6, 4, 64), (4, 4, 66), (8, 10, 130)])
+@pytest.mark.parametrize("f32", [False, True])
+def test_output_grids(gpu, n, f32):
+    """sfplt, kgrid and kgridplt (dens.py:323-344) against the oracle, each alone as well, into
+    buffers that are aligned to 8 bytes only."""
+    from mdsf import _lib, engine
+    from oracle import dens_oracle as O
+    nx, ny, nz = n
+    L = np.array([4.5, 5.25, 6.125], dtype=np.float32 if f32 else np.float64)
+    sf = np.random.default_rng(sum(n)).random((nx, ny, nz // 2 + 1)) + 0.5
+    # an axis of two points leaves no plot grid
+    splt = O.get_dplot(sf) if min(nx, ny) > 2 else np.zeros((nx - 2, ny - 2, nz - 1))
+    if nz == 2 and splt.size:
+        # the mean in the centre reads a plane that get_dplot leaves as np.empty made it
+        splt[splt.shape[0] // 2, splt.shape[1] // 2, 0] = (sf[1, 0, 0] + sf[0, 1, 0]
+                                                           + sf[0, 0, 1]) * (1.0 / 3.0)
+    kg, kgp = O.kgrids(sf.shape, L, splt)
+    plan = engine.Plan(list(n), 0, [1.0] * 3, np.eye(3), [], [], [], [])
+    p = _lib.c_void_p
+    d_sf = torch.from_numpy(sf).cuda()
+
+    def run(which):
+        sizes = [splt.size, sf.size * 4, kgp.size]
+        bufs = [torch.full((m + 2,), -7.0, dtype=torch.float64, device="cuda") for m in sizes]
+        ptr = [p(b.data_ptr() + 8) if w else p(0) for b, w in zip(bufs, which)]
+        _lib.check(_lib.load().mdsf_outputs(plan._handle, p(d_sf.data_ptr()),
+                                            _lib.doubles([float(x) for x in L]), int(f32), *ptr,
+                                            p(torch.cuda.current_stream().cuda_stream)))
+        out = [b.cpu().numpy() for b in bufs]
+        for o, m, w in zip(out, sizes, which):
+            assert o[0] == -7.0 and o[m + 1] == -7.0
+        return [o[1:-1] for o in out]
+
+    all3 = run((1, 1, 1))
+    assert np.array_equal(all3[0], splt.ravel())
+    assert np.array_equal(all3[1], kg.ravel())
+    assert np.array_equal(all3[2], kgp.ravel())
+    for k in range(3):
+        alone = run([j == k for j in range(3)])
+        for j in range(3):
+            assert np.array_equal(alone[j], all3[j] if j == k else np.full_like(all3[j], -7.0))
+    plan.close()
