@@ -334,6 +334,9 @@ struct PassArgs {
   // bytes from one frame to the next
   int nfr;
   long long res_F;
+  // log2 of the width B of the residuals' x blocks (their layout is
+  // [kz][x / B][ky][x % B]: fft.hip, res_block), 0: rows [kz][ky][x]; ny
+  int res_lb, res_ny;
 };
 
 // One Nyquist-plane pencil per block, every stage in LDS (FP64): of the block's

@@ -58,3 +58,11 @@ def test_each_length_on_each_axis(gpu, n):
 @pytest.mark.parametrize("n", [(104, 90, 80), (106, 92, 82), (30, 34, 38), (18, 250, 26)])
 def test_fp32_plans(gpu, n):
     _check(n, fp64=False)
+
+
+@pytest.mark.parametrize("nx,ny", [(16, 16), (16, 512), (512, 16), (64, 1024), (1024, 64), (32, 256),
+                                   (256, 128), (512, 512), (1024, 1024), (64, 90), (90, 64)])
+def test_residual_blocks(gpu, nx, ny):
+    """FP32 plans of power-of-two lengths pass the y pass's residuals in blocks of x: every width
+    next to lengths that keep rows."""
+    _check((nx, ny, 4), fp64=False)
