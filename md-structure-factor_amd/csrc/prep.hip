@@ -346,9 +346,10 @@ __global__ void k_tables(SysDev sys, const TypeDev* __restrict__ td, const int4*
   tables[g] = v;
 }
 
-// Tile slices for the deposition from tile lists.  16 lanes per (sorted atom, axis),
-// lane i owning cell i of every slice, so that each slice row is written as
-// one contiguous 64-byte segment.  Slice j holds cell c = 16 T + i of tile
+// Tile slices for the deposition from tile lists.  Four lanes per (sorted atom, axis),
+// each owning four adjacent cells of every slice, so that each slice row is written
+// as one contiguous segment by 16-byte stores and the atom's and type's data are
+// fetched once for four cells.  Slice j holds cell c = 16 T + i of tile
 // T = (T0 + j) mod ntiles (T0 = tile of the window start lo mod N); its value
 // is the sum over the periodic images u = c + sN (s = -1, 0, 1) inside the
 // window [lo, lo + 2A) of amp^[d==0] exp(-g_dd (r - u dr)^2 / 2 s^2): the
@@ -366,6 +367,13 @@ __global__ void k_tables(SysDev sys, const TypeDev* __restrict__ td, const int4*
 //
 // F: the plan's element type.  FP64 plans (orthogonal cells) take the exponent and
 // exp as k_tables does, without derivatives.
+//
+// Bound by the stores and by the fetches before them: 4 frames of 50,000 atoms at
+// 104 x 90 x 80 (about 115 MB) take 46 us; with a lane per cell, which fetched
+// everything sixteen times and stored 4 bytes, 86 us.
+constexpr int kSliceCells = 4;                        // cells of a lane
+constexpr int kSliceLanes = kTile / kSliceCells;      // lanes of an (atom, axis)
+
 template <typename F>
 __global__ void k_slices(SysDev sys, const TypeDev* __restrict__ td, const int4* __restrict__ s_ir,
                          const double* __restrict__ s_r, const int* __restrict__ boff,
@@ -380,7 +388,8 @@ __global__ void k_slices(SysDev sys, const TypeDev* __restrict__ td, const int4*
   dslices += fr * sys.f_slices;
   bslices += fr * sys.f_bslices;
   const long long g = blockIdx.x * (long long)blockDim.x + threadIdx.x;
-  const int pair = (int)(g / kTile), i = (int)(g - (long long)pair * kTile);
+  const int pair = (int)(g / kSliceLanes);
+  const int i = kSliceCells * (int)(g - (long long)pair * kSliceLanes);   // first cell
   const int s = pair / 3, d = pair - 3 * (pair / 3);
   if (s >= boff[sys.nbuckets]) return;
   const int4 q = s_ir[s];
@@ -391,8 +400,8 @@ __global__ void k_slices(SysDev sys, const TypeDev* __restrict__ td, const int4*
   if (slot < 0 || slot >= ty.count) return;  // only after a reported error
   const int N = d == 0 ? sys.n[0] : (d == 1 ? sys.n[1] : sys.n[2]);
   const int nt = d == 0 ? sys.ntiles[0] : (d == 1 ? sys.ntiles[1] : sys.ntiles[2]);
-  const int A = d == 0 ? ty.half[0] : (d == 1 ? ty.half[1] : ty.half[2]);
-  const int nsl = d == 0 ? ty.nsl[0] : (d == 1 ? ty.nsl[1] : ty.nsl[2]);
+  const int A = ty.half[d];
+  const int nsl = ty.nsl[d];
   const int ir = d == 0 ? q.x : (d == 1 ? q.y : q.z);
   const double dr = d == 0 ? sys.dr[0] : (d == 1 ? sys.dr[1] : sys.dr[2]);
   const double gm = d == 0 ? sys.g00 : (d == 1 ? sys.g11 : sys.g22);
@@ -424,9 +433,10 @@ __global__ void k_slices(SysDev sys, const TypeDev* __restrict__ td, const int4*
       return am * exp(-((gm * (b * b)) / ts2));
     }
   };
-  auto put = [&](long long o, F v, F dv) {
-    if (wv) slices[o] = v;
-    if (wd) dslices[o] = dv;
+  using F4 = F __attribute__((ext_vector_type(kSliceCells)));
+  auto put = [&](long long o, F4 v, F4 dv) {
+    if (wv) *reinterpret_cast<F4*>(slices + o) = v;
+    if (wd) *reinterpret_cast<F4*>(dslices + o) = dv;
   };
   // xy-coupled cells (the branch is uniform across the grid; within it only
   // the bslices store depends on the axis)
@@ -443,26 +453,58 @@ __global__ void k_slices(SysDev sys, const TypeDev* __restrict__ td, const int4*
   };
   int T = pos_mod(lo, N) / kTile;
   for (int j = 0; j < nsl; ++j) {
-    const int c = T * kTile + i;
-    const bool in = c < N;
-    F dL = 0, dC = 0, dH = 0;
-    F vL = in ? f(c - N, dL) : (F)0, vC = in ? f(c, dC) : (F)0, vH = in ? f(c + N, dH) : (F)0;
+    const int c0 = T * kTile + i;
+    F4 vL = (F4)(F)0, vC = vL, vH = vL, dL = vL, dC = vL, dH = vL;
+    // images of the four cells that the window can reach (most atoms: one)
+    const bool iL = c0 + (kSliceCells - 1) - N >= lo, iH = c0 + N < hi;
+#pragma unroll
+    for (int e = 0; e < kSliceCells; ++e) {
+      const int c = c0 + e;
+      F dv;
+      if (c < N) {
+        vC[e] = f(c, dv);
+        dC[e] = dv;
+      }
+    }
+    if (iL || iH) {
+#pragma unroll
+      for (int e = 0; e < kSliceCells; ++e) {
+        const int c = c0 + e;
+        F dv;
+        if (c < N) {
+          vL[e] = f(c - N, dv);
+          dL[e] = dv;
+          vH[e] = f(c + N, dv);
+          dH[e] = dv;
+        }
+      }
+    }
+    F4 v = vC + vL + vH;
     if (xy) {
       // at most one image in the window (the plan's condition): its b gives
       // CX (x) or BY (y); y values become log2 (then the regular value, the
       // one image's, is the largest of the three)
-      const int us = inw(c) ? c : (inw(c - N) ? c - N : c + N);
-      const bool any = in && inw(us);
-      const double bs = r - (double)us * dr;
-      if (d < 2) bslices[aoff + j * kTile] = any ? (float)(d == 0 ? cxy * bs : bs) : 0.f;
-      if (ylog) {
-        vL = in ? lg(c - N) : -__builtin_inff();
-        vC = in ? lg(c) : -__builtin_inff();
-        vH = in ? lg(c + N) : -__builtin_inff();
+      F4 bv = (F4)(F)0;
+#pragma unroll
+      for (int e = 0; e < kSliceCells; ++e) {
+        const int c = c0 + e;
+        const bool in = c < N;
+        const int us = inw(c) ? c : (inw(c - N) ? c - N : c + N);
+        const bool any = in && inw(us);
+        const double bs = r - (double)us * dr;
+        bv[e] = any ? (F)(d == 0 ? cxy * bs : bs) : (F)0;
+        if (ylog) {
+          vL[e] = in ? lg(c - N) : -__builtin_inff();
+          vC[e] = in ? lg(c) : -__builtin_inff();
+          vH[e] = in ? lg(c + N) : -__builtin_inff();
+          v[e] = (F)fmaxf(fmaxf((float)vL[e], (float)vC[e]), (float)vH[e]);
+        }
+      }
+      if constexpr (F32) {
+        if (d < 2) *reinterpret_cast<F4*>(bslices + aoff + j * kTile) = bv;
       }
     }
-    put(aoff + j * kTile, ylog ? (F)fmaxf(fmaxf((float)vL, (float)vC), (float)vH) : vC + vL + vH,
-        dC + dL + dH);
+    put(aoff + j * kTile, v, dC + dL + dH);
     if (corner) {
       // the components the corner virtual atoms take (dens.py:101-107): on z
       // the slots where the reference's corner copy lands for y on L / on H
@@ -474,10 +516,20 @@ __global__ void k_slices(SysDev sys, const TypeDev* __restrict__ td, const int4*
         put(acoff + (nsl + j) * kTile, vL, dL);
         put(acoff + (2 * nsl + j) * kTile, vH, dH);
       } else {
-        const int u1 = c + sys.nb, u2 = c - sys.nb;
-        F d1 = 0, d2 = 0;
-        const F v1 = in && u1 >= N ? f(u1, d1) : (F)0;
-        const F v2 = in && u2 < 0 ? f(u2, d2) : (F)0;
+        F4 v1 = (F4)(F)0, v2 = v1, d1 = v1, d2 = v1;
+#pragma unroll
+        for (int e = 0; e < kSliceCells; ++e) {
+          const int c = c0 + e, u1 = c + sys.nb, u2 = c - sys.nb;
+          F dv;
+          if (c < N && u1 >= N) {
+            v1[e] = f(u1, dv);
+            d1[e] = dv;
+          }
+          if (c < N && u2 < 0) {
+            v2[e] = f(u2, dv);
+            d2[e] = dv;
+          }
+        }
         put(acoff + j * kTile, vC + vL + v1, dC + dL + d1);
         put(acoff + (nsl + j) * kTile, vC + vH + v2, dC + dH + d2);
       }
@@ -546,7 +598,7 @@ hipError_t launch_rescale(void* coords, int dtype, int arith, long long nframes,
 hipError_t launch_slice_derivs(Plan& p, hipStream_t s) {
   const int n = p.sys.natoms;
   if (n == 0 || p.slice_floats == 0 || !p.dslices) return hipSuccess;
-  hipLaunchKernelGGL(k_slices<float>, dim3((unsigned)((3LL * kTile * n + 255) / 256), p.nfr),
+  hipLaunchKernelGGL(k_slices<float>, dim3((unsigned)((3LL * kSliceLanes * n + 255) / 256), p.nfr),
                      dim3(256), 0, s, p.sys, p.types, p.s_ir, p.s_r, p.bucket_off, p.slices, p.dslices, p.bslices,
                      2);
   return hipGetLastError();
@@ -603,7 +655,7 @@ hipError_t launch_binning(Plan& p, hipStream_t s, bool derivs, hipStream_t aux,
                      (int)(p.spill ? p.spill_tiles : 0));
   // the corner-fold spill, staged for the deposition of this frame
   if ((e = launch_spill_stage(p, cs)) != hipSuccess) return e;
-  const dim3 sgrid((unsigned)((3LL * kTile * n + 255) / 256), nf);
+  const dim3 sgrid((unsigned)((3LL * kSliceLanes * n + 255) / 256), nf);
   if (p.slice_floats > 0 && p.fft64)
     hipLaunchKernelGGL(k_slices<double>, sgrid, dim3(256), 0, s, p.sys, p.types, p.s_ir, p.s_r,
                        p.bucket_off, reinterpret_cast<double*>(p.slices),
