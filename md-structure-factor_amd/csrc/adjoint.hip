@@ -406,7 +406,7 @@ hipError_t launch_deposit_adjoint(Plan& p, const void* grho, const double* scale
   if (!grad_zeroed && (e = launch_fill_zero(grad, 3LL * n * p.nfr, s)) != hipSuccess) return e;
   const int* nvalid = p.bucket_off + p.sys.nbuckets;
   if (p.adj_tslots > 0 && p.adj_tpart && p.dslices) {
-    // FP32 orthogonal cells: MFMA transpose of the tiled deposition
+    // FP32 plans with tile slices: MFMA transpose of the tiled deposition
     if (!derivs_ready && (e = launch_slice_derivs(p, s)) != hipSuccess) return e;
     if ((e = launch_adjoint_tiles(p, static_cast<const float*>(grho), s)) != hipSuccess) return e;
     hipLaunchKernelGGL(k_adjoint_tile_reduce,

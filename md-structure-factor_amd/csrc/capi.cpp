@@ -34,13 +34,6 @@ namespace {
 // (each bucket is sorted by one thread to fix the gather order).
 int bucket_edge(int half) { return half < 24 ? 16 : 32; }
 
-template <typename T>
-hipError_t dalloc(T** p, size_t count) {
-  *p = nullptr;
-  if (count == 0) count = 1;
-  return hipMalloc(reinterpret_cast<void**>(p), count * sizeof(T));
-}
-
 // A plan's buffers, cut from one device allocation: a hipMalloc and a hipMemset
 // each for some 80 buffers were most of a small plan's set-up.  Buffers that start
 // at zero come first, so that one fill clears them.
@@ -117,10 +110,7 @@ void free_plan(Plan* p) {
     for (hipEvent_t e : {p->ev_prep[b], p->ev_dep[b], p->ev_fft[b]})
       if (e) (void)hipEventDestroy(e);
   for (hipEvent_t e : p->tev) (void)hipEventDestroy(e);
-  for (FrameState& f : p->slot)
-    if (f.dslices) (void)hipFree(f.dslices);
-  for (void* q : {static_cast<void*>(p->adj_part), static_cast<void*>(p->adj_w),
-                  static_cast<void*>(p->adj_tpart), p->arena})
+  for (void* q : {p->adj_arena, p->arena})
     if (q) (void)hipFree(q);
   delete p;
 }
@@ -145,15 +135,29 @@ int ensure_adjoint(Plan& p) {
   const size_t nxy = (size_t)p.sys.n[0] * p.sys.n[1];
   const size_t m = (size_t)p.sys.n[2] / 2;
   const size_t g = (size_t)p.group;
-  if (!p.adj_part) MDSF_HIP(dalloc(&p.adj_part, 3 * g * (size_t)std::max(p.adj_items, 1LL)));
-  if (!p.adj_w) MDSF_HIP(dalloc(&p.adj_w, nxy * (m + 1)));
-  if (p.adj_tslots > 0 && !p.adj_tpart) {
-    // tiled adjoint: slice derivatives per frame slot and the result slots
-    for (FrameState& f : p.slot)
-      if (!f.dslices) MDSF_HIP(dalloc(&f.dslices, g * (size_t)p.slice_floats));
-    MDSF_HIP(dalloc(&p.adj_tpart, 3 * g * (size_t)p.adj_tslots));
-    p.use_slot(p.cur_slot);
+  if (p.adj_arena) return MDSF_OK;
+  // one device allocation: the spectrum's weights, and the tiled adjoint's slice
+  // derivatives (per frame slot) and result slots or the gather's partial sums
+  auto take = [&] {
+    Arena arena;
+    arena.add(&p.adj_w, nxy * (m + 1));
+    if (p.adj_tslots > 0) {
+      for (FrameState& f : p.slot) arena.add(&f.dslices, g * (size_t)p.slice_floats);
+      arena.add(&p.adj_tpart, 3 * g * (size_t)p.adj_tslots);
+    } else {
+      arena.add(&p.adj_part, 3 * g * (size_t)p.adj_items);
+    }
+    return arena.take(&p.adj_arena);
+  };
+  hipError_t e = take();
+  if (e == hipErrorOutOfMemory && p.adj_tslots > 0 && p.sys.mode == MODE_XY) {
+    (void)hipGetLastError();   // xy-coupled cells: the gather, which needs less
+    p.adj_tslots = 0;
+    e = take();
   }
+  if (e != hipSuccess) p.adj_arena = nullptr;
+  MDSF_HIP(e);
+  p.use_slot(p.cur_slot);
   return MDSF_OK;
 }
 
@@ -353,7 +357,9 @@ int mdsf_plan_create(const mdsf_grid_desc* desc, mdsf_plan** out) {
       ty.adjt_base = slots;
       slots += (long long)ty.count * ty.nsl[0] * ty.nsl[1] * ty.nsl[2];
     }
-    p->adj_tslots = (p->slice_floats > 0 && s.mode == MODE_DIAG && !p->fft64) ? slots : 0;
+    // result slots are numbered in 32 bits where the tile lists are the source
+    const bool lists = p->tl_cap > 0 && slots < (1LL << 31);
+    if (p->slice_floats > 0 && !p->fft64 && (s.mode == MODE_DIAG || lists)) p->adj_tslots = slots;
   }
   // adjoint work items (atom, x-chunk of <= 64 planes, chunk of (y, z)
   // pairs sized for ~16k window voxels), heaviest windows numbered first so

@@ -2018,7 +2018,7 @@ void k_deposit_lists64(SysDev sys, const TypeDev* __restrict__ td, const int2* _
 }
 
 // ---------------------------------------------------------------------------
-// Adjoint of the MFMA deposition (FP32 orthogonal cells).  With G = dL/drho
+// Adjoint of the MFMA deposition (FP32 orthogonal cells; without tile lists).  With G = dL/drho
 // on the folded grid and a virtual atom's tile slices X, Y, Z and their
 // derivatives in the atom position dX, dY, dZ, the atom's gradient from one
 // tile is
@@ -2266,6 +2266,343 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4, 8))
     return nreal;
   };
   enumerate_tile(sys, td, boff, s_ir, tl, sh, NV, process);
+}
+
+// The same adjoint from the tile lists, for orthogonal and xy-coupled cells: the
+// deposition's batches (64 regular atoms, or 16 corner atoms as 64 virtual ones, four
+// lanes each, the next batch's rows fetched while this one's MFMAs run), and per wave
+// only the rows with a nonzero X on its 4 x rows.  A batch's results are summed over
+// the waves and stored in the atoms' slots.
+//
+// XY: with E = Y[y] 2^(CX[x] BY[y]) (Y itself, from dslices: the log2 that the
+// deposition takes would add its rounding error times the exponent) the lanes sum
+//   S1 = sum E dX U,  S2 = sum E X b_y U,  S3 = sum E X V,   dX = X (-2 g00 b_x / 2 s^2)
+// and the gradient is (S1 + c S2, (g01 / g00) S1 + (g11 / g01) c S2, S3) with
+// c = -2 g01 / 2 s^2.
+//
+// Quarter rows of X, dX and CX are rotated by row / 4, so that the 16 rows' quarters
+// that a wave reads at once lie in different banks.
+//
+// Bound by the matrix instructions and the fetches of the rows.  Orthogonal, 20,000
+// atoms at 128^3: 37 us a frame (k_adjoint_mfma, which enumerates its candidates and
+// contracts every row: 61).  xy-coupled, 6,000 atoms at 90 x 90 x 80: 20 us a frame,
+// the per-voxel gather 48, with the same error against FP64 (0.9e-7; 1.3e-7 with the
+// x and y sums in FP32).
+template <bool XY>
+struct StageAdjRows {
+  __align__(16) float vx[NV + 1][T];  // row NV stays zero: the lists' padding row
+  __align__(16) float vy[NV + 1][T];
+  __align__(16) float vz[NV + 1][T];
+  __align__(16) float dx[NV + 1][T];
+  __align__(16) float dz[NV + 1][T];
+  __align__(16) float dy[NV + 1][T];  // XY: BY
+  __align__(16) float cx[XY ? NV + 1 : 1][T];
+  // per-wave sums of each virtual atom
+  typename std::conditional<XY, double, float>::type red[kThreads / 64][NV][3];
+  __align__(4) unsigned char vq[NV][4];
+  unsigned char wl[kThreads / 64][NV + 16];
+  int pidx[2][NV];                    // result slot of the batch's atoms, -1: none
+  int pt[2][NV];                      // their types
+};
+
+template <int MT, bool XY>
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(XY ? 3 : 4, 8))) void k_adjoint_lists(
+    SysDev sys, const TypeDev* __restrict__ td, const int2* __restrict__ pool,
+    const int4* __restrict__ heads, const float* __restrict__ slices,
+    const float* __restrict__ bslices, const float* __restrict__ dslices,
+    const float* __restrict__ grho, double* __restrict__ tpart) {
+  __shared__ StageAdjRows<XY> st;
+  __shared__ struct {
+    int pre[MT][3], cpre[MT][3], cs[MT][3], nsl[MT][3];
+    int slice_base[MT], slice_stride[MT], corner_base[MT], corner_stride[MT], type_start[MT];
+    int part_base[MT];
+  } ty;
+  const int tid = threadIdx.x;
+  const int wave = tid >> 6, lane = tid & 63;
+  const int n16 = lane & 15, q4l = lane >> 4;
+  const int fr = blockIdx.y;   // frame of the group
+  pool += fr * (long long)sys.f_pool;
+  heads += fr * (long long)sys.f_tiles;
+  slices += fr * sys.f_slices;
+  bslices += fr * sys.f_bslices;
+  dslices += fr * sys.f_slices;
+  grho += fr * sys.f_points;
+  tpart += 3 * fr * sys.f_adjt;
+  for (int i = tid; i < sys.ntypes; i += kThreads) {
+    const TypeDev& d = td[i];
+    ty.pre[i][0] = 0;
+    ty.pre[i][1] = d.nsl[0];
+    ty.pre[i][2] = d.nsl[0] + d.nsl[1];
+    ty.cpre[i][0] = 0;
+    ty.cpre[i][1] = 2 * d.nsl[0];
+    ty.cpre[i][2] = 2 * d.nsl[0] + 3 * d.nsl[1];
+    for (int k = 0; k < 3; ++k) {
+      ty.cs[i][k] = T * d.nsl[k];
+      ty.nsl[i][k] = d.nsl[k];
+    }
+    ty.slice_base[i] = (int)d.slice_base;
+    ty.slice_stride[i] = d.slice_stride;
+    ty.corner_base[i] = (int)d.corner_base;
+    ty.corner_stride[i] = d.corner_stride;
+    ty.type_start[i] = d.type_start;
+    ty.part_base[i] = (int)d.adjt_base;
+  }
+  if (tid < T) {
+    st.vx[NV][tid] = st.vy[NV][tid] = st.vz[NV][tid] = 0.f;
+    st.dx[NV][tid] = st.dy[NV][tid] = st.dz[NV][tid] = 0.f;
+    if constexpr (XY) st.cx[NV][tid] = 0.f;
+  }
+  Tile tl;
+  tile_coords(sys, tl);
+  const int4 hd = heads[tl.idx];
+  const int base = hd.x, nreg = hd.y, ncor = hd.z, nc = hd.w;
+  if (nreg + ncor == 0) return;   // uniform over the block
+  // this wave's share of the tile, zero outside the grid
+  float g[4][4];
+  {
+    const int gy = tl.t0[1] + n16;
+#pragma unroll
+    for (int b = 0; b < 4; ++b) {
+      const int gx = tl.t0[0] + 4 * wave + b;
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        const int gz = tl.t0[2] + 4 * q4l + c;
+        g[b][c] = (gx < tl.t1[0] && gy < tl.t1[1] && gz < tl.t1[2])
+                      ? grho[((size_t)gx * sys.n[1] + gy) * sys.n[2] + gz]
+                      : 0.f;
+      }
+    }
+  }
+  __syncthreads();
+
+  const int q4 = tid & 3;
+  auto rot = [](int q, int row) { return 4 * ((q + (row >> 2)) & 3); };
+  // a virtual atom's quarter rows; offsets as in deposit_lists (-1: none)
+  struct Rows {
+    float4 x, y, z, dx, dy, dz, cx;
+  };
+  const float4 z4 = make_float4(0.f, 0.f, 0.f, 0.f);
+  auto load = [&](int o0, int o1, int o2, int ox, int oy, Rows& v) {
+    auto quarter = [&](const float* p, int o) {
+      return *reinterpret_cast<const float4*>(p + max(o, 0) + 4 * q4);
+    };
+    v.x = quarter(slices, o0);
+    v.y = quarter(XY ? dslices : slices, o1);
+    v.z = quarter(slices, o2);
+    v.dx = quarter(dslices, o0);
+    v.dz = quarter(dslices, o2);
+    if constexpr (XY) {
+      v.cx = quarter(bslices, ox);
+      v.dy = quarter(bslices, oy);
+      if (ox < 0) v.cx = z4;
+      if (oy < 0) v.dy = z4;
+    } else {
+      v.dy = quarter(dslices, o1);
+      if (o1 < 0) v.dy = z4;
+    }
+    if (o0 < 0) v.x = v.dx = z4;
+    if (o1 < 0) v.y = z4;
+    if (o2 < 0) v.z = v.dz = z4;
+  };
+  auto stage = [&](int row, const Rows& v) {
+    const int rp = rot(q4, row);
+    *reinterpret_cast<float4*>(&st.vx[row][rp]) = v.x;
+    *reinterpret_cast<float4*>(&st.dx[row][rp]) = v.dx;
+    if constexpr (XY) *reinterpret_cast<float4*>(&st.cx[row][rp]) = v.cx;
+    *reinterpret_cast<float4*>(&st.vy[row][4 * q4]) = v.y;
+    *reinterpret_cast<float4*>(&st.vz[row][4 * q4]) = v.z;
+    *reinterpret_cast<float4*>(&st.dy[row][4 * q4]) = v.dy;
+    *reinterpret_cast<float4*>(&st.dz[row][4 * q4]) = v.dz;
+    st.vq[row][q4] = (v.x.x != 0 || v.x.y != 0 || v.x.z != 0 || v.x.w != 0) ? 1 : 0;
+  };
+  // the wave's sums of staged rows [0, vtot), into st.red
+  auto contract = [&](int vtot) {
+    const bool on = lane < vtot && st.vq[lane][wave] != 0;
+    const unsigned long long bm = __ballot(on);
+    const int pos = __popcll(bm & ((1ull << lane) - 1));
+    if (on) st.wl[wave][pos] = (unsigned char)lane;
+    else st.red[wave][lane][0] = st.red[wave][lane][1] = st.red[wave][lane][2] = 0;
+    const int cnt = __popcll(bm);
+    const int kend = (cnt + 15) & ~15;
+    if (lane < 16) st.wl[wave][cnt + lane] = (unsigned char)NV;
+    __builtin_amdgcn_wave_barrier();
+    for (int k0 = 0; k0 < kend; k0 += 16) {
+      const int k = st.wl[wave][k0 + n16];
+      const float4 zf = *reinterpret_cast<const float4*>(&st.vz[k][4 * q4l]);
+      const float4 dzf = *reinterpret_cast<const float4*>(&st.dz[k][4 * q4l]);
+      const int rp = rot(wave, k);
+      const v4f xf = *reinterpret_cast<const v4f*>(&st.vx[k][rp]);
+      const v4f dxf = *reinterpret_cast<const v4f*>(&st.dx[k][rp]);
+      // U, V rows held by this lane: y = 4 (lane / 16) + r
+      const v4f yf = *reinterpret_cast<const v4f*>(&st.vy[k][4 * q4l]);
+      const v4f dyf = *reinterpret_cast<const v4f*>(&st.dy[k][4 * q4l]);
+      v4f cxf = v4f{0.f, 0.f, 0.f, 0.f};
+      if constexpr (XY) cxf = *reinterpret_cast<const v4f*>(&st.cx[k][rp]);
+      // xy-coupled cells: the contractions of x and y in FP64, as their gather's were
+      // (a third of the kernel's error in FP32, whose sums here are of differences)
+      using S = typename std::conditional<XY, double, float>::type;
+      typedef S S4 __attribute__((ext_vector_type(4)));
+      S4 w1 = S4{0, 0, 0, 0}, w2 = w1, w3 = w1;
+      S sx = 0, sy = 0, sz = 0;
+#pragma unroll
+      for (int b = 0; b < 4; ++b) {
+        v4f u = v4f{0.f, 0.f, 0.f, 0.f}, vv = u;
+        u = __builtin_amdgcn_mfma_f32_16x16x4f32(g[b][0], zf.x, u, 0, 0, 0);
+        vv = __builtin_amdgcn_mfma_f32_16x16x4f32(g[b][0], dzf.x, vv, 0, 0, 0);
+        u = __builtin_amdgcn_mfma_f32_16x16x4f32(g[b][1], zf.y, u, 0, 0, 0);
+        vv = __builtin_amdgcn_mfma_f32_16x16x4f32(g[b][1], dzf.y, vv, 0, 0, 0);
+        u = __builtin_amdgcn_mfma_f32_16x16x4f32(g[b][2], zf.z, u, 0, 0, 0);
+        vv = __builtin_amdgcn_mfma_f32_16x16x4f32(g[b][2], dzf.z, vv, 0, 0, 0);
+        u = __builtin_amdgcn_mfma_f32_16x16x4f32(g[b][3], zf.w, u, 0, 0, 0);
+        vv = __builtin_amdgcn_mfma_f32_16x16x4f32(g[b][3], dzf.w, vv, 0, 0, 0);
+        if constexpr (XY) {
+          double p1 = 0.0, p2 = 0.0, p3 = 0.0;
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            const double e = (double)(__builtin_amdgcn_exp2f(cxf[b] * dyf[r]) * yf[r]);
+            const double eu = e * (double)u[r];
+            p1 += eu;
+            p2 += eu * (double)dyf[r];
+            p3 += e * (double)vv[r];
+          }
+          sx += (double)dxf[b] * p1;
+          sy += (double)xf[b] * p2;
+          sz += (double)xf[b] * p3;
+        } else {
+          w1 += dxf[b] * u;
+          w2 += xf[b] * u;
+          w3 += xf[b] * vv;
+        }
+      }
+      if constexpr (!XY) {
+        sx = yf[0] * w1[0] + yf[1] * w1[1] + yf[2] * w1[2] + yf[3] * w1[3];
+        sy = dyf[0] * w2[0] + dyf[1] * w2[1] + dyf[2] * w2[2] + dyf[3] * w2[3];
+        sz = yf[0] * w3[0] + yf[1] * w3[1] + yf[2] * w3[2] + yf[3] * w3[3];
+      }
+      sx += __shfl_xor(sx, 16, 64);
+      sy += __shfl_xor(sy, 16, 64);
+      sz += __shfl_xor(sz, 16, 64);
+      sx += __shfl_xor(sx, 32, 64);
+      sy += __shfl_xor(sy, 32, 64);
+      sz += __shfl_xor(sz, 32, 64);
+      if (q4l == 0 && k < NV) {
+        st.red[wave][k][0] = sx;
+        st.red[wave][k][1] = sy;
+        st.red[wave][k][2] = sz;
+      }
+    }
+  };
+  // atom a's nv virtual atoms over the waves, in a fixed order, to its slot
+  auto finish = [&](int a, int vb, int nv, int buf) {
+    const int pi = st.pidx[buf][a];
+    if (pi < 0) return;
+    double s1 = 0.0, s2 = 0.0, s3 = 0.0;
+    for (int v = vb; v < vb + nv; ++v)
+#pragma unroll
+      for (int w = 0; w < kThreads / 64; ++w) {
+        s1 += (double)st.red[w][v][0];
+        s2 += (double)st.red[w][v][1];
+        s3 += (double)st.red[w][v][2];
+      }
+    double* o = tpart + 3 * (long long)pi;
+    if constexpr (XY) {
+      const double c2 = -2.0 / td[st.pt[buf][a]].two_sig2 * s2;
+      o[0] = s1 + sys.g01 * c2;
+      o[1] = sys.g01 / sys.g00 * s1 + sys.g11 * c2;
+    } else {
+      o[0] = s1;
+      o[1] = s2;
+    }
+    o[2] = s3;
+  };
+  auto slot_of = [&](int t, int slot, int j0, int j1, int j2) {
+    if (j0 == kListNoSlice || j1 == kListNoSlice || j2 == kListNoSlice) return -1;
+    return ty.part_base[t] + ((slot * ty.nsl[t][0] + j0) * ty.nsl[t][1] + j1) * ty.nsl[t][2] + j2;
+  };
+
+  // regular atoms: lanes 4a .. 4a + 3 take atom a of the batch
+  int buf = 0;
+  if (nreg > 0) {
+    const int a = tid >> 2;
+    auto fetch = [&](const int2& e, bool valid, Rows& v) {
+      const int t = (int)((unsigned)e.y >> 24);
+      const int j0 = e.y & 255, j1 = (e.y >> 8) & 255, j2 = (e.y >> 16) & 255;
+      const int o0 = valid && j0 != kListNoSlice ? e.x + T * (ty.pre[t][0] + j0) : -1;
+      const int o1 = valid && j1 != kListNoSlice ? e.x + T * (ty.pre[t][1] + j1) : -1;
+      const int o2 = valid && j2 != kListNoSlice ? e.x + T * (ty.pre[t][2] + j2) : -1;
+      load(o0, o1, o2, o0, o1, v);
+    };
+    auto place = [&](const int2& e, bool valid, int b) {
+      if (q4 != 0) return;
+      const int t = (int)((unsigned)e.y >> 24);
+      st.pt[b][a] = t;
+      st.pidx[b][a] = valid ? slot_of(t, (e.x - ty.slice_base[t]) / ty.slice_stride[t], e.y & 255,
+                                      (e.y >> 8) & 255, (e.y >> 16) & 255)
+                            : -1;
+    };
+    Rows v;
+    int2 e = a < nreg ? pool[base + a] : make_int2(0, 0), en = make_int2(0, 0);
+    fetch(e, a < nreg, v);
+    if (NV + a < nreg) en = pool[base + NV + a];
+    stage(a, v);
+    place(e, a < nreg, 0);
+    __syncthreads();
+    for (int b0 = 0; b0 < nreg; b0 += NV, buf ^= 1) {
+      const bool more = b0 + NV < nreg;
+      if (more) {   // the next batch into the registers, the entries after it
+        e = en;
+        fetch(e, b0 + NV + a < nreg, v);
+        if (b0 + 2 * NV + a < nreg) en = pool[base + b0 + 2 * NV + a];
+      }
+      contract(min(NV, nreg - b0));
+      __syncthreads();   // the rows are read, the sums complete
+      if (more) {
+        stage(a, v);
+        place(e, b0 + NV + a < nreg, buf ^ 1);
+      }
+      if (tid < NV && b0 + tid < nreg) finish(tid, tid, 1, buf);
+      __syncthreads();   // the sums are read, the next rows staged
+    }
+  }
+  // corner atoms: lanes 16 ca .. 16 ca + 15 take corner atom ca, four per virtual atom v
+  for (int c0 = 0; c0 < ncor; c0 += NV / 4) {
+    const int nca = min(NV / 4, ncor - c0);
+    const int ca = tid >> 4, v = (tid >> 2) & 3;
+    int o0 = -1, o1 = -1, o2 = -1, ox = -1, oy = -1;
+    int t = 0, pi = -1;
+    if (ca < nca) {
+      const int2 e = pool[base + nc - 1 - (c0 + ca)];
+      t = (int)((unsigned)e.y >> 24);
+      const int slot = e.x - ty.type_start[t];
+      const int ab = ty.slice_base[t] + slot * ty.slice_stride[t];
+      const int cb = ty.corner_base[t] + slot * ty.corner_stride[t];
+      const int j0 = e.y & 255, j1 = (e.y >> 8) & 255, j2 = (e.y >> 16) & 255;
+      const int so0 = j0 != kListNoSlice ? ab + T * (ty.pre[t][0] + j0) : -1;
+      const int so1 = j1 != kListNoSlice ? ab + T * (ty.pre[t][1] + j1) : -1;
+      const int so2 = j2 != kListNoSlice ? ab + T * (ty.pre[t][2] + j2) : -1;
+      const int cb0 = j0 != kListNoSlice ? cb + T * (ty.cpre[t][0] + j0) : -1;
+      const int cb1 = j1 != kListNoSlice ? cb + T * (ty.cpre[t][1] + j1) : -1;
+      const int cb2 = j2 != kListNoSlice ? cb + T * (ty.cpre[t][2] + j2) : -1;
+      o0 = cb0 >= 0 ? cb0 + (v == 0 ? 0 : ty.cs[t][0]) : -1;
+      o1 = v == 0 ? so1 : (cb1 >= 0 ? cb1 + (v - 1) * ty.cs[t][1] : -1);
+      o2 = v < 2 ? so2 : (cb2 >= 0 ? cb2 + (v - 2) * ty.cs[t][2] : -1);
+      ox = so0;
+      oy = so1;
+      pi = slot_of(t, slot, j0, j1, j2);
+    }
+    Rows w;
+    load(o0, o1, o2, ox, oy, w);
+    stage(tid >> 2, w);   // row 4 ca + v
+    if ((tid & 15) == 0) {
+      st.pidx[0][ca] = pi;
+      st.pt[0][ca] = t;
+    }
+    __syncthreads();
+    contract(4 * nca);
+    __syncthreads();
+    if (tid < nca) finish(tid, 4 * tid, 4, 0);
+    __syncthreads();
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -2659,6 +2996,14 @@ hipError_t launch_adjoint_tiles(Plan& p, const float* grho, hipStream_t s) {
   const long long ntiles = (long long)sys.ntiles[0] * sys.ntiles[1] * sys.ntiles[2];
   if (ntiles == 0) return hipSuccess;
   const dim3 grid((unsigned)ntiles, p.nfr), block(kThreads);
+  if (p.tl_cap > 0 && p.adj_tslots < (1LL << 31)) {
+    auto k = sys.mode == MODE_XY
+                 ? (sys.ntypes <= 16 ? k_adjoint_lists<16, true> : k_adjoint_lists<kMaxTypes, true>)
+                 : (sys.ntypes <= 16 ? k_adjoint_lists<16, false> : k_adjoint_lists<kMaxTypes, false>);
+    hipLaunchKernelGGL(k, grid, block, 0, s, sys, p.types, p.tl_pool, p.tl_head, p.slices,
+                       p.bslices, p.dslices, grho, p.adj_tpart);
+    return hipGetLastError();
+  }
   if (sys.ntypes <= 16)
     hipLaunchKernelGGL(k_adjoint_mfma<16>, grid, block, 0, s, sys, p.types, p.bucket_off, p.s_ir,
                        p.slices, p.dslices, grho, p.adj_tpart);

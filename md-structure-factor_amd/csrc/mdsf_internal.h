@@ -86,7 +86,7 @@ struct TypeDev {
   int adj_ppi;
   int adj_npc;
   long long adj_item_base;
-  // tiled adjoint (FP32 DIAG): one result slot of 3 FP64 per (atom, tile
+  // tiled adjoint (FP32 plans): one result slot of 3 FP64 per (atom, tile
   // slice triple j0, j1, j2), nsl[0] nsl[1] nsl[2] per atom, from adjt_base
   long long adjt_base;
 };
@@ -292,6 +292,7 @@ struct Plan {
   hipEvent_t ev_prep[kSlots] = {}, ev_dep[kSlots] = {}, ev_fft[kSlots] = {};
   // adjoint (allocated on first use)
   long long adj_items = 0;
+  void* adj_arena = nullptr;     // the adjoint's buffers (ensure_adjoint)
   double* adj_part = nullptr;    // 3 FP64 partial sums per work item
   long long adj_tslots = 0;      // tiled adjoint result slots
   double* adj_tpart = nullptr;   // 3 FP64 per slot

@@ -363,7 +363,7 @@ __global__ void k_tables(SysDev sys, const TypeDev* __restrict__ td, const int4*
 // and corner components) LY = log2 of the y factor (-inf outside the window)
 // instead of the factor; bslices holds CX = -2 g01 log2(e) / 2 s^2 b_x at the
 // regular x slice cells and BY = b_y at the regular y slice cells (0 outside
-// the window).
+// the window).  dslices holds the y factor itself in the y slices.
 //
 // F: the plan's element type.  FP64 plans (orthogonal cells) take the exponent and
 // exp as k_tables does, without derivatives.
@@ -419,6 +419,7 @@ __global__ void k_slices(SysDev sys, const TypeDev* __restrict__ td, const int4*
   const long long acoff = ty.corner_base + (long long)slot * ty.corner_stride + coff_d + i;
   // mode 0: slices, 1: slices and derivatives, 2: derivatives only
   const bool wv = mode != 2, wd = F32 && mode != 0;
+  const bool xyd = wd && sys.mode == MODE_XY;
   // factor of the image at grid coordinate u, 0 outside the window, and its
   // derivative in r: am exp(-gk b^2) and am exp(-gk b^2) (-2 gk b), b = r - u dr
   auto f = [&](int u, F& df) -> F {
@@ -427,7 +428,9 @@ __global__ void k_slices(SysDev sys, const TypeDev* __restrict__ td, const int4*
     const double b = r - (double)u * dr;
     if constexpr (F32) {
       const float v = am * expf(-(float)(gk * (b * b)));
-      df = v * (float)(-2.0 * gk * b);
+      // xy-coupled cells: rounded once, as their gather's factors are
+      if (xyd) df = (float)((double)am * exp(-(gk * (b * b))) * (-2.0 * gk * b));
+      else df = v * (float)(-2.0 * gk * b);
       return v;
     } else {
       return am * exp(-((gm * (b * b)) / ts2));
@@ -494,6 +497,9 @@ __global__ void k_slices(SysDev sys, const TypeDev* __restrict__ td, const int4*
         const double bs = r - (double)us * dr;
         bv[e] = any ? (F)(d == 0 ? cxy * bs : bs) : (F)0;
         if (ylog) {
+          dL[e] = vL[e];
+          dC[e] = vC[e];
+          dH[e] = vH[e];
           vL[e] = in ? lg(c - N) : -__builtin_inff();
           vC[e] = in ? lg(c) : -__builtin_inff();
           vH[e] = in ? lg(c + N) : -__builtin_inff();
