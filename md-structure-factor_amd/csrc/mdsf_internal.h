@@ -193,8 +193,8 @@ struct Plan {
   // binning
   int* bucket_count = nullptr;
   int* bucket_off = nullptr;
-  int* bucket_cur = nullptr;
-  int* bucket_aux = nullptr;     // per-1024-block totals of the bucket scan
+  int* bucket_cur = nullptr;     // offsets within the bucket scan's blocks
+  int* bucket_aux = nullptr;     // totals of the bucket scan's blocks
   int* s_tmp = nullptr;          // bucket fill (arbitrary order within a bucket)
   int* s_idx = nullptr;          // atom indices sorted by (type, bucket, index)
   int4* s_ir = nullptr;

@@ -30,8 +30,8 @@ __global__ void k_prep(T* __restrict__ coords, SysDev sys, const TypeDev* __rest
                        const int32_t* __restrict__ types, const double* __restrict__ scale,
                        double L0, double L1, double L2, long long wlo, long long whi,
                        int4* __restrict__ ir4, int* __restrict__ key, double* __restrict__ rpos,
-                       int* __restrict__ bcount, unsigned* __restrict__ occ,
-                       int* __restrict__ home, int* __restrict__ err, int coords_only,
+                       int* __restrict__ bcount, int* __restrict__ pos,
+                       unsigned* __restrict__ occ, int* __restrict__ home, int* __restrict__ err, int coords_only,
                        int write_back, int home_frame) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= sys.natoms) return;
@@ -42,6 +42,7 @@ __global__ void k_prep(T* __restrict__ coords, SysDev sys, const TypeDev* __rest
   key += fr * sys.f_atoms();
   rpos += 3 * fr * sys.f_atoms();
   bcount += fr * sys.f_buckets();
+  pos += fr * sys.f_atoms();
   if (fr != home_frame) home = nullptr;
   T x[3];
   x[0] = coords[3 * (size_t)i + 0];
@@ -114,14 +115,17 @@ __global__ void k_prep(T* __restrict__ coords, SysDev sys, const TypeDev* __rest
   rpos[3 * (size_t)i + 0] = (double)x[0];
   rpos[3 * (size_t)i + 1] = (double)x[1];
   rpos[3 * (size_t)i + 2] = (double)x[2];
-  atomicAdd(&bcount[b], 1);
+  // the atom's place in its bucket, in the order the atomics arrive in
+  pos[i] = atomicAdd(&bcount[b], 1);
   if (occ && finite) atomicAdd(&occ[((size_t)h[0] * sys.n[1] + h[1]) * sys.n[2] + h[2]], 1u);
 }
 
-// Exclusive scan of the bucket counts in two coalesced passes: per-block
-// scans (k_scan_blocks), then block offsets (k_scan_add).  The counts are
-// cleared for the next frame and the fill cursors seeded.
+// Exclusive scan of the bucket counts: offsets within blocks of kScanItems buckets
+// and the blocks' totals (k_scan_blocks); k_fill adds the totals before a block as it
+// places the atoms and writes the offsets.
 constexpr int kScanThreads = 1024;
+constexpr int kScanPer = 8;                            // buckets of a thread
+constexpr int kScanItems = kScanPer * kScanThreads;
 
 __device__ __forceinline__ int block_excl_scan(int v, int* wsum, int* total) {
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -146,64 +150,71 @@ __device__ __forceinline__ int block_excl_scan(int v, int* wsum, int* total) {
 // clear: zero the counts for the slot's next frame (plans with tile lists
 // leave them to k_tile_lists, after k_tile_count has read them)
 __global__ __launch_bounds__(kScanThreads) void k_scan_blocks(int* __restrict__ bcount,
-                                                              int* __restrict__ boff,
+                                                              int* __restrict__ loc,
                                                               int* __restrict__ aux, int nbk,
-                                                              int clear, int naux) {
+                                                              int clear, int naux,
+                                                              int* __restrict__ corners) {
   __shared__ int wsum[kScanThreads / 64];
   bcount += blockIdx.y * (nbk + 1LL);
-  boff += blockIdx.y * (nbk + 1LL);
+  loc += blockIdx.y * (nbk + 1LL);
   aux += blockIdx.y * naux;
-  const int i = blockIdx.x * kScanThreads + threadIdx.x;
-  const int v = i < nbk ? bcount[i] : 0;
+  if (blockIdx.x == 0 && threadIdx.x == 0) corners[blockIdx.y * kCornerInts] = 0;  // k_rank_gather
+  const int i = blockIdx.x * kScanItems + kScanPer * threadIdx.x;
+  int v[kScanPer], sum = 0;
+#pragma unroll
+  for (int k = 0; k < kScanPer; ++k) {
+    v[k] = i + k < nbk ? bcount[i + k] : 0;
+    sum += v[k];
+  }
   int total;
-  const int ex = block_excl_scan(v, wsum, &total);
-  if (i < nbk) {
-    boff[i] = ex;
-    if (clear) bcount[i] = 0;
+  int ex = block_excl_scan(sum, wsum, &total);
+#pragma unroll
+  for (int k = 0; k < kScanPer; ++k) {
+    if (i + k < nbk) {
+      loc[i + k] = ex;
+      if (clear) bcount[i + k] = 0;
+    }
+    ex += v[k];
   }
   if (threadIdx.x == 0) aux[blockIdx.x] = total;
 }
 
-__global__ __launch_bounds__(kScanThreads) void k_scan_add(int* __restrict__ boff,
-                                                           int* __restrict__ bcur,
-                                                           const int* __restrict__ aux, int nbk,
-                                                           int nblocks, int* __restrict__ corners,
-                                                           int naux) {
-  __shared__ int base_sh;
-  boff += blockIdx.y * (nbk + 1LL);
-  bcur += blockIdx.y * (nbk + 1LL);
-  aux += blockIdx.y * naux;
-  corners += blockIdx.y * kCornerInts;
-  if (blockIdx.x == 0 && threadIdx.x == 0) corners[0] = 0;  // refilled by k_rank_gather
-  if (threadIdx.x < 64) {
-    int s = 0;
-    for (int b = threadIdx.x; b < (int)blockIdx.x; b += 64) s += aux[b];
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) s += __shfl_down(s, o, 64);
-    if (threadIdx.x == 0) base_sh = s;
-  }
-  __syncthreads();
-  const int base = base_sh;
-  const int i = blockIdx.x * kScanThreads + threadIdx.x;
-  if (i < nbk) {
-    const int v = boff[i] + base;
-    boff[i] = v;
-    bcur[i] = v;
-  }
-  if (blockIdx.x == nblocks - 1 && threadIdx.x == 0) boff[nbk] = base + aux[blockIdx.x];
-}
-
-__global__ void k_fill(const int* __restrict__ key, int* __restrict__ bcur,
-                       int* __restrict__ s_tmp, int natoms, int nbk) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= natoms) return;
+// Atoms to their buckets (in k_prep's arrival order) and the buckets' offsets, a
+// thread for both.  Bound by the scattered stores: 22 us for a million atoms.  With
+// cursors of its own, advanced by atomics, it took 83 us, and a pass before it wrote
+// the offsets and the cursors.
+constexpr int kFillThreads = 256;
+__global__ __launch_bounds__(kFillThreads) void k_fill(const int* __restrict__ key,
+                                                       const int* __restrict__ pos,
+                                                       const int* __restrict__ loc,
+                                                       const int* __restrict__ aux,
+                                                       int* __restrict__ boff,
+                                                       int* __restrict__ s_tmp, int natoms, int nbk,
+                                                       int nblocks, int naux) {
+  extern __shared__ int pre[];   // totals of the blocks before each block
+  __shared__ int wsum[kFillThreads / 64];
+  const int tid = threadIdx.x;
   key += blockIdx.y * (long long)natoms;
+  pos += blockIdx.y * (long long)natoms;
   s_tmp += blockIdx.y * (long long)natoms;
-  bcur += blockIdx.y * (nbk + 1LL);
+  loc += blockIdx.y * (nbk + 1LL);
+  boff += blockIdx.y * (nbk + 1LL);
+  aux += blockIdx.y * naux;
+  int total = 0;
+  for (int b0 = 0; b0 < nblocks; b0 += kFillThreads) {   // uniform over the block
+    const int b = b0 + tid;
+    int t;
+    const int ex = block_excl_scan(b < nblocks ? aux[b] : 0, wsum, &t);
+    if (b < nblocks) pre[b] = total + ex;
+    total += t;
+    __syncthreads();
+  }
+  const int i = blockIdx.x * kFillThreads + tid;
+  if (i <= nbk) boff[i] = i < nbk ? loc[i] + pre[i / kScanItems] : total;
+  if (i >= natoms) return;
   const int b = key[i];
   if (b < 0) return;
-  const int pos = atomicAdd(&bcur[b], 1);
-  s_tmp[pos] = i;
+  s_tmp[loc[b] + pre[b / kScanItems] + pos[i]] = i;
 }
 
 // Restores atom-index order inside each bucket, so that the gather visits
@@ -558,18 +569,18 @@ hipError_t launch_prep(Plan& p, void* coords, int dtype, int arith, const int32_
   if (dtype == MDSF_F32 && arith == MDSF_F32) {
     hipLaunchKernelGGL((k_prep<float, float>), grid, block, 0, s, (float*)coords, p.sys, p.types,
                        types, scale3, box[0], box[1], box[2], (long long)wrap_lo,
-                       (long long)wrap_hi, p.ir4, p.key, p.rpos, p.bucket_count, occ, home, p.err, co, wb,
-                       home_frame);
+                       (long long)wrap_hi, p.ir4, p.key, p.rpos, p.bucket_count, p.s_idx, occ, home, p.err,
+                       co, wb, home_frame);
   } else if (dtype == MDSF_F32) {
     hipLaunchKernelGGL((k_prep<float, double>), grid, block, 0, s, (float*)coords, p.sys, p.types,
                        types, scale3, box[0], box[1], box[2], (long long)wrap_lo,
-                       (long long)wrap_hi, p.ir4, p.key, p.rpos, p.bucket_count, occ, home, p.err, co, wb,
-                       home_frame);
+                       (long long)wrap_hi, p.ir4, p.key, p.rpos, p.bucket_count, p.s_idx, occ, home, p.err,
+                       co, wb, home_frame);
   } else {
     hipLaunchKernelGGL((k_prep<double, double>), grid, block, 0, s, (double*)coords, p.sys,
                        p.types, types, scale3, box[0], box[1], box[2], (long long)wrap_lo,
-                       (long long)wrap_hi, p.ir4, p.key, p.rpos, p.bucket_count, occ, home, p.err, co, wb,
-                       home_frame);
+                       (long long)wrap_hi, p.ir4, p.key, p.rpos, p.bucket_count, p.s_idx, occ, home, p.err,
+                       co, wb, home_frame);
   }
   return hipGetLastError();
 }
@@ -587,16 +598,16 @@ hipError_t launch_rescale(void* coords, int dtype, int arith, long long nframes,
     if (dtype == MDSF_F32 && arith == MDSF_F32)
       hipLaunchKernelGGL((k_prep<float, float>), grid, block, 0, s, (float*)coords + t * fstride,
                          sys, nullptr, nullptr, scale + 3 * t, 0.0, 0.0, 0.0, 0LL, 0LL, nullptr,
-                         nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, 1, 1, 0);
+                         nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, 1, 1, 0);
     else if (dtype == MDSF_F32)
       hipLaunchKernelGGL((k_prep<float, double>), grid, block, 0, s, (float*)coords + t * fstride,
                          sys, nullptr, nullptr, scale + 3 * t, 0.0, 0.0, 0.0, 0LL, 0LL, nullptr,
-                         nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, 1, 1, 0);
+                         nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, 1, 1, 0);
     else
       hipLaunchKernelGGL((k_prep<double, double>), grid, block, 0, s,
                          (double*)coords + t * fstride, sys, nullptr, nullptr, scale + 3 * t, 0.0,
                          0.0, 0.0, 0LL, 0LL, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr,
-                         nullptr, 1, 1, 0);
+                         nullptr, nullptr, 1, 1, 0);
   }
   return hipGetLastError();
 }
@@ -614,7 +625,7 @@ hipError_t launch_binning(Plan& p, hipStream_t s, bool derivs, hipStream_t aux,
                           hipStream_t side, bool join, hipEvent_t aux_end) {
   const int n = p.sys.natoms;
   const int nbk = p.sys.nbuckets;
-  const int nblk = (nbk + kScanThreads - 1) / kScanThreads;
+  const int nblk = (nbk + kScanItems - 1) / kScanItems;
   if (nblk == 0) return hipSuccess;
   // Branches (when the streams are given): the tile lists on `aux` (their
   // regions need only the bucket counts, from here on; their entries the
@@ -632,12 +643,11 @@ hipError_t launch_binning(Plan& p, hipStream_t s, bool derivs, hipStream_t aux,
   }
   const unsigned nf = (unsigned)p.nfr;
   hipLaunchKernelGGL(k_scan_blocks, dim3(nblk, nf), dim3(kScanThreads), 0, s, p.bucket_count,
-                     p.bucket_off, p.bucket_aux, nbk, lists ? 0 : 1, p.sys.f_aux);
-  hipLaunchKernelGGL(k_scan_add, dim3(nblk, nf), dim3(kScanThreads), 0, s, p.bucket_off,
-                     p.bucket_cur, p.bucket_aux, nbk, nblk, p.corners, p.sys.f_aux);
+                     p.bucket_cur, p.bucket_aux, nbk, lists ? 0 : 1, p.sys.f_aux, p.corners);
+  hipLaunchKernelGGL(k_fill, dim3(std::max(n, nbk + 1) / kFillThreads + 1, nf), dim3(kFillThreads),
+                     (size_t)nblk * sizeof(int), s, p.key, p.s_idx, p.bucket_cur, p.bucket_aux,
+                     p.bucket_off, p.s_tmp, n, nbk, nblk, p.sys.f_aux);
   if (n == 0) return hipGetLastError();
-  hipLaunchKernelGGL(k_fill, dim3((n + 255) / 256, nf), dim3(256), 0, s, p.key, p.bucket_cur,
-                     p.s_tmp, n, nbk);
   hipLaunchKernelGGL(k_rank_gather, dim3((n + 255) / 256, nf), dim3(256), 0, s, p.key,
                      p.bucket_off, p.s_tmp, p.s_idx, p.ir4, p.rpos, p.s_ir, p.s_r, n, nbk,
                      p.corners);
