@@ -20,7 +20,9 @@ constexpr int kMaxSpillBufTiles = 4096;  // spill tiles staged per frame slot (e
 constexpr int kCornerCap = 512;     // corner atoms listed per frame for the spill pass
 constexpr int kCornerInts = 2 + 2 * kCornerCap;  // the list's ints per frame (FrameState::corners)
 constexpr int kListNoSlice = 255;  // tile-list entry: no slice on that axis (a byte per axis)
-constexpr long long kSplitPrepTiles = 2048;  // tiles from which the frame loop splits its prepare stage
+// tiles, or atoms of a group, from which the frame loop splits its prepare stage (split_prep)
+constexpr long long kSplitPrepTiles = 2048;
+constexpr long long kSplitPrepAtoms = 65536;
 // stage-timing events per frame: prepare start / end (caller's stream), the
 // deposition kernel's begin / end, the three FFT passes' begin / end, and the
 // end of the prepare stage's tile-list branch
