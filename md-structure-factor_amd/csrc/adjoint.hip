@@ -363,9 +363,11 @@ __global__ void k_adjoint_tile_reduce(SysDev sys, const TypeDev* __restrict__ td
   }
 }
 
-__global__ void k_fill_zero(double* __restrict__ p, long long n) {
+__global__ void k_fill_zero(double* __restrict__ p, long long n, double* __restrict__ q,
+                            long long m) {
   const long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x;
   if (i < n) p[i] = 0.0;
+  else if (i - n < m) q[i - n] = 0.0;
 }
 
 // w_main[kz][y][x] = 2 g[x, y, kz] (kz < m), w_nyq[x][y] = 2 g[x, y, m]: the
@@ -383,9 +385,10 @@ __global__ __launch_bounds__(kHalfThreads) void k_adjoint_weights(const double* 
 
 }  // namespace
 
-hipError_t launch_fill_zero(double* p, long long n, hipStream_t s) {
-  if (n <= 0) return hipSuccess;
-  hipLaunchKernelGGL(k_fill_zero, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, p, n);
+hipError_t launch_fill_zero(double* p, long long n, hipStream_t s, double* q, long long m) {
+  if (n + m <= 0) return hipSuccess;
+  hipLaunchKernelGGL(k_fill_zero, dim3((unsigned)((n + m + 255) / 256)), dim3(256), 0, s, p, n, q,
+                     m);
   return hipGetLastError();
 }
 

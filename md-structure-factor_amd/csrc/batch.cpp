@@ -68,8 +68,7 @@ hipError_t enqueue_system(Batch& b, int i, hipStream_t s) {
   Plan& p = *reinterpret_cast<Plan*>(b.plans[i]);
   const SysFrames& f = b.frames[i];
   const long long nxy = (long long)p.sys.n[0] * p.sys.n[1];
-  hipError_t e = launch_fill_zero(p.sf_main, nxy * (p.sys.n[2] / 2), s);
-  if (e == hipSuccess) e = launch_fill_zero(p.sf_nyq, nxy, s);
+  hipError_t e = launch_fill_zero(p.sf_main, nxy * (p.sys.n[2] / 2), s, p.sf_nyq, nxy);
   const size_t esz = f.dtype == MDSF_F32 ? 4 : 8;
   const size_t fstride = (size_t)p.sys.natoms * 3 * esz;
   const int64_t ngroups = (f.nframes + p.group - 1) / p.group;

@@ -104,7 +104,7 @@ hipError_t pipeline_streams(int device, hipStream_t* dep, hipStream_t* fft, hipS
 
 void free_plan(Plan* p) {
   if (!p) return;
-  for (hipEvent_t e : {p->ev_fork, p->ev_lfork, p->ev_lgath, p->ev_ljoin})
+  for (hipEvent_t e : {p->ev_fork, p->ev_done, p->ev_lfork, p->ev_lgath, p->ev_ljoin})
     if (e) (void)hipEventDestroy(e);
   for (int b = 0; b < kSlots; ++b)
     for (hipEvent_t e : {p->ev_prep[b], p->ev_dep[b], p->ev_fft[b]})
@@ -127,11 +127,30 @@ int make_axis(FftAxis& ax, int n, Arena& arena) {
 // The prepare stage's branches go on their own streams on large grids and for groups of
 // many atoms; with less work the cross-stream waits (about 10 us each) cost more than
 // the branches overlap.  16 frames of 50,000 atoms at 104 x 90 x 80 in groups of 4: 1,443
-// us without the split, 1,405 with; 10 frames of 2,700 at 64^3 gain nothing.
+// us without the split, 1,405 with.  One group alone, which without the split needs no
+// waits at all, splits at four times the atoms: one of 80,000 at 128^3 takes 366 us in
+// one stream, 409 split; a million atoms at 512^3 are split by their tiles.
 bool split_prep(const Plan& p, int64_t nframes) {
   const long long ntiles = (long long)p.sys.ntiles[0] * p.sys.ntiles[1] * p.sys.ntiles[2];
+  const long long least = (nframes <= p.group ? 4 : 1) * kSplitPrepAtoms;
   return ntiles >= kSplitPrepTiles ||
-         p.sys.natoms * (long long)std::min<int64_t>(p.group, nframes) >= kSplitPrepAtoms;
+         p.sys.natoms * (long long)std::min<int64_t>(p.group, nframes) >= least;
+}
+
+// Is `s` being captured into a graph?  Then a frame loop neither waits for earlier calls
+// nor leaves work that later calls would wait for (its event would be the graph's).
+bool capturing(hipStream_t s) {
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(s, &st) != hipSuccess) {
+    (void)hipGetLastError();
+    return true;
+  }
+  return st != hipStreamCaptureStatusNone;
+}
+
+// `to` waits for the event, unless it is the stream that recorded it.
+hipError_t wait_for(hipStream_t to, hipEvent_t ev, hipStream_t from) {
+  return to == from ? hipSuccess : hipStreamWaitEvent(to, ev, 0);
 }
 
 // Sets the frames the plan's launches cover, and one again when it goes.
@@ -505,7 +524,8 @@ int mdsf_plan_create(const mdsf_grid_desc* desc, mdsf_plan** out) {
     return rc;
   }
   e = pipeline_streams(p->device, &p->dep_stream, &p->fft_stream, &p->aux_stream);
-  for (hipEvent_t* ev : {&p->ev_fork, &p->ev_lfork, &p->ev_lgath, &p->ev_ljoin})
+  for (hipEvent_t* ev : {&p->ev_fork, &p->ev_done, &p->ev_lfork, &p->ev_lgath,
+                         &p->ev_ljoin})
     if (e == hipSuccess) e = hipEventCreateWithFlags(ev, hipEventDisableTiming);
   for (int b = 0; b < kSlots && e == hipSuccess; ++b)
     for (hipEvent_t* ev : {&p->ev_prep[b], &p->ev_dep[b], &p->ev_fft[b]})
@@ -543,8 +563,7 @@ int mdsf_sf_reset(mdsf_plan* plan, mdsf_stream stream) {
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   const long long nxy = (long long)p->sys.n[0] * p->sys.n[1];
   // a fill kernel rather than a memset node keeps this capturable in graphs
-  MDSF_HIP(launch_fill_zero(p->sf_main, nxy * (p->sys.n[2] / 2), s));
-  MDSF_HIP(launch_fill_zero(p->sf_nyq, nxy, s));
+  MDSF_HIP(launch_fill_zero(p->sf_main, nxy * (p->sys.n[2] / 2), s, p->sf_nyq, nxy));
   return MDSF_OK;
 }
 
@@ -590,12 +609,17 @@ int mdsf_accumulate_frames(mdsf_plan* plan, void* d_coords, int dtype, int64_t n
   // wait for the FFT of the group just before the previous one (the FFT
   // shares the GPU with the deposition and finishes later than it).  The
   // S(q) sum stays in frame order on one stream.
-  hipStream_t d = p->dep_stream, f = p->fft_stream;
   FrameGroup group(*p);
   const int64_t ngroups = (nframes + p->group - 1) / p->group;
+  // One group has nothing to overlap with: its stages stay on `s` (dep_stream where
+  // the prepare stage splits), which saves the waits from stream to stream.  The
+  // slots are then not ordered by the shared streams, so calls wait for the plan's
+  // previous one.
+  const bool split = split_prep(*p, nframes);
+  const bool cap = capturing(s), one = ngroups == 1 && !cap;
+  hipStream_t d = one && !split ? s : p->dep_stream, f = one ? d : p->fft_stream;
   // groups of nearly equal size
   auto first_of = [&](int64_t k) { return k * (nframes / ngroups) + std::min(k, nframes % ngroups); };
-  const bool split = split_prep(*p, nframes);
   const bool pair = nframes >= 2 && fft_x_pairs(*p);   // plans with one frame per group
   // timed groups accumulate over calls until mdsf_stage_times reads them
   // (group k of this call is timed group tb + k), so that one-frame calls
@@ -618,10 +642,13 @@ int mdsf_accumulate_frames(mdsf_plan* plan, void* d_coords, int dtype, int64_t n
     if (!p->timing || (p->timing == 2 && k != 2 && k != 3)) return hipSuccess;
     return hipEventRecord(p->tev[kTimedEvents * (tb + t) + k], st);
   };
-  MDSF_HIP(hipEventRecord(p->ev_fork, s));
-  MDSF_HIP(hipStreamWaitEvent(d, p->ev_fork, 0));
-  MDSF_HIP(hipStreamWaitEvent(f, p->ev_fork, 0));
-  for (int b = 0; b < kSlots; ++b) {
+  if (!cap) MDSF_HIP(hipStreamWaitEvent(s, p->ev_done, 0));
+  if (d != s) {
+    MDSF_HIP(hipEventRecord(p->ev_fork, s));
+    MDSF_HIP(hipStreamWaitEvent(d, p->ev_fork, 0));
+    if (f != d) MDSF_HIP(hipStreamWaitEvent(f, p->ev_fork, 0));
+  }
+  for (int b = 0; b < kSlots && !one; ++b) {
     MDSF_HIP(hipEventRecord(p->ev_dep[b], d));
     MDSF_HIP(hipEventRecord(p->ev_fft[b], f));
   }
@@ -632,7 +659,7 @@ int mdsf_accumulate_frames(mdsf_plan* plan, void* d_coords, int dtype, int64_t n
     char* c = static_cast<char*>(d_coords) + (size_t)t0 * fstride;
     int32_t* home = (t == ngroups - 1) ? d_home_cells : nullptr;   // the last frame's
     p->use_slot(b);
-    MDSF_HIP(hipStreamWaitEvent(s, p->ev_dep[b], 0));
+    if (!one) MDSF_HIP(hipStreamWaitEvent(s, p->ev_dep[b], 0));
     MDSF_HIP(mark(t, 0, s));
     MDSF_HIP(launch_prep(*p, c, dtype, arith, d_types, d_scale + 3 * t0, box, wrap_lo, wrap_hi,
                          d_occupancy, home, s, false, true, p->nfr - 1));
@@ -647,10 +674,12 @@ int mdsf_accumulate_frames(mdsf_plan* plan, void* d_coords, int dtype, int64_t n
                             /*join=*/false, aux_end));
     MDSF_HIP(mark(t, 1, s));
     if (p->timing == 1 && !aux_end) MDSF_HIP(mark(t, 10, s));
-    MDSF_HIP(hipEventRecord(p->ev_prep[b], s));
-    MDSF_HIP(hipStreamWaitEvent(d, p->ev_prep[b], 0));
+    if (d != s) {
+      MDSF_HIP(hipEventRecord(p->ev_prep[b], s));
+      MDSF_HIP(hipStreamWaitEvent(d, p->ev_prep[b], 0));
+    }
     if (lsplit) MDSF_HIP(hipStreamWaitEvent(d, p->ev_ljoin, 0));
-    MDSF_HIP(hipStreamWaitEvent(d, p->ev_fft[b], 0));
+    if (!one) MDSF_HIP(hipStreamWaitEvent(d, p->ev_fft[b], 0));
     // the deposition's events are recorded with the tiled kernel's own
     // dispatch (its begin and end, without the queue's dispatch latency)
     if (p->timing) {
@@ -664,8 +693,10 @@ int mdsf_accumulate_frames(mdsf_plan* plan, void* d_coords, int dtype, int64_t n
     // ev_dep[b], because they read the slot's atom state, which preparing
     // group t + kSlots overwrites as soon as ev_dep[b] has passed
     MDSF_HIP(launch_parked(*p, p->rho, d));
-    MDSF_HIP(hipEventRecord(p->ev_dep[b], d));
-    MDSF_HIP(hipStreamWaitEvent(f, p->ev_dep[b], 0));
+    if (!one) {
+      MDSF_HIP(hipEventRecord(p->ev_dep[b], d));
+      MDSF_HIP(hipStreamWaitEvent(f, p->ev_dep[b], 0));
+    }
     // x passes in pairs (one frame per group): frame t (even) waits for frame
     // t + 1, and one launch adds both frames' |F|^2, reading and writing the
     // FP64 sums once; frame t's slot is released with frame t + 1's (preparing
@@ -699,10 +730,11 @@ int mdsf_accumulate_frames(mdsf_plan* plan, void* d_coords, int dtype, int64_t n
     }
     if (!defer) {
       if (paired) MDSF_HIP(hipEventRecord(p->ev_fft[(t - 1) % kSlots], f));
-      MDSF_HIP(hipEventRecord(p->ev_fft[b], f));
+      if (f != s) MDSF_HIP(hipEventRecord(p->ev_fft[b], f));
     }
   }
-  MDSF_HIP(hipStreamWaitEvent(s, p->ev_fft[(ngroups - 1) % kSlots], 0));
+  MDSF_HIP(wait_for(s, p->ev_fft[(ngroups - 1) % kSlots], f));
+  if (!cap) MDSF_HIP(hipEventRecord(p->ev_done, s));
   return MDSF_OK;
 }
 
@@ -894,14 +926,19 @@ int mdsf_adjoint_frames(mdsf_plan* plan, void* d_coords, int dtype, int64_t nfra
   // with the weights and gathered on fft_stream.  Slot b is reused by group
   // t + kSlots only after group t's gather (the last reader of its atom state
   // and density buffer) has finished.
-  hipStream_t d = p->dep_stream, f = p->fft_stream;
   FrameGroup group(*p);
   const int64_t ngroups = (nframes + p->group - 1) / p->group;
+  // one group: all on `s`, as in the forward frame loop
+  const bool cap = capturing(s), one = ngroups == 1 && !cap;
+  hipStream_t d = one ? s : p->dep_stream, f = one ? s : p->fft_stream;
   auto first_of = [&](int64_t k) { return k * (nframes / ngroups) + std::min(k, nframes % ngroups); };
-  MDSF_HIP(hipEventRecord(p->ev_fork, s));
-  MDSF_HIP(hipStreamWaitEvent(d, p->ev_fork, 0));
-  MDSF_HIP(hipStreamWaitEvent(f, p->ev_fork, 0));
-  for (int b = 0; b < kSlots; ++b) MDSF_HIP(hipEventRecord(p->ev_fft[b], f));
+  if (!cap) MDSF_HIP(hipStreamWaitEvent(s, p->ev_done, 0));
+  if (!one) {
+    MDSF_HIP(hipEventRecord(p->ev_fork, s));
+    MDSF_HIP(hipStreamWaitEvent(d, p->ev_fork, 0));
+    MDSF_HIP(hipStreamWaitEvent(f, p->ev_fork, 0));
+    for (int b = 0; b < kSlots; ++b) MDSF_HIP(hipEventRecord(p->ev_fft[b], f));
+  }
   for (int64_t t = 0; t < ngroups; ++t) {
     const int b = (int)(t % kSlots);
     const int64_t t0 = first_of(t);
@@ -909,25 +946,30 @@ int mdsf_adjoint_frames(mdsf_plan* plan, void* d_coords, int dtype, int64_t nfra
     char* c = static_cast<char*>(d_coords) + (size_t)t0 * fstride;
     double* grad_t = d_grad + (size_t)t0 * p->sys.natoms * 3;
     p->use_slot(b);
-    MDSF_HIP(hipStreamWaitEvent(s, p->ev_fft[b], 0));
+    if (!one) MDSF_HIP(hipStreamWaitEvent(s, p->ev_fft[b], 0));
     // off the gather's stream
     MDSF_HIP(launch_fill_zero(grad_t, 3LL * p->sys.natoms * p->nfr, s));
     MDSF_HIP(launch_prep(*p, c, dtype, arith, d_types, d_scale + 3 * t0, box, wrap_lo, wrap_hi,
                          nullptr, nullptr, s));
     MDSF_HIP(launch_binning(*p, s, /*derivs=*/true));
-    MDSF_HIP(hipEventRecord(p->ev_prep[b], s));
-    MDSF_HIP(hipStreamWaitEvent(d, p->ev_prep[b], 0));
+    if (!one) {
+      MDSF_HIP(hipEventRecord(p->ev_prep[b], s));
+      MDSF_HIP(hipStreamWaitEvent(d, p->ev_prep[b], 0));
+    }
     MDSF_HIP(launch_deposit(*p, p->rho, d));
-    MDSF_HIP(hipEventRecord(p->ev_dep[b], d));
-    MDSF_HIP(hipStreamWaitEvent(f, p->ev_dep[b], 0));
+    if (!one) {
+      MDSF_HIP(hipEventRecord(p->ev_dep[b], d));
+      MDSF_HIP(hipStreamWaitEvent(f, p->ev_dep[b], 0));
+    }
     MDSF_HIP(launch_parked(*p, p->rho, f));
     MDSF_HIP(fft_forward(*p, p->rho, false, f));
     MDSF_HIP(fft_inverse(*p, p->adj_w, w_nyq, p->rho, f));
     MDSF_HIP(launch_deposit_adjoint(*p, p->rho, d_scale + 3 * t0, grad_t, f,
                                     /*derivs_ready=*/true, /*grad_zeroed=*/true));
-    MDSF_HIP(hipEventRecord(p->ev_fft[b], f));
+    if (!one) MDSF_HIP(hipEventRecord(p->ev_fft[b], f));
   }
-  MDSF_HIP(hipStreamWaitEvent(s, p->ev_fft[(ngroups - 1) % kSlots], 0));
+  MDSF_HIP(wait_for(s, p->ev_fft[(ngroups - 1) % kSlots], f));
+  if (!cap) MDSF_HIP(hipEventRecord(p->ev_done, s));
   return MDSF_OK;
 }
 

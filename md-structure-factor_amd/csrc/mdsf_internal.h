@@ -291,6 +291,7 @@ struct Plan {
   int64_t timed_groups = 0;  // groups timed since the last mdsf_stage_times
   int64_t timed_frames = 0;  // and their frames
   hipEvent_t ev_fork = nullptr;
+  hipEvent_t ev_done = nullptr;  // end of the plan's last frame loop, on its caller's stream
   hipEvent_t ev_prep[kSlots] = {}, ev_dep[kSlots] = {}, ev_fft[kSlots] = {};
   // adjoint (allocated on first use)
   long long adj_items = 0;
@@ -373,7 +374,8 @@ size_t fft_spec_bytes(const int n[3], int fft64);
 size_t fft_res_bytes(const int n[3], int fft64);
 hipError_t fft_autotune(Plan& p, hipStream_t s);
 
-hipError_t launch_fill_zero(double* p, long long n, hipStream_t s);
+hipError_t launch_fill_zero(double* p, long long n, hipStream_t s, double* q = nullptr,
+                            long long m = 0);
 // adj_w <- 2 dsf split into main / Nyquist parts
 hipError_t launch_adjoint_weights(Plan& p, const double* dsf, hipStream_t s);
 // grad[atom] = scale3 * dL/dr for the last prepared frame from dL/drho (grho,
