@@ -75,8 +75,8 @@ typedef struct mdsf_grid_desc {
 /* Plan lifecycle.  Validates the descriptor (Nborder <= N, even N),
  * allocates workspaces on the current device and generates the FFT twiddles
  * in FP64 on the GPU.  Any 3x3 ucell is accepted (dens.py:301): cells whose
- * metric couples z with x or y deposit through an FP64 per-voxel gather (any
- * plan precision); the adjoint entry points reject such plans with
+ * metric couples z with x or y deposit in FP64 from exponentials per z column
+ * (any plan precision); the adjoint entry points reject such plans with
  * MDSF_ERR_UNSUPPORTED. */
 int mdsf_plan_create(const mdsf_grid_desc* desc, mdsf_plan** out);
 int mdsf_plan_destroy(mdsf_plan* plan);
@@ -96,7 +96,7 @@ int mdsf_sf_reset(mdsf_plan* plan, mdsf_stream stream);
  * nothing, one cut by the high edge adds its kept part, one wholly at
  * negative indices is counted from the far end of the padded grid).
  * MDSF_ERR_UNSUPPORTED reports an internal size bound the frame exceeded
- * (the tile-list pool of FP32 orthogonal-cell plans). */
+ * (the tile-list pool). */
 int mdsf_check_errors(mdsf_plan* plan, mdsf_stream stream);
 
 /* The frame loop of dens.py:277-321 for `nframes` frames.
@@ -114,9 +114,9 @@ int mdsf_check_errors(mdsf_plan* plan, mdsf_stream stream);
  *   d_home_cells optional int32[natoms*3]: ir of the LAST frame (dens.py:285);
  *              INT32_MIN for a non-finite coordinate or |r / dr| >= 1e9.
  * Adds sum_frames |rfftn(folded density)|^2 into the plan accumulator, in
- * frame order (the x passes of frames 2k and 2k + 1 may share one launch,
- * which adds the two frames' terms one after the other: the same result as
- * frame by frame). */
+ * frame order (frames of a group, or the x passes of frames 2k and 2k + 1, may
+ * share one launch, which adds the frames' terms one after the other: the same
+ * result as frame by frame). */
 int mdsf_accumulate_frames(mdsf_plan* plan, void* d_coords, int dtype,
                            int64_t nframes, const int32_t* d_types,
                            const double* d_scale, const double box[3], int arith,
