@@ -712,32 +712,39 @@ __global__ __launch_bounds__(kThreads) void k_deposit(SysDev sys, const TypeDev*
 // precision.  Lane = one (x, y) column with 16 z accumulators; the
 // enumeration and visit order are the other kernels'.
 //
-// Column atoms: an atom off the corner regions that meets each axis of the tile
-// through one image has b_z evenly spaced along a column, so that
+// Column atoms (FP32 plans): an atom off the corner regions that meets each axis of
+// the tile through one image has b_z evenly spaced along a column, so that
 //   exp(-(b^T G b) k2) = Z(z) E rho^(z - h),   k2 = 1 / 2 s^2,
 //   Z = exp(-k2 g22 b_z^2) (staged, 0 outside the window), c = 2 (g02 b_x + g12 b_y),
 //   E = exp(-k2 (g00 b_x^2 + 2 g01 b_x b_y + g11 b_y^2 + c b_z(h))), rho = exp(k2 c dr_z):
 // with the anchors h = 4 and 12, four exponentials per column instead of sixteen;
-// the powers are products outward from the anchors (at most 4 roundings; S(q) of FP64
-// plans stays as near to 64 bits as with an exponential per voxel, 4e-16).  The
-// kernel is bound by its FP64 instructions: four frames of 8,000 atoms in a
-// dodecahedral cell on a grid of 100^3 took 2,317 us in all with an exponential
-// per voxel and image and take 912 (866 with one exponential per column and the
-// cross factors of each pair of axes staged per atom, which rounds more often).
-// Types whose factors could leave FP64's range (a cell matrix far from unit edges)
-// and the atoms left over take the full evaluation per voxel and image.
+// the powers are products outward from the anchors (at most 4 roundings).  Four
+// frames of 8,000 atoms in a dodecahedral cell on a grid of 100^3 took 2,317 us in
+// all with an exponential per voxel and image and take 912 (866 with one exponential
+// per column and the cross factors of each pair of axes staged per atom: the
+// exponentials are not what is left).  Types whose factors could leave FP64's range
+// (a cell matrix far from unit edges) and the atoms left over take the full
+// evaluation per voxel and image.  So do FP64 plans: ln Z and ln E cancel, and three
+// factors and their powers round more often than one exponential.  Weighted by the
+// values, the terms are 1.2e-16 to 2.9e-16 from exact with an exponential each and
+// 1.9e-16 to 5.9e-16 in the column form (cells of 0.3 to 0.8 Angstrom, dodecahedral
+// to strongly oblique); the density of 300 atoms at 1 Angstrom 1.5e-17 and 2.2e-17 of
+// its maximum (rms).  The price: the same four frames with an FP64 plan take 2,339 us,
+// 861 in the column form.
 //
 // Of those, per (x, y) image pair the z sources of tile cell c are u = c - N, c,
 // c + N, except where the corner slot applies (x and y off the core): for y on L
 // the H source is u = c + Nb (u >= N), for y on H the L source is u = c - Nb (u < 0).
+template <bool COL>
 struct StageGen {
   double r[NB][3];
   double amp[NB], k2[NB];  // Nel / sigma^3, 1 / (2 sigma^2)
   int lo[NB][3], len[NB][3];
-  // column atoms: the cells met along x and y, b at the cells, Z, and b_z at the
-  // tile's cells 4 and 12
-  int col[NB], xm[NB], ym[NB];
-  double bx[NB][T], by[NB][T], z[NB][T], bz[NB][2];
+  // column atoms (COL): the cells met along x and y, b at the cells, Z, and b_z at
+  // the tile's cells 4 and 12
+  static constexpr int NC = COL ? NB : 1;
+  int col[NC], xm[NC], ym[NC];
+  double bx[NC][T], by[NC][T], z[NC][T], bz[NC][2];
 };
 
 // The one image (side) through which the window [lo, lo + len) meets the tile's
@@ -767,7 +774,8 @@ void k_deposit_gen(SysDev sys,
                                                           const ACC* __restrict__ spill,
                                                           const int* __restrict__ spill_flag,
                                                           ACC* __restrict__ rho) {
-  __shared__ StageGen st;
+  constexpr bool COL = sizeof(ACC) == 4;
+  __shared__ StageGen<COL> st;
   __shared__ EnumShared<kMaxTypes> sh;
   const int tid = threadIdx.x;
   const int wave = tid >> 6, lane = tid & 63;
@@ -808,43 +816,47 @@ void k_deposit_gen(SysDev sys,
       st.amp[tid] = ty.amp;
       const double k2 = 1.0 / ty.two_sig2;
       st.k2[tid] = k2;
-      // column atom?  Its columns lie within (A + 1) dr along x and y, the tile's
-      // cells within (A + 17) dr along z
-      const double Bx = (ty.half[0] + 1) * sys.dr[0], By = (ty.half[1] + 1) * sys.dr[1],
-                   Bz = (ty.half[2] + 17) * sys.dr[2];
-      const double big = k2 * (g00 * Bx * Bx + g11 * By * By + fabs(g01x2) * Bx * By +
-                               (fabs(g02x2) * Bx + fabs(g12x2) * By) * Bz);
-      bool col = ok && !(q.w & kAtomCorner) && big < 600.0;
+      if constexpr (COL) {
+        // column atom?  Its columns lie within (A + 1) dr along x and y, the tile's
+        // cells within (A + 17) dr along z
+        const double Bx = (ty.half[0] + 1) * sys.dr[0], By = (ty.half[1] + 1) * sys.dr[1],
+                     Bz = (ty.half[2] + 17) * sys.dr[2];
+        const double big = k2 * (g00 * Bx * Bx + g11 * By * By + fabs(g01x2) * Bx * By +
+                                 (fabs(g02x2) * Bx + fabs(g12x2) * By) * Bz);
+        bool col = ok && !(q.w & kAtomCorner) && big < 600.0;
 #pragma unroll
-      for (int d = 0; d < 3; ++d)
-        col = col && one_image(ir[d] - ty.half[d], 2 * ty.half[d], tl.t0[d], tl.t1[d] - tl.t0[d],
-                               sys.n[d]) != kNoImage;
-      st.col[tid] = col;
-      st.xm[tid] = st.ym[tid] = 0;
-    }
-    __syncthreads();
-    // rows of the column atoms: 16 lanes per (atom, axis)
-    for (int it = tid; it < nbatch * 3 * T; it += kThreads) {
-      const int i = it % T, ad = it / T, a = ad / 3, d = ad - 3 * a;
-      if (!st.col[a]) continue;
-      const int t0 = pick3(tl.t0, d), tn = pick3(tl.t1, d) - t0, N = pick3(sys.n, d);
-      const int lo = st.lo[a][d], len = st.len[a][d];
-      const int u = t0 + i + one_image(lo, len, t0, tn, N);
-      const bool in = i < tn && u >= lo && u < lo + len;
-      const double dr = d == 0 ? sys.dr[0] : (d == 1 ? sys.dr[1] : sys.dr[2]);
-      const double bv = st.r[a][d] - (double)u * dr;
-      if (d < 2) {
-        (d == 0 ? st.bx : st.by)[a][i] = bv;
-        if (in) atomicOr(d == 0 ? &st.xm[a] : &st.ym[a], 1 << i);
-      } else {
-        st.z[a][i] = in ? exp(-(g22 * bv * bv) * st.k2[a]) : 0.0;
-        if (i == 4 || i == 12) st.bz[a][i / 8] = bv;
+        for (int d = 0; d < 3; ++d)
+          col = col && one_image(ir[d] - ty.half[d], 2 * ty.half[d], tl.t0[d], tl.t1[d] - tl.t0[d],
+                                 sys.n[d]) != kNoImage;
+        st.col[tid] = col;
+        st.xm[tid] = st.ym[tid] = 0;
       }
     }
     __syncthreads();
+    if constexpr (COL) {
+      // rows of the column atoms: 16 lanes per (atom, axis)
+      for (int it = tid; it < nbatch * 3 * T; it += kThreads) {
+        const int i = it % T, ad = it / T, a = ad / 3, d = ad - 3 * a;
+        if (!st.col[a]) continue;
+        const int t0 = pick3(tl.t0, d), tn = pick3(tl.t1, d) - t0, N = pick3(sys.n, d);
+        const int lo = st.lo[a][d], len = st.len[a][d];
+        const int u = t0 + i + one_image(lo, len, t0, tn, N);
+        const bool in = i < tn && u >= lo && u < lo + len;
+        const double dr = d == 0 ? sys.dr[0] : (d == 1 ? sys.dr[1] : sys.dr[2]);
+        const double bv = st.r[a][d] - (double)u * dr;
+        if (d < 2) {
+          (d == 0 ? st.bx : st.by)[a][i] = bv;
+          if (in) atomicOr(d == 0 ? &st.xm[a] : &st.ym[a], 1 << i);
+        } else {
+          st.z[a][i] = in ? exp(-(g22 * bv * bv) * st.k2[a]) : 0.0;
+          if (i == 4 || i == 12) st.bz[a][i / 8] = bv;
+        }
+      }
+      __syncthreads();
+    }
     if (gx < N0 && gy < N1) {
       for (int a = 0; a < nbatch; ++a) {
-        if (st.col[a]) {
+        if (COL && st.col[a]) {
           const int xm = __builtin_amdgcn_readfirstlane(st.xm[a]);
           const int ym = __builtin_amdgcn_readfirstlane(st.ym[a]);
           if (((xm >> ((wave & 1) * 8)) & 0xff) == 0 || ((ym >> ((wave >> 1) * 8)) & 0xff) == 0)
