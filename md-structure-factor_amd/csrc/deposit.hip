@@ -2286,29 +2286,42 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4, 8))
 // only the rows with a nonzero X on its 4 x rows.  A batch's results are summed over
 // the waves and stored in the atoms' slots.
 //
-// XY: with E = Y[y] 2^(CX[x] BY[y]) (Y itself, from dslices: the log2 that the
-// deposition takes would add its rounding error times the exponent) the lanes sum
-//   S1 = sum E dX U,  S2 = sum E X b_y U,  S3 = sum E X V,   dX = X (-2 g00 b_x / 2 s^2)
-// and the gradient is (S1 + c S2, (g01 / g00) S1 + (g11 / g01) c S2, S3) with
-// c = -2 g01 / 2 s^2.
+// XY: the atom's factor over the tile is X[x] Y[y] 2^(c b_x b_y) Z[z], c = -2 g01
+// log2(e) / 2 s^2 (X and Y themselves, rounded once, from dslices: the log2 that the
+// deposition takes would add its rounding error times the exponent).  With
+// E = Y 2^(c b_x b_y) the lanes sum in FP64
+//   S1 = sum E X b_x U,  S2 = sum E X b_y U,  S3 = sum E X V
+// and the gradient is (-2 / 2 s^2 (g00 S1 + g01 S2), -2 / 2 s^2 (g01 S1 + g11 S2), S3).
+// b_x and b_y in FP64 follow from the atom's position and the cell: of the images of a
+// cell only the nearest to the atom's home cell can lie in the window (2A <= N - 16).
 //
-// Quarter rows of X, dX and CX are rotated by row / 4, so that the 16 rows' quarters
+// Quarter rows of X and dX are rotated by row / 4, so that the 16 rows' quarters
 // that a wave reads at once lie in different banks.
 //
 // Bound by the matrix instructions and the fetches of the rows.  Orthogonal, 20,000
 // atoms at 128^3: 37 us a frame (k_adjoint_mfma, which enumerates its candidates and
-// contracts every row: 61).  xy-coupled, 6,000 atoms at 90 x 90 x 80: 20 us a frame,
-// the per-voxel gather 48, with the same error against FP64 (0.9e-7; 1.3e-7 with the
-// x and y sums in FP32).
+// contracts every row: 61).  xy-coupled, 6,000 atoms at 90 x 90 x 80: 32 us a frame, the
+// per-voxel gather 48.
+//
+// xy-coupled cells contract z with v_mfma_f64_16x16x4f64 and sum in FP64, as the gather
+// did: with FP32 products (20 us a frame) the x and y components were further from FP64
+// than the gather's.  Rms errors of the x / y / z components over twelve systems (angles
+// 120, 100 and 70 degrees, cells of 0.42 to 1 Angstrom), in units of 1e-8: gather 4.9 to
+// 10 / 6.9 to 13 / 6.8 to 14, FP32 products and X from expf 5.6 to 11 / 7.2 to 15 / 4.7
+// to 8.5, now 3.5 to 6.9 / 3.5 to 7.4 / 3.7 to 6.8.
 template <bool XY>
 struct StageAdjRows {
+  static constexpr int ND = XY ? 1 : NV + 1, NP = XY ? NV + 1 : 1;
   __align__(16) float vx[NV + 1][T];  // row NV stays zero: the lists' padding row
   __align__(16) float vy[NV + 1][T];
   __align__(16) float vz[NV + 1][T];
-  __align__(16) float dx[NV + 1][T];
   __align__(16) float dz[NV + 1][T];
-  __align__(16) float dy[NV + 1][T];  // XY: BY
-  __align__(16) float cx[XY ? NV + 1 : 1][T];
+  __align__(16) float dx[ND][T];
+  __align__(16) float dy[ND][T];
+  // XY: the rows' atoms: position and home cell along x and y, c
+  __align__(16) double rp[NP][2];
+  double rc[NP];
+  int ri[NP][2];
   // per-wave sums of each virtual atom
   typename std::conditional<XY, double, float>::type red[kThreads / 64][NV][3];
   __align__(4) unsigned char vq[NV][4];
@@ -2320,14 +2333,15 @@ struct StageAdjRows {
 template <int MT, bool XY>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(XY ? 3 : 4, 8))) void k_adjoint_lists(
     SysDev sys, const TypeDev* __restrict__ td, const int2* __restrict__ pool,
-    const int4* __restrict__ heads, const float* __restrict__ slices,
-    const float* __restrict__ bslices, const float* __restrict__ dslices,
+    const int4* __restrict__ heads, const int4* __restrict__ s_ir, const double* __restrict__ s_r,
+    const float* __restrict__ slices, const float* __restrict__ dslices,
     const float* __restrict__ grho, double* __restrict__ tpart) {
   __shared__ StageAdjRows<XY> st;
   __shared__ struct {
     int pre[MT][3], cpre[MT][3], cs[MT][3], nsl[MT][3];
     int slice_base[MT], slice_stride[MT], corner_base[MT], corner_stride[MT], type_start[MT];
     int part_base[MT];
+    double cxy[XY ? MT : 1];
   } ty;
   const int tid = threadIdx.x;
   const int wave = tid >> 6, lane = tid & 63;
@@ -2335,8 +2349,9 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(XY ? 3
   const int fr = blockIdx.y;   // frame of the group
   pool += fr * (long long)sys.f_pool;
   heads += fr * (long long)sys.f_tiles;
+  s_ir += fr * sys.f_atoms();
+  s_r += 3 * fr * sys.f_atoms();
   slices += fr * sys.f_slices;
-  bslices += fr * sys.f_bslices;
   dslices += fr * sys.f_slices;
   grho += fr * sys.f_points;
   tpart += 3 * fr * sys.f_adjt;
@@ -2358,11 +2373,17 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(XY ? 3
     ty.corner_stride[i] = d.corner_stride;
     ty.type_start[i] = d.type_start;
     ty.part_base[i] = (int)d.adjt_base;
+    if constexpr (XY) ty.cxy[i] = -2.0 * sys.g01 * 1.4426950408889634 / d.two_sig2;
   }
   if (tid < T) {
-    st.vx[NV][tid] = st.vy[NV][tid] = st.vz[NV][tid] = 0.f;
-    st.dx[NV][tid] = st.dy[NV][tid] = st.dz[NV][tid] = 0.f;
-    if constexpr (XY) st.cx[NV][tid] = 0.f;
+    st.vx[NV][tid] = st.vy[NV][tid] = st.vz[NV][tid] = st.dz[NV][tid] = 0.f;
+    if constexpr (!XY) st.dx[NV][tid] = st.dy[NV][tid] = 0.f;
+  }
+  if constexpr (XY) {
+    if (tid == 0) {
+      st.rp[NV][0] = st.rp[NV][1] = st.rc[NV] = 0.0;
+      st.ri[NV][0] = st.ri[NV][1] = 0;
+    }
   }
   Tile tl;
   tile_coords(sys, tl);
@@ -2370,6 +2391,8 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(XY ? 3
   const int base = hd.x, nreg = hd.y, ncor = hd.z, nc = hd.w;
   if (nreg + ncor == 0) return;   // uniform over the block
   // this wave's share of the tile, zero outside the grid
+  using S = typename std::conditional<XY, double, float>::type;
+  using M = Mfma<S>;
   float g[4][4];
   {
     const int gy = tl.t0[1] + n16;
@@ -2391,41 +2414,67 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(XY ? 3
   auto rot = [](int q, int row) { return 4 * ((q + (row >> 2)) & 3); };
   // a virtual atom's quarter rows; offsets as in deposit_lists (-1: none)
   struct Rows {
-    float4 x, y, z, dx, dy, dz, cx;
+    float4 x, y, z, dz, dx, dy;
+    double r[2], c;   // XY: the atom's position, home cell and c
+    int ir[2];
   };
   const float4 z4 = make_float4(0.f, 0.f, 0.f, 0.f);
-  auto load = [&](int o0, int o1, int o2, int ox, int oy, Rows& v) {
+  auto load = [&](int o0, int o1, int o2, Rows& v) {
     auto quarter = [&](const float* p, int o) {
       return *reinterpret_cast<const float4*>(p + max(o, 0) + 4 * q4);
     };
-    v.x = quarter(slices, o0);
+    v.x = quarter(XY ? dslices : slices, o0);
     v.y = quarter(XY ? dslices : slices, o1);
     v.z = quarter(slices, o2);
-    v.dx = quarter(dslices, o0);
     v.dz = quarter(dslices, o2);
-    if constexpr (XY) {
-      v.cx = quarter(bslices, ox);
-      v.dy = quarter(bslices, oy);
-      if (ox < 0) v.cx = z4;
-      if (oy < 0) v.dy = z4;
-    } else {
+    if constexpr (!XY) {
+      v.dx = quarter(dslices, o0);
       v.dy = quarter(dslices, o1);
+      if (o0 < 0) v.dx = z4;
       if (o1 < 0) v.dy = z4;
     }
-    if (o0 < 0) v.x = v.dx = z4;
+    if (o0 < 0) v.x = z4;
     if (o1 < 0) v.y = z4;
     if (o2 < 0) v.z = v.dz = z4;
+  };
+  // XY: sorted atom s of type t (kept in range: a list entry is off only after a
+  // reported error)
+  auto locate = [&](int s, int t, Rows& v) {
+    if constexpr (XY) {
+      s = min(max(s, 0), sys.natoms - 1);
+      v.r[0] = s_r[3 * (size_t)s + 0];
+      v.r[1] = s_r[3 * (size_t)s + 1];
+      const int2 q = *reinterpret_cast<const int2*>(s_ir + s);
+      v.ir[0] = q.x;
+      v.ir[1] = q.y;
+      v.c = ty.cxy[t];
+    }
   };
   auto stage = [&](int row, const Rows& v) {
     const int rp = rot(q4, row);
     *reinterpret_cast<float4*>(&st.vx[row][rp]) = v.x;
-    *reinterpret_cast<float4*>(&st.dx[row][rp]) = v.dx;
-    if constexpr (XY) *reinterpret_cast<float4*>(&st.cx[row][rp]) = v.cx;
     *reinterpret_cast<float4*>(&st.vy[row][4 * q4]) = v.y;
     *reinterpret_cast<float4*>(&st.vz[row][4 * q4]) = v.z;
-    *reinterpret_cast<float4*>(&st.dy[row][4 * q4]) = v.dy;
     *reinterpret_cast<float4*>(&st.dz[row][4 * q4]) = v.dz;
+    if constexpr (XY) {
+      if (q4 == 0) {
+        st.rp[row][0] = v.r[0];
+        st.rp[row][1] = v.r[1];
+        st.rc[row] = v.c;
+        st.ri[row][0] = v.ir[0];
+        st.ri[row][1] = v.ir[1];
+      }
+    } else {
+      *reinterpret_cast<float4*>(&st.dx[row][rp]) = v.dx;
+      *reinterpret_cast<float4*>(&st.dy[row][4 * q4]) = v.dy;
+    }
     st.vq[row][q4] = (v.x.x != 0 || v.x.y != 0 || v.x.z != 0 || v.x.w != 0) ? 1 : 0;
+  };
+  // b of cell c: of its images the nearest to the home cell
+  auto offset = [&](int c, int home, int n, double dr, double r) {
+    const int du = c - home;
+    const int u = du > n / 2 ? c - n : (du < -(n / 2) ? c + n : c);
+    return r - (double)u * dr;
   };
   // the wave's sums of staged rows [0, vtot), into st.red
   auto contract = [&](int vtot) {
@@ -2440,44 +2489,60 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(XY ? 3
     __builtin_amdgcn_wave_barrier();
     for (int k0 = 0; k0 < kend; k0 += 16) {
       const int k = st.wl[wave][k0 + n16];
-      const float4 zf = *reinterpret_cast<const float4*>(&st.vz[k][4 * q4l]);
-      const float4 dzf = *reinterpret_cast<const float4*>(&st.dz[k][4 * q4l]);
+      const v4f zf = *reinterpret_cast<const v4f*>(&st.vz[k][4 * q4l]);
+      const v4f dzf = *reinterpret_cast<const v4f*>(&st.dz[k][4 * q4l]);
       const int rp = rot(wave, k);
       const v4f xf = *reinterpret_cast<const v4f*>(&st.vx[k][rp]);
-      const v4f dxf = *reinterpret_cast<const v4f*>(&st.dx[k][rp]);
-      // U, V rows held by this lane: y = 4 (lane / 16) + r
-      const v4f yf = *reinterpret_cast<const v4f*>(&st.vy[k][4 * q4l]);
-      const v4f dyf = *reinterpret_cast<const v4f*>(&st.dy[k][4 * q4l]);
-      v4f cxf = v4f{0.f, 0.f, 0.f, 0.f};
-      if constexpr (XY) cxf = *reinterpret_cast<const v4f*>(&st.cx[k][rp]);
-      // xy-coupled cells: the contractions of x and y in FP64, as their gather's were
-      // (a third of the kernel's error in FP32, whose sums here are of differences)
-      using S = typename std::conditional<XY, double, float>::type;
+      // Y at the U, V rows held by this lane
+      v4f yf;
+      if constexpr (XY) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) yf[r] = st.vy[k][M::row(lane, r)];
+      } else {
+        yf = *reinterpret_cast<const v4f*>(&st.vy[k][4 * q4l]);
+      }
+      v4f dxf = v4f{0.f, 0.f, 0.f, 0.f}, dyf = dxf;
+      double by[4];
+      if constexpr (XY) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          by[r] = yf[r] != 0.f ? offset(tl.t0[1] + M::row(lane, r), st.ri[k][1], sys.n[1], sys.dr[1],
+                                        st.rp[k][1])
+                               : 0.0;   // outside the window (2^(...) could overflow)
+      } else {
+        dxf = *reinterpret_cast<const v4f*>(&st.dx[k][rp]);
+        dyf = *reinterpret_cast<const v4f*>(&st.dy[k][4 * q4l]);
+      }
       typedef S S4 __attribute__((ext_vector_type(4)));
       S4 w1 = S4{0, 0, 0, 0}, w2 = w1, w3 = w1;
       S sx = 0, sy = 0, sz = 0;
 #pragma unroll
       for (int b = 0; b < 4; ++b) {
-        v4f u = v4f{0.f, 0.f, 0.f, 0.f}, vv = u;
-        u = __builtin_amdgcn_mfma_f32_16x16x4f32(g[b][0], zf.x, u, 0, 0, 0);
-        vv = __builtin_amdgcn_mfma_f32_16x16x4f32(g[b][0], dzf.x, vv, 0, 0, 0);
-        u = __builtin_amdgcn_mfma_f32_16x16x4f32(g[b][1], zf.y, u, 0, 0, 0);
-        vv = __builtin_amdgcn_mfma_f32_16x16x4f32(g[b][1], dzf.y, vv, 0, 0, 0);
-        u = __builtin_amdgcn_mfma_f32_16x16x4f32(g[b][2], zf.z, u, 0, 0, 0);
-        vv = __builtin_amdgcn_mfma_f32_16x16x4f32(g[b][2], dzf.z, vv, 0, 0, 0);
-        u = __builtin_amdgcn_mfma_f32_16x16x4f32(g[b][3], zf.w, u, 0, 0, 0);
-        vv = __builtin_amdgcn_mfma_f32_16x16x4f32(g[b][3], dzf.w, vv, 0, 0, 0);
+        S4 u = S4{0, 0, 0, 0}, vv = u;
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+          float gv = g[b][c];
+          // (converted here each time: held in FP64 they would spill)
+          if constexpr (XY) asm volatile("" : "+v"(gv));
+          u = M::mul((S)gv, (S)zf[c], u);
+          vv = M::mul((S)gv, (S)dzf[c], vv);
+        }
         if constexpr (XY) {
+          const double bx = xf[b] != 0.f ? offset(tl.t0[0] + 4 * wave + b, st.ri[k][0], sys.n[0],
+                                                  sys.dr[0], st.rp[k][0])
+                                         : 0.0;
+          const double cx = st.rc[k] * bx;
           double p1 = 0.0, p2 = 0.0, p3 = 0.0;
 #pragma unroll
           for (int r = 0; r < 4; ++r) {
-            const double e = (double)(__builtin_amdgcn_exp2f(cxf[b] * dyf[r]) * yf[r]);
-            const double eu = e * (double)u[r];
+            const double e =
+                (double)__builtin_amdgcn_exp2f((float)(cx * by[r])) * (double)yf[r];
+            const double eu = e * u[r];
             p1 += eu;
-            p2 += eu * (double)dyf[r];
-            p3 += e * (double)vv[r];
+            p2 += eu * by[r];
+            p3 += e * vv[r];
           }
-          sx += (double)dxf[b] * p1;
+          sx += (double)xf[b] * bx * p1;
           sy += (double)xf[b] * p2;
           sz += (double)xf[b] * p3;
         } else {
@@ -2518,9 +2583,9 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(XY ? 3
       }
     double* o = tpart + 3 * (long long)pi;
     if constexpr (XY) {
-      const double c2 = -2.0 / td[st.pt[buf][a]].two_sig2 * s2;
-      o[0] = s1 + sys.g01 * c2;
-      o[1] = sys.g01 / sys.g00 * s1 + sys.g11 * c2;
+      const double inv = -2.0 / td[st.pt[buf][a]].two_sig2;
+      o[0] = inv * (sys.g00 * s1 + sys.g01 * s2);
+      o[1] = inv * (sys.g01 * s1 + sys.g11 * s2);
     } else {
       o[0] = s1;
       o[1] = s2;
@@ -2542,7 +2607,8 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(XY ? 3
       const int o0 = valid && j0 != kListNoSlice ? e.x + T * (ty.pre[t][0] + j0) : -1;
       const int o1 = valid && j1 != kListNoSlice ? e.x + T * (ty.pre[t][1] + j1) : -1;
       const int o2 = valid && j2 != kListNoSlice ? e.x + T * (ty.pre[t][2] + j2) : -1;
-      load(o0, o1, o2, o0, o1, v);
+      load(o0, o1, o2, v);
+      locate(ty.type_start[t] + (e.x - ty.slice_base[t]) / ty.slice_stride[t], t, v);
     };
     auto place = [&](const int2& e, bool valid, int b) {
       if (q4 != 0) return;
@@ -2580,16 +2646,16 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(XY ? 3
   for (int c0 = 0; c0 < ncor; c0 += NV / 4) {
     const int nca = min(NV / 4, ncor - c0);
     const int ca = tid >> 4, v = (tid >> 2) & 3;
-    int o0 = -1, o1 = -1, o2 = -1, ox = -1, oy = -1;
-    int t = 0, pi = -1;
+    int o0 = -1, o1 = -1, o2 = -1;
+    int t = 0, pi = -1, si = 0;
     if (ca < nca) {
       const int2 e = pool[base + nc - 1 - (c0 + ca)];
       t = (int)((unsigned)e.y >> 24);
+      si = e.x;
       const int slot = e.x - ty.type_start[t];
       const int ab = ty.slice_base[t] + slot * ty.slice_stride[t];
       const int cb = ty.corner_base[t] + slot * ty.corner_stride[t];
       const int j0 = e.y & 255, j1 = (e.y >> 8) & 255, j2 = (e.y >> 16) & 255;
-      const int so0 = j0 != kListNoSlice ? ab + T * (ty.pre[t][0] + j0) : -1;
       const int so1 = j1 != kListNoSlice ? ab + T * (ty.pre[t][1] + j1) : -1;
       const int so2 = j2 != kListNoSlice ? ab + T * (ty.pre[t][2] + j2) : -1;
       const int cb0 = j0 != kListNoSlice ? cb + T * (ty.cpre[t][0] + j0) : -1;
@@ -2598,12 +2664,11 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(XY ? 3
       o0 = cb0 >= 0 ? cb0 + (v == 0 ? 0 : ty.cs[t][0]) : -1;
       o1 = v == 0 ? so1 : (cb1 >= 0 ? cb1 + (v - 1) * ty.cs[t][1] : -1);
       o2 = v < 2 ? so2 : (cb2 >= 0 ? cb2 + (v - 2) * ty.cs[t][2] : -1);
-      ox = so0;
-      oy = so1;
       pi = slot_of(t, slot, j0, j1, j2);
     }
     Rows w;
-    load(o0, o1, o2, ox, oy, w);
+    load(o0, o1, o2, w);
+    locate(si, t, w);
     stage(tid >> 2, w);   // row 4 ca + v
     if ((tid & 15) == 0) {
       st.pidx[0][ca] = pi;
@@ -3012,8 +3077,8 @@ hipError_t launch_adjoint_tiles(Plan& p, const float* grho, hipStream_t s) {
     auto k = sys.mode == MODE_XY
                  ? (sys.ntypes <= 16 ? k_adjoint_lists<16, true> : k_adjoint_lists<kMaxTypes, true>)
                  : (sys.ntypes <= 16 ? k_adjoint_lists<16, false> : k_adjoint_lists<kMaxTypes, false>);
-    hipLaunchKernelGGL(k, grid, block, 0, s, sys, p.types, p.tl_pool, p.tl_head, p.slices,
-                       p.bslices, p.dslices, grho, p.adj_tpart);
+    hipLaunchKernelGGL(k, grid, block, 0, s, sys, p.types, p.tl_pool, p.tl_head, p.s_ir, p.s_r,
+                       p.slices, p.dslices, grho, p.adj_tpart);
     return hipGetLastError();
   }
   if (sys.ntypes <= 16)

@@ -145,7 +145,9 @@ struct FrameState {
   double* s_r = nullptr;
   void* tables = nullptr;
   float* slices = nullptr;   // (FP64 plans: doubles)
-  float* dslices = nullptr;  // derivatives of the slices in the atom position (adjoint)
+  // derivatives of the slices in the atom position (adjoint; xy-coupled cells: the x and
+  // y factors themselves, and the derivatives of z)
+  float* dslices = nullptr;
   // xy-coupled cells on tile lists: per regular x slice cell c_xy b_x, per
   // regular y slice cell b_y (same offsets as the slices), for the cross factor
   float* bslices = nullptr;

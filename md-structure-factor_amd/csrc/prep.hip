@@ -374,7 +374,8 @@ __global__ void k_tables(SysDev sys, const TypeDev* __restrict__ td, const int4*
 // and corner components) LY = log2 of the y factor (-inf outside the window)
 // instead of the factor; bslices holds CX = -2 g01 log2(e) / 2 s^2 b_x at the
 // regular x slice cells and BY = b_y at the regular y slice cells (0 outside
-// the window).  dslices holds the y factor itself in the y slices.
+// the window).  dslices holds the x and y factors themselves in the x and y slices,
+// rounded once from FP64.
 //
 // F: the plan's element type.  FP64 plans (orthogonal cells) take the exponent and
 // exp as k_tables does, without derivatives.
@@ -439,9 +440,14 @@ __global__ void k_slices(SysDev sys, const TypeDev* __restrict__ td, const int4*
     const double b = r - (double)u * dr;
     if constexpr (F32) {
       const float v = am * expf(-(float)(gk * (b * b)));
-      // xy-coupled cells: rounded once, as their gather's factors are
-      if (xyd) df = (float)((double)am * exp(-(gk * (b * b))) * (-2.0 * gk * b));
-      else df = v * (float)(-2.0 * gk * b);
+      // xy-coupled cells (k_adjoint_lists): rounded once from FP64, along x and y the
+      // factor itself
+      if (xyd) {
+        const double w = exp(-(gk * (b * b)));
+        df = (float)(d == 0 ? ty.amp * w : (d == 1 ? w : w * (-2.0 * gk * b)));
+      } else {
+        df = v * (float)(-2.0 * gk * b);
+      }
       return v;
     } else {
       return am * exp(-((gm * (b * b)) / ts2));
@@ -508,9 +514,6 @@ __global__ void k_slices(SysDev sys, const TypeDev* __restrict__ td, const int4*
         const double bs = r - (double)us * dr;
         bv[e] = any ? (F)(d == 0 ? cxy * bs : bs) : (F)0;
         if (ylog) {
-          dL[e] = vL[e];
-          dC[e] = vC[e];
-          dH[e] = vH[e];
           vL[e] = in ? lg(c - N) : -__builtin_inff();
           vC[e] = in ? lg(c) : -__builtin_inff();
           vH[e] = in ? lg(c + N) : -__builtin_inff();
