@@ -116,7 +116,9 @@ int mdsf_check_errors(mdsf_plan* plan, mdsf_stream stream);
  * Adds sum_frames |rfftn(folded density)|^2 into the plan accumulator, in
  * frame order (frames of a group, or the x passes of frames 2k and 2k + 1, may
  * share one launch, which adds the frames' terms one after the other: the same
- * result as frame by frame). */
+ * result as frame by frame).  Calls of one plan to this and to
+ * mdsf_adjoint_frames run in the order they are made, from whatever streams; the
+ * other entry points are ordered by their streams alone. */
 int mdsf_accumulate_frames(mdsf_plan* plan, void* d_coords, int dtype,
                            int64_t nframes, const int32_t* d_types,
                            const double* d_scale, const double box[3], int arith,

@@ -613,8 +613,8 @@ int mdsf_accumulate_frames(mdsf_plan* plan, void* d_coords, int dtype, int64_t n
   const int64_t ngroups = (nframes + p->group - 1) / p->group;
   // One group has nothing to overlap with: its stages stay on `s` (dep_stream where
   // the prepare stage splits), which saves the waits from stream to stream.  The
-  // slots are then not ordered by the shared streams, so calls wait for the plan's
-  // previous one.
+  // slots are then not ordered by the shared streams, so a call waits for the plan's
+  // previous frame loop (this one or the adjoint's).
   const bool split = split_prep(*p, nframes);
   const bool cap = capturing(s), one = ngroups == 1 && !cap;
   hipStream_t d = one && !split ? s : p->dep_stream, f = one ? d : p->fft_stream;
@@ -914,11 +914,14 @@ int mdsf_adjoint_frames(mdsf_plan* plan, void* d_coords, int dtype, int64_t nfra
   if (p->sys.natoms > 0 && nframes > 0 && !d_grad) return fail(MDSF_ERR_ARG, "null gradient");
   if (p->sys.mode == MODE_GEN) return fail(MDSF_ERR_UNSUPPORTED, kNoGenAdjoint);
   if ((rc = ensure_adjoint(*p)) != MDSF_OK) return rc;
+  if (nframes == 0) return MDSF_OK;
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   const long long nxy = (long long)p->sys.n[0] * p->sys.n[1];
   const double* w_nyq = p->adj_w + nxy * (p->sys.n[2] / 2);
+  const bool cap = capturing(s);
+  // the plan's last frame loop may still read the weights, on another stream
+  if (!cap) MDSF_HIP(hipStreamWaitEvent(s, p->ev_done, 0));
   MDSF_HIP(launch_adjoint_weights(*p, d_dsf, s));
-  if (nframes == 0) return MDSF_OK;
   const size_t esz = dtype == MDSF_F32 ? 4 : 8;
   const size_t fstride = (size_t)p->sys.natoms * 3 * esz;
   // Same slot pipeline as the forward frame loop: group t is prepared on
@@ -929,10 +932,9 @@ int mdsf_adjoint_frames(mdsf_plan* plan, void* d_coords, int dtype, int64_t nfra
   FrameGroup group(*p);
   const int64_t ngroups = (nframes + p->group - 1) / p->group;
   // one group: all on `s`, as in the forward frame loop
-  const bool cap = capturing(s), one = ngroups == 1 && !cap;
+  const bool one = ngroups == 1 && !cap;
   hipStream_t d = one ? s : p->dep_stream, f = one ? s : p->fft_stream;
   auto first_of = [&](int64_t k) { return k * (nframes / ngroups) + std::min(k, nframes % ngroups); };
-  if (!cap) MDSF_HIP(hipStreamWaitEvent(s, p->ev_done, 0));
   if (!one) {
     MDSF_HIP(hipEventRecord(p->ev_fork, s));
     MDSF_HIP(hipStreamWaitEvent(d, p->ev_fork, 0));
