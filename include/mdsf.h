@@ -118,7 +118,10 @@ int mdsf_check_errors(mdsf_plan* plan, mdsf_stream stream);
  * share one launch, which adds the frames' terms one after the other: the same
  * result as frame by frame).  Calls of one plan to this and to
  * mdsf_adjoint_frames run in the order they are made, from whatever streams; the
- * other entry points are ordered by their streams alone. */
+ * other entry points are ordered by their streams alone.  Neither can be captured
+ * into a HIP graph: on a capturing stream both return MDSF_ERR_UNSUPPORTED and
+ * enqueue nothing (mdsf_batch_run replays whole frame loops from a graph of its
+ * own). */
 int mdsf_accumulate_frames(mdsf_plan* plan, void* d_coords, int dtype,
                            int64_t nframes, const int32_t* d_types,
                            const double* d_scale, const double box[3], int arith,

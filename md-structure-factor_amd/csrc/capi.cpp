@@ -137,15 +137,19 @@ bool split_prep(const Plan& p, int64_t nframes) {
          p.sys.natoms * (long long)std::min<int64_t>(p.group, nframes) >= least;
 }
 
-// Is `s` being captured into a graph?  Then a frame loop neither waits for earlier calls
-// nor leaves work that later calls would wait for (its event would be the graph's).
-bool capturing(hipStream_t s) {
+// The frame loops fork to the plan's streams and order calls by an event of the plan,
+// neither of which belongs in a caller's graph (a trial of capturing them ended in a
+// crash inside hipStreamEndCapture whose cause is not known): refused, before anything
+// is enqueued.  A stream whose state cannot be asked (the null stream while another
+// stream is captured) is left to report its own errors.
+int refuse_capture(hipStream_t s, const char* call) {
   hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
   if (hipStreamIsCapturing(s, &st) != hipSuccess) {
     (void)hipGetLastError();
-    return true;
+    return MDSF_OK;
   }
-  return st != hipStreamCaptureStatusNone;
+  if (st == hipStreamCaptureStatusNone) return MDSF_OK;
+  return fail(MDSF_ERR_UNSUPPORTED, std::string(call) + " cannot be captured into a graph");
 }
 
 // `to` waits for the event, unless it is the stream that recorded it.
@@ -595,6 +599,7 @@ int mdsf_accumulate_frames(mdsf_plan* plan, void* d_coords, int dtype, int64_t n
   if (nframes < 0) return fail(MDSF_ERR_ARG, "negative frame count");
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   if (nframes == 0) return MDSF_OK;
+  if ((rc = refuse_capture(s, "mdsf_accumulate_frames")) != MDSF_OK) return rc;
   const size_t esz = dtype == MDSF_F32 ? 4 : 8;
   const size_t fstride = (size_t)p->sys.natoms * 3 * esz;
   // Three-stage pipeline over the kSlots frame slots (atom state + density
@@ -616,7 +621,7 @@ int mdsf_accumulate_frames(mdsf_plan* plan, void* d_coords, int dtype, int64_t n
   // slots are then not ordered by the shared streams, so a call waits for the plan's
   // previous frame loop (this one or the adjoint's).
   const bool split = split_prep(*p, nframes);
-  const bool cap = capturing(s), one = ngroups == 1 && !cap;
+  const bool one = ngroups == 1;
   hipStream_t d = one && !split ? s : p->dep_stream, f = one ? d : p->fft_stream;
   // groups of nearly equal size
   auto first_of = [&](int64_t k) { return k * (nframes / ngroups) + std::min(k, nframes % ngroups); };
@@ -642,7 +647,7 @@ int mdsf_accumulate_frames(mdsf_plan* plan, void* d_coords, int dtype, int64_t n
     if (!p->timing || (p->timing == 2 && k != 2 && k != 3)) return hipSuccess;
     return hipEventRecord(p->tev[kTimedEvents * (tb + t) + k], st);
   };
-  if (!cap) MDSF_HIP(hipStreamWaitEvent(s, p->ev_done, 0));
+  MDSF_HIP(hipStreamWaitEvent(s, p->ev_done, 0));
   if (d != s) {
     MDSF_HIP(hipEventRecord(p->ev_fork, s));
     MDSF_HIP(hipStreamWaitEvent(d, p->ev_fork, 0));
@@ -734,7 +739,7 @@ int mdsf_accumulate_frames(mdsf_plan* plan, void* d_coords, int dtype, int64_t n
     }
   }
   MDSF_HIP(wait_for(s, p->ev_fft[(ngroups - 1) % kSlots], f));
-  if (!cap) MDSF_HIP(hipEventRecord(p->ev_done, s));
+  MDSF_HIP(hipEventRecord(p->ev_done, s));
   return MDSF_OK;
 }
 
@@ -913,14 +918,14 @@ int mdsf_adjoint_frames(mdsf_plan* plan, void* d_coords, int dtype, int64_t nfra
   if (!d_dsf) return fail(MDSF_ERR_ARG, "null dL/dS");
   if (p->sys.natoms > 0 && nframes > 0 && !d_grad) return fail(MDSF_ERR_ARG, "null gradient");
   if (p->sys.mode == MODE_GEN) return fail(MDSF_ERR_UNSUPPORTED, kNoGenAdjoint);
-  if ((rc = ensure_adjoint(*p)) != MDSF_OK) return rc;
   if (nframes == 0) return MDSF_OK;
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+  if ((rc = refuse_capture(s, "mdsf_adjoint_frames")) != MDSF_OK) return rc;
+  if ((rc = ensure_adjoint(*p)) != MDSF_OK) return rc;
   const long long nxy = (long long)p->sys.n[0] * p->sys.n[1];
   const double* w_nyq = p->adj_w + nxy * (p->sys.n[2] / 2);
-  const bool cap = capturing(s);
   // the plan's last frame loop may still read the weights, on another stream
-  if (!cap) MDSF_HIP(hipStreamWaitEvent(s, p->ev_done, 0));
+  MDSF_HIP(hipStreamWaitEvent(s, p->ev_done, 0));
   MDSF_HIP(launch_adjoint_weights(*p, d_dsf, s));
   const size_t esz = dtype == MDSF_F32 ? 4 : 8;
   const size_t fstride = (size_t)p->sys.natoms * 3 * esz;
@@ -932,7 +937,7 @@ int mdsf_adjoint_frames(mdsf_plan* plan, void* d_coords, int dtype, int64_t nfra
   FrameGroup group(*p);
   const int64_t ngroups = (nframes + p->group - 1) / p->group;
   // one group: all on `s`, as in the forward frame loop
-  const bool one = ngroups == 1 && !cap;
+  const bool one = ngroups == 1;
   hipStream_t d = one ? s : p->dep_stream, f = one ? s : p->fft_stream;
   auto first_of = [&](int64_t k) { return k * (nframes / ngroups) + std::min(k, nframes % ngroups); };
   if (!one) {
@@ -971,7 +976,7 @@ int mdsf_adjoint_frames(mdsf_plan* plan, void* d_coords, int dtype, int64_t nfra
     if (!one) MDSF_HIP(hipEventRecord(p->ev_fft[b], f));
   }
   MDSF_HIP(wait_for(s, p->ev_fft[(ngroups - 1) % kSlots], f));
-  if (!cap) MDSF_HIP(hipEventRecord(p->ev_done, s));
+  MDSF_HIP(hipEventRecord(p->ev_done, s));
   return MDSF_OK;
 }
 
