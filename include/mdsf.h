@@ -79,6 +79,20 @@ typedef struct mdsf_grid_desc {
  * (any plan precision); the adjoint entry points reject such plans with
  * MDSF_ERR_UNSUPPORTED. */
 int mdsf_plan_create(const mdsf_grid_desc* desc, mdsf_plan** out);
+
+/* mdsf_plan_create for calls of at most `max_frames` frames (0: any number).  The
+ * frame loops hand each kernel a group of frames of a small grid at once, and the
+ * plan holds the state of a whole group in each of its three slots (up to 16
+ * frames, 2 GiB in all and as much again for gradients).  A plan that will only see
+ * a few frames per call takes less memory when it is told; longer calls still work,
+ * in smaller groups.  Groups also shrink where less than about half of the device's
+ * memory is free, down to one frame when memory is out.  Results do not depend on
+ * the group. */
+int mdsf_plan_create_frames(const mdsf_grid_desc* desc, int64_t max_frames, mdsf_plan** out);
+
+/* Frames per group of the plan, and of its gradients (0 before the first gradient
+ * call).  Either pointer may be NULL. */
+int mdsf_plan_group(mdsf_plan* plan, int32_t* frames, int32_t* adjoint_frames);
 int mdsf_plan_destroy(mdsf_plan* plan);
 const char* mdsf_last_error(void);
 int mdsf_version(void);
@@ -291,6 +305,10 @@ typedef struct mdsf_batch mdsf_batch;
 
 int mdsf_batch_create(const mdsf_grid_desc* descs, int32_t nsys,
                       mdsf_batch** out);
+/* The same for at most max_frames[i] frames of system i (0: any number; see
+ * mdsf_plan_create_frames). */
+int mdsf_batch_create_frames(const mdsf_grid_desc* descs, const int64_t* max_frames, int32_t nsys,
+                             mdsf_batch** out);
 int mdsf_batch_destroy(mdsf_batch* batch);
 
 /* The plan of system `sys` (for mdsf_sf_read, mdsf_outputs, ...); NULL if out

@@ -146,6 +146,11 @@ using namespace mdsf;
 extern "C" {
 
 int mdsf_batch_create(const mdsf_grid_desc* descs, int32_t nsys, mdsf_batch** out) {
+  return mdsf_batch_create_frames(descs, nullptr, nsys, out);
+}
+
+int mdsf_batch_create_frames(const mdsf_grid_desc* descs, const int64_t* max_frames, int32_t nsys,
+                             mdsf_batch** out) {
   if (!descs || !out || nsys <= 0) return fail(MDSF_ERR_ARG, "need at least one system");
   *out = nullptr;
   Batch* b = new Batch();
@@ -153,7 +158,7 @@ int mdsf_batch_create(const mdsf_grid_desc* descs, int32_t nsys, mdsf_batch** ou
     mdsf_grid_desc d = descs[i];
     d.flags |= MDSF_AUTOTUNE;
     mdsf_plan* p = nullptr;
-    const int rc = mdsf_plan_create(&d, &p);
+    const int rc = mdsf_plan_create_frames(&d, max_frames ? max_frames[i] : 0, &p);
     if (rc != MDSF_OK) {
       const std::string msg = mdsf_last_error();
       free_batch(b);

@@ -61,7 +61,12 @@ struct Arena {
       if (zero) cleared = off;
     }
     hipError_t e = hipMalloc(base, std::max(off, (size_t)1));
-    if (e != hipSuccess) return e;
+    if (e != hipSuccess) {
+      (void)hipGetLastError();
+      *base = nullptr;
+      for (Item& it : items) *it.p = nullptr;
+      return e;
+    }
     for (size_t i = 0; i < items.size(); ++i) *items[i].p = static_cast<char*>(*base) + at[i];
     return cleared ? hipMemset(*base, 0, cleared) : hipSuccess;
   }
@@ -115,15 +120,6 @@ void free_plan(Plan* p) {
   delete p;
 }
 
-int make_axis(FftAxis& ax, int n, Arena& arena) {
-  ax.n = n;
-  if (!fft_factor(n, ax.radix, &ax.nstages))
-    return fail(MDSF_ERR_UNSUPPORTED, "FFT length " + std::to_string(n) + " needs too many stages");
-  arena.add(&ax.tw, (size_t)n);
-  arena.add(&ax.tw64, (size_t)n);
-  return MDSF_OK;
-}
-
 // The prepare stage's branches go on their own streams on large grids and for groups of
 // many atoms; with less work the cross-stream waits (about 10 us each) cost more than
 // the branches overlap.  16 frames of 50,000 atoms at 104 x 90 x 80 in groups of 4: 1,443
@@ -164,27 +160,40 @@ struct FrameGroup {
   ~FrameGroup() { p.nfr = 1; }
 };
 
+// Free and total memory of the current device, zeros if they cannot be asked.
+void device_memory(size_t* free, size_t* total) {
+  if (hipMemGetInfo(free, total) == hipSuccess) return;
+  (void)hipGetLastError();
+  *free = *total = 0;
+}
+
 int ensure_adjoint(Plan& p) {
   const size_t nxy = (size_t)p.sys.n[0] * p.sys.n[1];
   const size_t m = (size_t)p.sys.n[2] / 2;
-  const size_t g = (size_t)p.group;
   if (p.adj_arena) return MDSF_OK;
   // one device allocation: the spectrum's weights, and the tiled adjoint's slice
-  // derivatives (per frame slot) and result slots or the gather's partial sums
+  // derivatives (per frame slot) and result slots or the gather's partial sums, for as
+  // many frames of a group as fit a budget of their own
   auto take = [&] {
-    Arena arena;
-    arena.add(&p.adj_w, nxy * (m + 1));
-    if (p.adj_tslots > 0) {
-      for (FrameState& f : p.slot) arena.add(&f.dslices, g * (size_t)p.slice_floats);
-      arena.add(&p.adj_tpart, 3 * g * (size_t)p.adj_tslots);
-    } else {
-      arena.add(&p.adj_part, 3 * g * (size_t)p.adj_items);
-    }
-    return arena.take(&p.adj_arena);
+    const bool tiled = p.adj_tslots > 0;
+    const size_t slots = (size_t)(tiled ? p.adj_tslots : p.adj_items);
+    const size_t bytes = 24 * slots + (tiled ? kSlots * 4 * (size_t)p.slice_floats : 0);
+    size_t free, total;
+    device_memory(&free, &total);
+    p.adj_group = std::min(p.group, group_fit(bytes, free, total));
+    return take_group(&p.adj_group, hipErrorOutOfMemory, [&](int frames) {
+      const size_t g = (size_t)frames;
+      Arena arena;
+      arena.add(&p.adj_w, nxy * (m + 1));
+      if (tiled)
+        for (FrameState& f : p.slot) arena.add(&f.dslices, g * (size_t)p.slice_floats);
+      arena.add(tiled ? &p.adj_tpart : &p.adj_part, 3 * g * slots);
+      return arena.take(&p.adj_arena);
+    });
   };
   hipError_t e = take();
   if (e == hipErrorOutOfMemory && p.adj_tslots > 0 && p.sys.mode == MODE_XY) {
-    (void)hipGetLastError();   // xy-coupled cells: the gather, which needs less
+    // xy-coupled cells: the gather, which needs less
     p.adj_tslots = 0;
     e = take();
   }
@@ -227,8 +236,13 @@ const char* mdsf_last_error(void) { return g_last_error.c_str(); }
 int mdsf_version(void) { return 10000; }
 
 int mdsf_plan_create(const mdsf_grid_desc* desc, mdsf_plan** out) {
+  return mdsf_plan_create_frames(desc, 0, out);
+}
+
+int mdsf_plan_create_frames(const mdsf_grid_desc* desc, int64_t max_frames, mdsf_plan** out) {
   if (!desc || !out) return fail(MDSF_ERR_ARG, "null descriptor or output");
   *out = nullptr;
+  if (max_frames < 0) return fail(MDSF_ERR_ARG, "negative frame count");
   for (int d = 0; d < 3; ++d) {
     const int n = desc->n[d];
     if (n < 2 || (n % 2) != 0) return fail(MDSF_ERR_ARG, "grid sizes must be even and >= 2");
@@ -424,98 +438,112 @@ int mdsf_plan_create(const mdsf_grid_desc* desc, mdsf_plan** out) {
   }
   (void)hipGetDevice(&p->device);
 
-  // frames per group (kGroupTiles), within the state budget
-  s.f_slices = p->slice_floats;
-  s.f_bslices = p->bslice_floats;
-  const bool tables = p->fft64 && s.mode != MODE_GEN && p->slice_floats == 0;
-  s.f_tables = tables ? table_floats : 0;
-  const bool staged = p->spill_tiles > 0 && p->spill_tiles <= kMaxSpillBufTiles;
-  s.f_spill = staged ? p->spill_tiles * kTile * kTile * kTile : 0;
   s.f_points = (long long)desc->n[0] * desc->n[1] * desc->n[2];
   s.f_adjt = p->adj_tslots;
   s.f_adji = p->adj_items;
-  s.f_pool = (int)p->tl_cap;
   s.f_aux = s.nbuckets / 1024 + 2;
   s.f_tiles = s.ntiles[0] * s.ntiles[1] * s.ntiles[2];
-  {
-    const size_t rs = p->fft64 ? 8 : 4;
+  const bool staged = p->spill_tiles > 0 && p->spill_tiles <= kMaxSpillBufTiles;
+  s.f_spill = staged ? p->spill_tiles * kTile * kTile * kTile : 0;
+  for (FftAxis* ax : {&p->ax_x, &p->ax_y, &p->ax_zc}) {
+    ax->n = ax == &p->ax_x ? desc->n[0] : (ax == &p->ax_y ? desc->n[1] : desc->n[2] / 2);
+    if (!fft_factor(ax->n, ax->radix, &ax->nstages)) {
+      const int n = ax->n;
+      free_plan(p);
+      return fail(MDSF_ERR_UNSUPPORTED, "FFT length " + std::to_string(n) + " needs too many stages");
+    }
+  }
+  const size_t nx = desc->n[0], ny = desc->n[1], nz = desc->n[2];
+  const size_t m = nz / 2;
+  const size_t rs = p->fft64 ? 8 : 4;
+  const size_t spec_bytes = fft_spec_bytes(s.n, p->fft64), res_bytes = fft_res_bytes(s.n, p->fft64);
+  // the plan's buffers with `frames` frames in every slot
+  auto allocate = [&](int frames) {
+    const size_t grp = (size_t)frames, nat = grp * (size_t)desc->natoms;
+    Arena arena;
+    arena.add(&p->types, (size_t)kMaxTypes);
+    for (FrameState& f : p->slot) {
+      arena.add(&f.ir4, nat);
+      arena.add(&f.key, nat);
+      arena.add(&f.rpos, 3 * nat);
+      const size_t nbk = grp * ((size_t)s.nbuckets + 1);
+      arena.add(&f.bucket_count, nbk, true);
+      arena.add(&f.bucket_off, nbk, true);
+      arena.add(&f.bucket_cur, nbk);
+      arena.add(&f.bucket_aux, grp * (size_t)s.f_aux);
+      arena.add(&f.s_idx, nat);
+      arena.add(&f.s_tmp, nat);
+      arena.add(&f.s_ir, nat);
+      arena.add(&f.s_r, 3 * nat);
+      arena.add(reinterpret_cast<double**>(&f.tables), grp * (size_t)s.f_tables);
+      arena.add(&f.slices, grp * (size_t)p->slice_floats * (p->fft64 ? 2 : 1));   // plan precision
+      if (p->bslice_floats > 0) arena.add(&f.bslices, grp * (size_t)p->bslice_floats);
+      arena.add(&f.corners, grp * kCornerInts, true);
+      if (staged) {
+        arena.add(reinterpret_cast<unsigned char**>(&f.spill), grp * (size_t)s.f_spill * rs);
+        // no tile is read before a frame's binning flags it (a frame without atoms
+        // never runs the binning)
+        arena.add(&f.spill_flag, grp * (size_t)p->spill_tiles, true);
+      }
+      if (p->tl_cap > 0) {
+        arena.add(&f.tl_pool, grp * (size_t)p->tl_cap);
+        arena.add(&f.tl_head, grp * (size_t)s.f_tiles);
+      }
+    }
+    arena.add(&p->err, (size_t)1, true);
+    for (int b = 0; b < kSlots; ++b) {
+      arena.add(reinterpret_cast<unsigned char**>(&p->rho_buf[b]), grp * nx * ny * nz * rs);
+      arena.add(reinterpret_cast<unsigned char**>(&p->spec_buf[b]), grp * spec_bytes);
+      arena.add(reinterpret_cast<double2**>(&p->nyq_buf[b]), grp * nx * ny);
+      if (res_bytes > 0)
+        arena.add(reinterpret_cast<unsigned char**>(&p->res_buf[b]), grp * res_bytes);
+    }
+    arena.add(&p->sf_main, nx * ny * m, true);
+    arena.add(&p->sf_nyq, nx * ny, true);
+    for (FftAxis* ax : {&p->ax_x, &p->ax_y, &p->ax_zc}) {
+      arena.add(&ax->tw, (size_t)ax->n);
+      arena.add(&ax->tw64, (size_t)ax->n);
+    }
+    arena.add(&p->tw_r2c, nz);
+    arena.add(&p->tw_r2c64, nz);
+    return arena.take(&p->arena);
+  };
+  // frames per group (group.h): fewer while memory is out, and last the factor tables
+  // of FP64 orthogonal cells in place of their tile slices and lists, which take more
+  auto take = [&] {
+    s.f_slices = p->slice_floats;
+    s.f_bslices = p->bslice_floats;
+    s.f_tables = p->fft64 && s.mode != MODE_GEN && p->slice_floats == 0 ? table_floats : 0;
+    s.f_pool = (int)p->tl_cap;
     const size_t bytes = (size_t)desc->natoms * 112 + (size_t)s.nbuckets * 12 +
                          (size_t)p->slice_floats * rs + (size_t)p->bslice_floats * 4 +
                          (size_t)s.f_tables * 8 + (size_t)s.f_spill * rs + (size_t)p->tl_cap * 8 +
-                         (size_t)s.f_points * rs + fft_spec_bytes(s.n, p->fft64) +
-                         fft_res_bytes(s.n, p->fft64) + (size_t)desc->n[0] * desc->n[1] * 16;
-    const long long fit = (long long)(kGroupBytes / (kSlots * bytes));
-    const long long want = (kGroupTiles + s.f_tiles - 1) / s.f_tiles;
-    p->group = (int)std::max(1LL, std::min({want, fit, (long long)kMaxGroup}));
+                         (size_t)s.f_points * rs + spec_bytes + res_bytes + nx * ny * 16;
+    size_t free, total;
+    device_memory(&free, &total);
+    p->group = group_frames(s.f_tiles, max_frames, kSlots * bytes, free, total);
+    return take_group(&p->group, hipErrorOutOfMemory, allocate);
+  };
+  hipError_t e = take();
+  if (e == hipErrorOutOfMemory && p->fft64 && p->slice_floats > 0) {
+    p->slice_floats = p->tl_cap = 0;
+    e = take();
   }
-  const size_t grp = (size_t)p->group;
-
-  const size_t nat = grp * (size_t)desc->natoms;
-  const size_t nx = desc->n[0], ny = desc->n[1], nz = desc->n[2];
-  const size_t m = nz / 2;
-  hipError_t e = hipSuccess;
-#define TRY(x)                          \
-  do {                                  \
-    e = (x);                            \
-    if (e != hipSuccess) {              \
-      int rc = hip_fail(e, #x);         \
-      free_plan(p);                     \
-      return rc;                        \
-    }                                   \
-  } while (0)
-  Arena arena;
-  arena.add(&p->types, (size_t)kMaxTypes);
-  for (FrameState& f : p->slot) {
-    arena.add(&f.ir4, nat);
-    arena.add(&f.key, nat);
-    arena.add(&f.rpos, 3 * nat);
-    const size_t nbk = grp * ((size_t)s.nbuckets + 1);
-    arena.add(&f.bucket_count, nbk, true);
-    arena.add(&f.bucket_off, nbk, true);
-    arena.add(&f.bucket_cur, nbk);
-    arena.add(&f.bucket_aux, grp * (size_t)s.f_aux);
-    arena.add(&f.s_idx, nat);
-    arena.add(&f.s_tmp, nat);
-    arena.add(&f.s_ir, nat);
-    arena.add(&f.s_r, 3 * nat);
-    arena.add(reinterpret_cast<double**>(&f.tables), grp * (size_t)s.f_tables);
-    arena.add(&f.slices, grp * (size_t)p->slice_floats * (p->fft64 ? 2 : 1));   // plan precision
-    if (p->bslice_floats > 0) arena.add(&f.bslices, grp * (size_t)p->bslice_floats);
-    arena.add(&f.corners, grp * kCornerInts, true);
-    if (staged) {
-      arena.add(reinterpret_cast<unsigned char**>(&f.spill),
-                grp * (size_t)s.f_spill * (p->fft64 ? 8 : 4));
-      // no tile is read before a frame's binning flags it (a frame without atoms
-      // never runs the binning)
-      arena.add(&f.spill_flag, grp * (size_t)p->spill_tiles, true);
-    }
-    if (p->tl_cap > 0) {
-      arena.add(&f.tl_pool, grp * (size_t)p->tl_cap);
-      arena.add(&f.tl_head, grp * (size_t)s.f_tiles);
-    }
-  }
-  arena.add(&p->err, (size_t)1, true);
-  for (int b = 0; b < kSlots; ++b) {
-    arena.add(reinterpret_cast<unsigned char**>(&p->rho_buf[b]),
-              grp * nx * ny * nz * (p->fft64 ? 8 : 4));
-    arena.add(reinterpret_cast<unsigned char**>(&p->spec_buf[b]), grp * fft_spec_bytes(s.n, p->fft64));
-    arena.add(reinterpret_cast<double2**>(&p->nyq_buf[b]), grp * nx * ny);
-    if (fft_res_bytes(s.n, p->fft64) > 0)
-      arena.add(reinterpret_cast<unsigned char**>(&p->res_buf[b]),
-                grp * fft_res_bytes(s.n, p->fft64));
-  }
-  arena.add(&p->sf_main, nx * ny * m, true);
-  arena.add(&p->sf_nyq, nx * ny, true);
   int rc;
-  if ((rc = make_axis(p->ax_x, desc->n[0], arena)) != MDSF_OK ||
-      (rc = make_axis(p->ax_y, desc->n[1], arena)) != MDSF_OK ||
-      (rc = make_axis(p->ax_zc, desc->n[2] / 2, arena)) != MDSF_OK) {
+#define TRY(x)                    \
+  do {                            \
+    e = (x);                      \
+    if (e != hipSuccess) {        \
+      rc = hip_fail(e, #x);       \
+      free_plan(p);               \
+      return rc;                  \
+    }                             \
+  } while (0)
+  if (e != hipSuccess) {
+    rc = hip_fail(e, "plan buffers");
     free_plan(p);
     return rc;
   }
-  arena.add(&p->tw_r2c, nz);
-  arena.add(&p->tw_r2c64, nz);
-  TRY(arena.take(&p->arena));
   TRY(hipMemcpy(p->types, p->types_host, sizeof(TypeDev) * kMaxTypes, hipMemcpyHostToDevice));
   for (FftAxis* ax : {&p->ax_x, &p->ax_y, &p->ax_zc})
     TRY(fft_make_twiddles(ax->tw, ax->tw64, ax->n, nullptr));
@@ -550,6 +578,14 @@ int mdsf_plan_create(const mdsf_grid_desc* desc, mdsf_plan** out) {
     }
   }
   *out = reinterpret_cast<mdsf_plan*>(p);
+  return MDSF_OK;
+}
+
+int mdsf_plan_group(mdsf_plan* plan, int32_t* frames, int32_t* adjoint_frames) {
+  const Plan* p = reinterpret_cast<Plan*>(plan);
+  if (!p) return fail(MDSF_ERR_ARG, "null plan");
+  if (frames) *frames = p->group;
+  if (adjoint_frames) *adjoint_frames = p->adj_arena ? p->adj_group : 0;
   return MDSF_OK;
 }
 
@@ -935,7 +971,7 @@ int mdsf_adjoint_frames(mdsf_plan* plan, void* d_coords, int dtype, int64_t nfra
   // t + kSlots only after group t's gather (the last reader of its atom state
   // and density buffer) has finished.
   FrameGroup group(*p);
-  const int64_t ngroups = (nframes + p->group - 1) / p->group;
+  const int64_t ngroups = (nframes + p->adj_group - 1) / p->adj_group;
   // one group: all on `s`, as in the forward frame loop
   const bool one = ngroups == 1;
   hipStream_t d = one ? s : p->dep_stream, f = one ? s : p->fft_stream;

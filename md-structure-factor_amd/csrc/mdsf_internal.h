@@ -8,6 +8,7 @@
 #include <vector>
 
 #include "../../include/mdsf.h"
+#include "group.h"
 
 namespace mdsf {
 
@@ -170,19 +171,6 @@ struct FrameState {
 // deposited and the ones before it transformed without waiting for a buffer.
 constexpr int kSlots = 3;
 
-// Frames per group.  A small grid's frame leaves most of the chip idle (64
-// tiles of a 64^3 grid for 256 CUs) and its dozen and a half launches each take
-// their few microseconds of latency, so the frame loops hand every kernel the
-// frames of a group at once, as blockIdx.y: as many as make kGroupTiles tiles,
-// at most kMaxGroup, within kGroupBytes of state for the slots together.  Grids
-// of kGroupTiles tiles and more fill the chip with one frame.  Before and after:
-// ten frames of 2,700 atoms at 64^3 1,091 -> 292 us, sixteen forward and backward
-// frames at 128^3 4,865 -> 3,242 us, eight systems of 64^3 to 192^3 in one graph
-// 11,778 -> 9,012 us; one frame per group at 256^3, 4,930 and 4,915 us.
-constexpr int kGroupTiles = 2048;
-constexpr int kMaxGroup = 16;
-constexpr size_t kGroupBytes = (size_t)2 << 30;
-
 struct Plan {
   SysDev sys{};
   TypeDev types_host[kMaxTypes]{};
@@ -235,7 +223,8 @@ struct Plan {
   // Frame slot b: its atom state and density / spectrum buffer become the
   // ones the launches below use (kernel arguments are taken at launch).
   int cur_slot = 0;
-  int group = 1;                 // frames a slot holds
+  int group = 1;                 // frames a slot holds (group.h)
+  int adj_group = 1;             // frames the adjoint's buffers hold, at most `group`
   int nfr = 1;                   // frames the next launches cover (the frame loops set it)
   void use_slot(int b) {
     b %= kSlots;

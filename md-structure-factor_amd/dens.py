@@ -148,15 +148,24 @@ def get_dplot(dmag):
     return sfplt.cpu().numpy()
 
 
+def _call_frames(s):
+    """The most frames that a call of this run's plan has."""
+    if RANDOM_NOISE > 0:
+        return 1
+    return max(1, min(s.nframes, int(CHECKPOINT_FRAMES) if CHECKPOINT_FRAMES > 0 else s.nframes))
+
+
 def _frame0_plans(s, coords, types, scale, box):
     """FP32 and FP64 plans that have both run frame 0 (on a copy of it), and
     the max relative error of the FP32 S(q) against the FP64 one on the
-    voxels above 1e-6 of the maximum (0 without such voxels)."""
+    voxels above 1e-6 of the maximum (0 without such voxels).  The FP32 plan is
+    made for the run, the FP64 one for this frame."""
     import torch
     plans, out = [], []
     try:
         for fp64 in (False, True):
-            plans.append(engine.Plan.from_setup(s, device=coords.device, fft64=fp64))
+            plans.append(engine.Plan.from_setup(s, device=coords.device, fft64=fp64,
+                                                max_frames=1 if fp64 else _call_frames(s)))
             plans[-1].accumulate_frames(coords[:1].clone(), types, scale[:1], box, s.arith,
                                         s.wrap)
             plans[-1].check_errors()
@@ -179,14 +188,17 @@ def _make_plan(s, coords, types, scale, box):
     if FFT_PRECISION == "auto" and RANDOM_NOISE == 0 and s.nframes > 0 and s.natoms > 0:
         p32, p64, err = _frame0_plans(s, coords, types, scale, box)
         fp64 = err > AUTO_FP32_MAX_ERR
-        keep, drop = (p64, p32) if fp64 else (p32, p64)
-        drop.close()
-        keep.reset()
         LAST_PRECISION.update(fp64=fp64, frame0_fp32_err=err)
-        return keep
-    fp64 = FFT_PRECISION == "fp64"
-    LAST_PRECISION.update(fp64=fp64, frame0_fp32_err=None)
-    return engine.Plan.from_setup(s, device=coords.device, fft64=fp64)
+        p64.close()
+        if not fp64:
+            p32.reset()
+            return p32
+        p32.close()
+    else:
+        fp64 = FFT_PRECISION == "fp64"
+        LAST_PRECISION.update(fp64=fp64, frame0_fp32_err=None)
+    return engine.Plan.from_setup(s, device=coords.device, fft64=fp64,
+                                  max_frames=_call_frames(s))
 
 
 def _output_plan(n):

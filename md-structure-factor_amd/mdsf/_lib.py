@@ -43,6 +43,9 @@ class GridDesc(ctypes.Structure):
 # name -> (restype, argtypes); every symbol include/mdsf.h declares
 SIGNATURES = {
     "mdsf_plan_create": (c_int32, [ctypes.POINTER(GridDesc), ctypes.POINTER(c_void_p)]),
+    "mdsf_plan_create_frames": (c_int32, [ctypes.POINTER(GridDesc), c_int64,
+                                          ctypes.POINTER(c_void_p)]),
+    "mdsf_plan_group": (c_int32, [c_void_p, ctypes.POINTER(c_int32), ctypes.POINTER(c_int32)]),
     "mdsf_plan_destroy": (c_int32, [c_void_p]),
     "mdsf_last_error": (c_char_p, []),
     "mdsf_version": (c_int32, []),
@@ -89,6 +92,8 @@ SIGNATURES = {
                                       c_void_p, c_void_p, c_void_p]),
     "mdsf_density_adjoint": (c_int32, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p]),
     "mdsf_deposit_adjoint": (c_int32, [c_void_p, c_void_p, c_void_p, c_void_p]),
+    "mdsf_batch_create_frames": (c_int32, [ctypes.POINTER(GridDesc), ctypes.POINTER(c_int64),
+                                           c_int32, ctypes.POINTER(c_void_p)]),
     "mdsf_batch_create": (c_int32, [ctypes.POINTER(GridDesc), c_int32,
                                     ctypes.POINTER(c_void_p)]),
     "mdsf_batch_destroy": (c_int32, [c_void_p]),

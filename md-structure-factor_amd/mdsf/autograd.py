@@ -56,7 +56,8 @@ class SFModel:
         r = np.asarray(coords_like)
         ucell = np.eye(3) if ucell is None else ucell
         self.setup = s = engine.Setup(r, dims, typ, rad, sres, better, ucell)
-        self.plan = engine.Plan.from_setup(s, device=device, fft64=fp64)
+        self.plan = engine.Plan.from_setup(s, device=device, fft64=fp64,
+                                            max_frames=s.nframes)
         dev = self.plan.device
         self.types = torch.from_numpy(s.type_index.astype(np.int32).reshape(-1)).to(dev)
         self.scale = torch.from_numpy(np.ascontiguousarray(s.scale, dtype=np.float64)).to(dev)

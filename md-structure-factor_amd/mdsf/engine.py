@@ -6,6 +6,8 @@ with the reference's dtypes, and ``Plan`` drives ``libmdsf`` with torch device
 memory and the current torch stream.  All per-atom and per-voxel work runs in
 the HIP kernels.
 """
+import ctypes
+
 import numpy as np
 import torch
 
@@ -143,11 +145,13 @@ class Plan:
     """One system (grid, border, cell, types) bound to a libmdsf plan on a GPU.
 
     ``fft64`` selects FP64 deposition and FFT; ``autotune`` times the FFT tile
-    and kernel choices for this grid when the plan is created.
+    and kernel choices for this grid when the plan is created.  ``max_frames``: the
+    most frames a call will have (0: any number), which bounds the frame groups a
+    small grid's plan keeps memory for; longer calls run in smaller groups.
     """
 
     def __init__(self, n, nborder, dr, ucell, amp, two_sig2, half, counts, device=None,
-                 fft64=False, autotune=False, _handle=None):
+                 fft64=False, autotune=False, _handle=None, max_frames=0):
         self.lib = _lib.load()
         if not torch.cuda.is_available():
             raise RuntimeError("libmdsf needs a ROCm GPU (torch.cuda.is_available() is False)")
@@ -163,12 +167,12 @@ class Plan:
         desc, self._tarr = grid_desc(n, nborder, dr, ucell, amp, two_sig2, half, counts, flags)
         self._handle = _lib.c_void_p()
         with torch.cuda.device(self.device):
-            _lib.check(self.lib.mdsf_plan_create(desc, self._handle))
+            _lib.check(self.lib.mdsf_plan_create_frames(desc, int(max_frames), self._handle))
 
     @classmethod
-    def from_setup(cls, s, device=None, fft64=False, autotune=False):
+    def from_setup(cls, s, device=None, fft64=False, autotune=False, max_frames=0):
         return cls(s.N, s.nborder, s.dr, s.ucell, s.amp, s.two_sig2, s.half, s.counts, device,
-                   fft64, autotune)
+                   fft64, autotune, max_frames=max_frames)
 
     # ----------------------------------------------------------------- utils
     def _stream(self):
@@ -189,6 +193,16 @@ class Plan:
             self.close()
         except Exception:
             pass
+
+    @property
+    def group(self):
+        """Frames per group of the frame loops, and of the gradients (0 before the first)."""
+        out = (_lib.c_int32 * 2)()
+        step = ctypes.sizeof(_lib.c_int32)
+        _lib.check(self.lib.mdsf_plan_group(self._handle, out,
+                                            ctypes.cast(ctypes.byref(out, step),
+                                                        ctypes.POINTER(_lib.c_int32))))
+        return int(out[0]), int(out[1])
 
     @property
     def half_shape(self):
@@ -332,7 +346,8 @@ class Batch:
     """Independent systems (each a ``Setup``) run together from one HIP graph.
 
     Every system gets an autotuned FP32 plan.  ``set_frames`` binds device
-    coordinates (never modified by the batch); ``run`` enqueues all systems'
+    coordinates (never modified by the batch; as many frames as the system's ``Setup``
+    has, or more in smaller groups); ``run`` enqueues all systems'
     frame loops as one graph launch (captured on the first run after the
     frames change); ``sf(i)`` reads system i's S(q).
     """
@@ -350,7 +365,9 @@ class Batch:
             keep.append(tarr)
         self._handle = _lib.c_void_p()
         with torch.cuda.device(self.device):
-            _lib.check(self.lib.mdsf_batch_create(descs, len(self.setups), self._handle))
+            frames = (_lib.c_int64 * len(self.setups))(*[s.nframes for s in self.setups])
+            _lib.check(self.lib.mdsf_batch_create_frames(descs, frames, len(self.setups),
+                                                         self._handle))
         self.plans = [Plan(s.N, 0, s.dr, s.ucell, [], [], [], s.counts, self.device,
                            _handle=self.lib.mdsf_batch_plan(self._handle, i))
                       for i, s in enumerate(self.setups)]
