@@ -73,6 +73,7 @@ hipError_t enqueue_system(Batch& b, int i, hipStream_t s) {
   const size_t fstride = (size_t)p.sys.natoms * 3 * esz;
   const int64_t ngroups = (f.nframes + p.group - 1) / p.group;
   int64_t t = 0;
+  p.use_slot(p.cur_slot);
   for (int64_t k = 0; k < ngroups && e == hipSuccess; ++k) {
     p.nfr = (int)((f.nframes - t) / (ngroups - k));   // groups of nearly equal size
     void* c = const_cast<char*>(static_cast<const char*>(f.coords)) + (size_t)t * fstride;
@@ -84,6 +85,7 @@ hipError_t enqueue_system(Batch& b, int i, hipStream_t s) {
     if (e == hipSuccess) e = fft_forward(p, p.rho, true, s);
     t += p.nfr;
   }
+  if (ngroups > 0) p.use_slot(p.cur_slot, p.nfr - 1);
   p.nfr = 1;
   return e;
 }

@@ -199,7 +199,7 @@ int ensure_adjoint(Plan& p) {
   }
   if (e != hipSuccess) p.adj_arena = nullptr;
   MDSF_HIP(e);
-  p.use_slot(p.cur_slot);
+  p.use_slot(p.cur_slot, p.frame_of[p.cur_slot]);
   return MDSF_OK;
 }
 
@@ -774,6 +774,7 @@ int mdsf_accumulate_frames(mdsf_plan* plan, void* d_coords, int dtype, int64_t n
       if (f != s) MDSF_HIP(hipEventRecord(p->ev_fft[b], f));
     }
   }
+  p->use_slot(p->cur_slot, p->nfr - 1);
   MDSF_HIP(wait_for(s, p->ev_fft[(ngroups - 1) % kSlots], f));
   MDSF_HIP(hipEventRecord(p->ev_done, s));
   return MDSF_OK;
@@ -879,7 +880,7 @@ int mdsf_set_frame_buffer(mdsf_plan* plan, int32_t which) {
   if (!p) return fail(MDSF_ERR_ARG, "null plan");
   if (which < 0 || which >= kSlots)
     return fail(MDSF_ERR_ARG, "frame buffer must be 0, 1 or 2");
-  p->use_slot(which);
+  p->use_slot(which, p->frame_of[which]);
   return MDSF_OK;
 }
 
@@ -1011,6 +1012,7 @@ int mdsf_adjoint_frames(mdsf_plan* plan, void* d_coords, int dtype, int64_t nfra
                                     /*derivs_ready=*/true, /*grad_zeroed=*/true));
     if (!one) MDSF_HIP(hipEventRecord(p->ev_fft[b], f));
   }
+  p->use_slot(p->cur_slot, p->nfr - 1);
   MDSF_HIP(wait_for(s, p->ev_fft[(ngroups - 1) % kSlots], f));
   MDSF_HIP(hipEventRecord(p->ev_done, s));
   return MDSF_OK;

@@ -221,39 +221,50 @@ struct Plan {
   void* spec_nyq = nullptr;      // Nx*Ny FP64 complex: the kz = Nz/2 plane, nyq[x][y]
   FrameState slot[kSlots];
   // Frame slot b: its atom state and density / spectrum buffer become the
-  // ones the launches below use (kernel arguments are taken at launch).
+  // ones the launches below use (kernel arguments are taken at launch), from
+  // frame `frame` of the group it holds.  The frame loops start at frame 0 and
+  // leave the slot at the last frame they prepared, which the single-frame
+  // entry points then find there (frame_of).
   int cur_slot = 0;
+  int frame_of[kSlots] = {};
   int group = 1;                 // frames a slot holds (group.h)
   int adj_group = 1;             // frames the adjoint's buffers hold, at most `group`
   int nfr = 1;                   // frames the next launches cover (the frame loops set it)
-  void use_slot(int b) {
+  void use_slot(int b, int frame = 0) {
     b %= kSlots;
     cur_slot = b;
+    frame_of[b] = frame;
     const FrameState& f = slot[b];
-    ir4 = f.ir4;
-    key = f.key;
-    rpos = f.rpos;
-    bucket_count = f.bucket_count;
-    bucket_off = f.bucket_off;
-    bucket_cur = f.bucket_cur;
-    bucket_aux = f.bucket_aux;
-    s_tmp = f.s_tmp;
-    s_idx = f.s_idx;
-    s_ir = f.s_ir;
-    s_r = f.s_r;
-    tables = f.tables;
-    slices = f.slices;
-    dslices = f.dslices;
-    bslices = f.bslices;
-    corners = f.corners;
-    spill = f.spill;
-    spill_flag = f.spill_flag;
-    tl_pool = f.tl_pool;
-    tl_head = f.tl_head;
-    rho = rho_buf[b];
-    spec = spec_buf[b];
-    res = res_buf[b];
-    spec_nyq = nyq_buf[b];
+    const size_t at = (size_t)frame, rs = fft64 ? 8 : 4;
+    const size_t na = at * sys.f_atoms(), nbk = at * sys.f_buckets();
+    auto bytes = [](void* p, size_t off) -> void* {
+      return p ? static_cast<char*>(p) + off : nullptr;
+    };
+    ir4 = f.ir4 + na;
+    key = f.key + na;
+    rpos = f.rpos + 3 * na;
+    bucket_count = f.bucket_count + nbk;
+    bucket_off = f.bucket_off + nbk;
+    bucket_cur = f.bucket_cur + nbk;
+    bucket_aux = f.bucket_aux + at * sys.f_aux;
+    s_tmp = f.s_tmp + na;
+    s_idx = f.s_idx + na;
+    s_ir = f.s_ir + na;
+    s_r = f.s_r + 3 * na;
+    tables = bytes(f.tables, at * sys.f_tables * 8);
+    slices = static_cast<float*>(bytes(f.slices, at * sys.f_slices * rs));
+    dslices = f.dslices;         // (made again for every single-frame call)
+    bslices = static_cast<float*>(bytes(f.bslices, at * sys.f_bslices * 4));
+    corners = f.corners + at * kCornerInts;
+    spill = bytes(f.spill, at * sys.f_spill * rs);
+    spill_flag = f.spill_flag ? f.spill_flag + at * spill_tiles : nullptr;
+    tl_pool = f.tl_pool ? f.tl_pool + at * sys.f_pool : nullptr;
+    tl_head = f.tl_head ? f.tl_head + at * sys.f_tiles : nullptr;
+    const size_t points = at * sys.f_points;
+    rho = bytes(rho_buf[b], points * rs);
+    spec = bytes(spec_buf[b], points * rs);
+    res = bytes(res_buf[b], points / 2);
+    spec_nyq = bytes(nyq_buf[b], at * sys.n[0] * sys.n[1] * 16);
   }
   double* sf_main = nullptr;     // FP64 accumulator sf[kz][ky][kx], kz < Nz/2
   double* sf_nyq = nullptr;      // FP64 accumulator of the kz = Nz/2 plane, [kx][ky]
