@@ -85,9 +85,10 @@ int mdsf_plan_create(const mdsf_grid_desc* desc, mdsf_plan** out);
  * plan holds the state of a whole group in each of its three slots (up to 16
  * frames, 2 GiB in all and as much again for gradients).  A plan that will only see
  * a few frames per call takes less memory when it is told; longer calls still work,
- * in smaller groups.  Groups also shrink where less than about half of the device's
- * memory is free, down to one frame when memory is out.  Results do not depend on
- * the group. */
+ * in smaller groups.  Groups also shrink where memory is short (all of a process's
+ * plans together keep at most a quarter of a device's memory for frames beyond one
+ * each, and a plan at most a sixteenth of what is free), down to one frame when it is
+ * out.  Results do not depend on the group. */
 int mdsf_plan_create_frames(const mdsf_grid_desc* desc, int64_t max_frames, mdsf_plan** out);
 
 /* Frames per group of the plan, and of its gradients (0 before the first gradient

@@ -2,6 +2,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
 #include <cmath>
 #include <cstring>
 #include <map>
@@ -107,8 +108,33 @@ hipError_t pipeline_streams(int device, hipStream_t* dep, hipStream_t* fft, hipS
   return hipSuccess;
 }
 
+// Bytes that the groups of a device's plans hold beyond one frame (group.h).
+constexpr int kDevices = 64;
+std::atomic<size_t> g_group_taken[kDevices];
+
+std::atomic<size_t>& group_taken(int device) {
+  return g_group_taken[device >= 0 && device < kDevices ? device : kDevices - 1];
+}
+
+// The plan's device must be the current one.
+GroupMemory group_memory(int device) {
+  GroupMemory mem;
+  if (hipMemGetInfo(&mem.free, &mem.total) != hipSuccess) {
+    (void)hipGetLastError();
+    return GroupMemory();
+  }
+  mem.taken = group_taken(device).load();
+  return mem;
+}
+
+void take_extra(Plan& p, size_t bytes) {
+  p.group_extra += bytes;
+  group_taken(p.device) += bytes;
+}
+
 void free_plan(Plan* p) {
   if (!p) return;
+  group_taken(p->device) -= p->group_extra;
   for (hipEvent_t e : {p->ev_fork, p->ev_done, p->ev_lfork, p->ev_lgath, p->ev_ljoin})
     if (e) (void)hipEventDestroy(e);
   for (int b = 0; b < kSlots; ++b)
@@ -160,13 +186,6 @@ struct FrameGroup {
   ~FrameGroup() { p.nfr = 1; }
 };
 
-// Free and total memory of the current device, zeros if they cannot be asked.
-void device_memory(size_t* free, size_t* total) {
-  if (hipMemGetInfo(free, total) == hipSuccess) return;
-  (void)hipGetLastError();
-  *free = *total = 0;
-}
-
 int ensure_adjoint(Plan& p) {
   const size_t nxy = (size_t)p.sys.n[0] * p.sys.n[1];
   const size_t m = (size_t)p.sys.n[2] / 2;
@@ -178,10 +197,8 @@ int ensure_adjoint(Plan& p) {
     const bool tiled = p.adj_tslots > 0;
     const size_t slots = (size_t)(tiled ? p.adj_tslots : p.adj_items);
     const size_t bytes = 24 * slots + (tiled ? kSlots * 4 * (size_t)p.slice_floats : 0);
-    size_t free, total;
-    device_memory(&free, &total);
-    p.adj_group = std::min(p.group, group_fit(bytes, free, total));
-    return take_group(&p.adj_group, hipErrorOutOfMemory, [&](int frames) {
+    p.adj_group = std::min(p.group, group_fit(bytes, group_memory(p.device)));
+    const hipError_t e = take_group(&p.adj_group, hipErrorOutOfMemory, [&](int frames) {
       const size_t g = (size_t)frames;
       Arena arena;
       arena.add(&p.adj_w, nxy * (m + 1));
@@ -190,6 +207,8 @@ int ensure_adjoint(Plan& p) {
       arena.add(tiled ? &p.adj_tpart : &p.adj_part, 3 * g * slots);
       return arena.take(&p.adj_arena);
     });
+    if (e == hipSuccess) take_extra(p, (size_t)(p.adj_group - 1) * bytes);
+    return e;
   };
   hipError_t e = take();
   if (e == hipErrorOutOfMemory && p.adj_tslots > 0 && p.sys.mode == MODE_XY) {
@@ -519,10 +538,10 @@ int mdsf_plan_create_frames(const mdsf_grid_desc* desc, int64_t max_frames, mdsf
                          (size_t)p->slice_floats * rs + (size_t)p->bslice_floats * 4 +
                          (size_t)s.f_tables * 8 + (size_t)s.f_spill * rs + (size_t)p->tl_cap * 8 +
                          (size_t)s.f_points * rs + spec_bytes + res_bytes + nx * ny * 16;
-    size_t free, total;
-    device_memory(&free, &total);
-    p->group = group_frames(s.f_tiles, max_frames, kSlots * bytes, free, total);
-    return take_group(&p->group, hipErrorOutOfMemory, allocate);
+    p->group = group_frames(s.f_tiles, max_frames, kSlots * bytes, group_memory(p->device));
+    const hipError_t e = take_group(&p->group, hipErrorOutOfMemory, allocate);
+    if (e == hipSuccess) take_extra(*p, (size_t)(p->group - 1) * kSlots * bytes);
+    return e;
   };
   hipError_t e = take();
   if (e == hipErrorOutOfMemory && p->fft64 && p->slice_floats > 0) {

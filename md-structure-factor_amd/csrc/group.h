@@ -19,29 +19,36 @@ namespace mdsf {
 constexpr int kGroupTiles = 2048;
 constexpr int kMaxGroup = 16;
 constexpr size_t kGroupBytes = (size_t)2 << 30;
-// What groups take beyond one frame comes out of the first half of the device's
-// memory, a plan's at most this share of what is free of it, so that any number of
-// plans that fits half the device with one frame each still fits (150 plans of
-// 140 MB took 21 GB with one frame each and would take 300 GB with whole groups).
+// What groups take beyond one frame is at most 1 / kGroupTotal of the device's memory
+// over all plans of the process, and a plan's at most 1 / kGroupShare of what is free,
+// so that plans which fit three quarters of the device with one frame each fit it still
+// (150 plans of 140 MB took 21 GB with one frame each and would take 300 GB with whole
+// groups).
 constexpr size_t kGroupShare = 16;
+constexpr size_t kGroupTotal = 4;
 
-// Frames whose state of `bytes` each fits kGroupBytes and the device's memory (free
-// and total: 0 if unknown), at least 1.
-inline int group_fit(size_t bytes, size_t free, size_t total) {
+// The device's memory (total 0: unknown) and what groups hold of it beyond one frame.
+struct GroupMemory {
+  size_t free = 0, total = 0, taken = 0;
+};
+
+// Frames whose state of `bytes` each fits kGroupBytes and the memory, at least 1.
+inline int group_fit(size_t bytes, const GroupMemory& mem) {
   if (bytes == 0) return kMaxGroup;
   size_t extra = kGroupBytes;
-  if (total > 0) {
-    const size_t used = total / 2 + bytes;
-    extra = free > used ? (free - used) / kGroupShare : 0;
+  if (mem.total > 0) {
+    const size_t most = mem.total / kGroupTotal;
+    extra = std::min(mem.free > bytes ? (mem.free - bytes) / kGroupShare : 0,
+                     most > mem.taken ? most - mem.taken : 0);
   }
   const size_t fit = std::min(kGroupBytes / bytes, 1 + extra / bytes);
   return (int)std::min<size_t>(std::max<size_t>(fit, 1), kMaxGroup);
 }
 
 // The group of a grid of `tiles` tiles for calls of at most `frames` frames (0: any).
-inline int group_frames(long long tiles, int64_t frames, size_t bytes, size_t free, size_t total) {
+inline int group_frames(long long tiles, int64_t frames, size_t bytes, const GroupMemory& mem) {
   const long long want = (kGroupTiles + tiles - 1) / std::max(tiles, 1LL);
-  long long g = std::min<long long>(want, group_fit(bytes, free, total));
+  long long g = std::min<long long>(want, group_fit(bytes, mem));
   if (frames > 0) g = std::min<long long>(g, frames);
   return (int)std::max(1LL, g);
 }

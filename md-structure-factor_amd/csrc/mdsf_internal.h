@@ -229,6 +229,7 @@ struct Plan {
   int frame_of[kSlots] = {};
   int group = 1;                 // frames a slot holds (group.h)
   int adj_group = 1;             // frames the adjoint's buffers hold, at most `group`
+  size_t group_extra = 0;        // bytes of both beyond one frame (GroupMemory::taken)
   int nfr = 1;                   // frames the next launches cover (the frame loops set it)
   void use_slot(int b, int frame = 0) {
     b %= kSlots;
