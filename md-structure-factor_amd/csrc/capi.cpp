@@ -150,8 +150,10 @@ void free_plan(Plan* p) {
 // many atoms; with less work the cross-stream waits (about 10 us each) cost more than
 // the branches overlap.  16 frames of 50,000 atoms at 104 x 90 x 80 in groups of 4: 1,443
 // us without the split, 1,405 with.  One group alone, which without the split needs no
-// waits at all, splits at four times the atoms: one of 80,000 at 128^3 takes 366 us in
-// one stream, 409 split; a million atoms at 512^3 are split by their tiles.
+// waits at all, splits at four times the atoms.  Atoms of the group, one stream / split:
+// one frame at 128^3 80,000 242 / 263 us, 160,000 395 / 401, 320,000 865 / 772, 640,000
+// 1,700 / 1,477; at 96^3 160,000 505 / 503, 320,000 1,185 / 959; four frames at 128^3
+// 160,000 331 / 354, 320,000 658 / 638; sixteen at 64^3 320,000 391 / 404.
 bool split_prep(const Plan& p, int64_t nframes) {
   const long long ntiles = (long long)p.sys.ntiles[0] * p.sys.ntiles[1] * p.sys.ntiles[2];
   const long long least = (nframes <= p.group ? 4 : 1) * kSplitPrepAtoms;

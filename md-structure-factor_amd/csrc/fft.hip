@@ -30,9 +30,9 @@
 // the previous one through LDS (real and imaginary parts in turn, one FP64
 // plane), and the last stage stores straight to global memory or folds |X|^2
 // into the accumulator.  Other lengths take the any-length passes of
-// fft_any.hip, and those that do not fit them (two prime factors above 13, above
-// 1024) the LDS-staged pass (every stage in LDS, radices 2/3/4/5/8/16 and generic
-// odd primes).
+// fft_any.hip, and those that do not fit them (above 1024, two prime factors above
+// 13, or a split with a middle radix above 8: any_plan) the LDS-staged pass (every
+// stage in LDS, radices 2/3/4/5/8/16 and generic odd primes).
 #include <map>
 #include <mutex>
 
@@ -784,8 +784,7 @@ int res_block(const Plan& p) {
 
 // choice: 0 = default (register-staged when n has a split, else the any-length
 // pass), kTuneReg = register-staged, 1..16 = the any-length pass with that many
-// pencils.  Lengths neither takes (two prime factors above 13, above 1024) run
-// the LDS-staged pass.
+// pencils.  Lengths neither takes (any_plan) run the LDS-staged pass.
 template <typename R>
 hipError_t run_pass(PassArgs<R> a, PassKind kind, hipStream_t s, int choice) {
   int r1, r2, r3;
@@ -1192,8 +1191,10 @@ hipError_t autotune_impl(Plan& p, hipStream_t s) {
     return err;
   }
   const int cand[5] = {kTuneReg, 2, 4, 8, 16};
-  // z pass: the register-staged kernel (m with a two-stage split) or the
-  // LDS-staged pass with that many rows
+  // z pass: the register-staged kernel (m with a two-stage split) or the any-length
+  // pass (else the LDS-staged one) with that many rows.  Tiles too large for the
+  // LDS-staged pass are left out for both: the any-length pass holds fewer values in
+  // LDS, but at most 4,096 a block, and would halve such a tile to one already timed.
   float best = 1e30f;
   int pick = 0;
   for (int c : cand) {
@@ -1208,7 +1209,7 @@ hipError_t autotune_impl(Plan& p, hipStream_t s) {
     }
   }
   p.tune_z = pick;
-  // y and x passes: the register-staged pass or the LDS-staged one
+  // y and x passes: the same choice
   for (int axis = 0; axis < 2 && err == hipSuccess; ++axis) {
     int& slot = axis == 0 ? p.tune_y : p.tune_x;
     const int n = p.sys.n[axis == 0 ? 1 : 0];

@@ -1,5 +1,6 @@
-// FFT passes of any length up to 1024: the grids whose sizes come out of a box and
-// a resolution (104, 90, 208, 106 = 2 x 53 ...) rather than powers of two.
+// FFT passes of lengths up to 1024 (all but the few that any_plan refuses): the grids
+// whose sizes come out of a box and a resolution (104, 90, 208, 106 = 2 x 53 ...)
+// rather than powers of two.
 //
 // A block takes P pencils.  The first stage reads its butterflies' inputs straight
 // from global memory and leaves them in LDS, the last one stores (or accumulates)
@@ -567,9 +568,8 @@ __global__ __launch_bounds__(kAnyThreads) void k_c2r_z_any(CArgs<R> a, AnyPlan p
 // --- plans (host) --------------------------------------------------------------------
 unsigned magic(int d) { return (unsigned)(((1ULL << 32) + d - 1) / d); }   // d > 1
 
-// Fewest stages of radices 2 to 16 with product s (middle ones at most 8, so that
-// a thread holds its butterflies across the in-place exchange), the largest radix
-// as small as can be.  Radices in ascending order in `best`.
+// Fewest stages of radices 2 to 16 with product s, the largest radix as small as can
+// be.  Radices in ascending order in `best`.
 void search(int s, int lo, int* cur, int depth, int* best, int* nbest) {
   if (s == 1) {
     if (depth < *nbest || (depth == *nbest && cur[depth - 1] < best[depth - 1])) {
@@ -586,8 +586,10 @@ void search(int s, int lo, int* cur, int depth, int* best, int* nbest) {
     }
 }
 
-// Stages of length n: false if n has two prime factors above 13, or needs more
-// than two radices above 8.
+// Stages of length n: false if n has two prime factors above 13, or if the radices
+// found put one above 8 in a middle stage, where a thread holds its butterflies across
+// the in-place exchange (of the even lengths 810, 900, 972, 990 and 1000; splits with
+// more stages or a larger last radix are not looked for).
 bool any_plan(int n, AnyPlan* pl) {
   if (n < 2 || n > kAnyMax) return false;
   pl->n = n;

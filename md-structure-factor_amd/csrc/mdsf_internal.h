@@ -24,7 +24,7 @@ constexpr int kListNoSlice = 255;  // tile-list entry: no slice on that axis (a 
 // tiles, or atoms of a group, from which the frame loop splits its prepare stage (split_prep)
 constexpr long long kSplitPrepTiles = 2048;
 constexpr long long kSplitPrepAtoms = 65536;
-// stage-timing events per frame: prepare start / end (caller's stream), the
+// stage-timing events per group: prepare start / end (caller's stream), the
 // deposition kernel's begin / end, the three FFT passes' begin / end, and the
 // end of the prepare stage's tile-list branch
 constexpr int kTimedEvents = 11;
@@ -272,8 +272,9 @@ struct Plan {
   // FFT
   int fft64 = 0;                 // deposition, density and FFT in FP64 (else FP32)
   FftAxis ax_x, ax_y, ax_zc;     // zc: complex length Nz/2
-  // FFT launch choices (0 = default): z rows per tile; y / x pencil kernel
-  // (kTuneReg = register-staged, 1..16 = generic LDS tile with that many pencils)
+  // FFT launch choices (0 = default): kTuneReg = register-staged, 1..16 = rows (z) or
+  // pencils (y, x) per block of the any-length pass, or of the LDS-staged one for the
+  // lengths that pass does not take
   int tune_z = 0, tune_y = 0, tune_x = 0;
   float2* tw_r2c = nullptr;      // W_Nz^k, k < Nz
   double2* tw_r2c64 = nullptr;
@@ -284,8 +285,9 @@ struct Plan {
   // the prepare stage's tile-list branch (frame loop; shared like the two above)
   hipStream_t aux_stream = nullptr;
   hipEvent_t ev_lfork = nullptr, ev_lgath = nullptr, ev_ljoin = nullptr;
-  // optional stage timing of mdsf_accumulate_frames: 10 timing events per
-  // frame (prepare, deposit, z, y, x: start / end, each on its stream)
+  // optional stage timing of mdsf_accumulate_frames: kTimedEvents events per
+  // group (prepare, deposit, z, y, x: start / end, each on its stream, and the
+  // end of the prepare stage's tile-list branch)
   int timing = 0;  // 0 off, 1 every stage, 2 the deposition only (per group)
   // events the next tiled deposition records with its own dispatch (begin,
   // end), or null: set by the timed frame loop around launch_deposit

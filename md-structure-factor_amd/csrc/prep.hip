@@ -380,9 +380,12 @@ __global__ void k_tables(SysDev sys, const TypeDev* __restrict__ td, const int4*
 // F: the plan's element type.  FP64 plans (orthogonal cells) take the exponent and
 // exp as k_tables does, without derivatives.
 //
-// Bound by the stores and by the fetches before them: 4 frames of 50,000 atoms at
-// 104 x 90 x 80 (about 115 MB) take 46 us; with a lane per cell, which fetched
-// everything sixteen times and stored 4 bytes, 86 us.
+// Groups are bound by the stores and the fetches before them: 4 frames of 50,000 atoms
+// at 104 x 90 x 80 (about 115 MB) take 46 us; with a lane per cell, which fetched
+// everything sixteen times and stored 4 bytes, 86 us.  One frame of 50,000 atoms at
+// 256^3 alone (28.7 MB) is bound by latency instead, a quarter of the lanes walking
+// the same chain of slices: 34 us, with a lane per cell 30; beside the frame loop's
+// other kernels the wider stores win (20 frames 4,863 -> 4,724 us).
 constexpr int kSliceCells = 4;                        // cells of a lane
 constexpr int kSliceLanes = kTile / kSliceCells;      // lanes of an (atom, axis)
 
