@@ -722,15 +722,18 @@ __global__ __launch_bounds__(kThreads) void k_deposit(SysDev sys, const TypeDev*
 // frames of 8,000 atoms in a dodecahedral cell on a grid of 100^3 took 2,317 us in
 // all with an exponential per voxel and image and take 912 (866 with one exponential
 // per column and the cross factors of each pair of axes staged per atom: the
-// exponentials are not what is left).  Types whose factors could leave FP64's range
-// (a cell matrix far from unit edges) and the atoms left over take the full
-// evaluation per voxel and image.  So do FP64 plans: ln Z and ln E cancel, and three
-// factors and their powers round more often than one exponential.  Weighted by the
-// values, the terms are 1.2e-16 to 2.9e-16 from exact with an exponential each and
-// 1.9e-16 to 5.9e-16 in the column form (cells of 0.3 to 0.8 Angstrom, dodecahedral
-// to strongly oblique); the density of 300 atoms at 1 Angstrom 1.5e-17 and 2.2e-17 of
-// its maximum (rms).  The price: the same four frames with an FP64 plan take 2,339 us,
-// 861 in the column form.
+// exponentials are a small part).  What is left is 37,000 VALU instructions a wave,
+// issued in half of the cycles by 2.4 waves per SIMD (1,372 blocks of unequal work).
+// Types whose factors could leave FP64's range (a cell matrix far from unit edges)
+// and the atoms left over take the full evaluation per voxel and image.
+//
+// So do FP64 plans: ln Z and ln E cancel, and three factors and their powers round
+// more often than one exponential.  Weighted by the values, the terms are 1.2e-16 to
+// 2.9e-16 from exact with an exponential each and 1.9e-16 to 5.9e-16 in the column
+// form (on the host: cells of 0.3 to 0.8 Angstrom, dodecahedral to strongly oblique);
+// the density of 300 atoms at 1 Angstrom 1.5e-17 and 2.2e-17 of its maximum (rms).
+// The price: the same four frames with an FP64 plan take 2,339 us, 861 in the column
+// form.
 //
 // Of those, per (x, y) image pair the z sources of tile cell c are u = c - N, c,
 // c + N, except where the corner slot applies (x and y off the core): for y on L
